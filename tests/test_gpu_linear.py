@@ -394,3 +394,32 @@ def test_linear_fused_rejects_half_norm(wrs, ctx):
             (wrs.ctypes.c_void_p * 1)(w.data_ptr()), None, 2, 64, 64, 0, 0,
             (wrs.ctypes.c_void_p * 1)(torch.zeros((2, 64), device="cuda").data_ptr()),
             (wrs.ctypes.c_size_t * 1)(128), 64, 64), "linear_fused")
+
+
+@pytest.mark.parametrize("n_in", [64, 512, 576, 1344, 2048, 2112, 5120, 5184])
+def test_linear_split_row_widths(wrs, ctx, n_in):
+    """f32 rows above the weight-stream size, at both sides of every register
+    row width of the split: rows that start on any dword (float64 within the
+    accumulation bound), and normalized rows (bit for bit the layer_norm
+    followed by the projection, also where the norm stays a launch of its own)."""
+    note(f"linear split widths K={n_in}")
+    n_tokens, n_out = 11, 68
+    rng = np.random.default_rng(n_in)
+    x = rng.standard_normal((n_tokens, n_in)).astype(np.float32)
+    x *= 10.0 ** rng.uniform(-8, 8, (n_tokens, 1)).astype(np.float32)
+    w = _weights(n_out, n_in, n_in + 1)
+    wd = torch.from_numpy(w).cuda()
+    buf = torch.zeros(1 + n_tokens * (n_in + 3), device="cuda")
+    xs = buf[1:].view(n_tokens, n_in + 3)[:, :n_in]
+    xs.copy_(dev(x))
+    out = torch.full((n_tokens, n_out), float("nan"), device="cuda")
+    wrs.linear(xs, wd, None, out, ctx=ctx)
+    assert (np.abs(host(out) - _exact(x, w, None)) <= _gamma_bound(x, w)).all()
+    gamma = dev((1.0 + 0.1 * rng.standard_normal(n_in)).astype(np.float32))
+    beta = dev((0.1 * rng.standard_normal(n_in)).astype(np.float32))
+    xd = dev(x)
+    wrs.linear_fused(xd, [wd], None, [out], ln=(gamma, beta, 1e-5), ctx=ctx)
+    normed, ref = torch.empty_like(xd), torch.empty_like(out)
+    wrs.layer_norm(xd, gamma, beta, 1e-5, normed, ctx=ctx)
+    wrs.linear(normed, wd, None, ref, ctx=ctx)
+    assert torch.equal(out, ref)

@@ -841,30 +841,106 @@ __global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_mfma(GemvArgs a, int 
   }
 }
 
-// f32 rows -> [hi | lo] f16 rows of 2 n_in, plus each row's 2^-shift.
-// One wave per row.
+// f32 rows -> [hi | lo] f16 rows of 2 n_in, plus each row's 2^-shift; with
+// kLn the rows are normalized first (norm.rs:116-143, the layer_norm_rows
+// arithmetic exactly). One wave per row. Bound by memory (4 bytes in, 4 out a
+// value): rows of up to 256 kCached values are loaded once, every 16-byte load
+// in flight before the maximum is taken, and leave as 8-byte stores; the
+// scalar form this replaces read each row twice, one dword per lane and trip
+// (1500 x 5120: 57 us; 37 x 1280: 6.4 us). x needs dword alignment only.
 __device__ inline float pow2(int e) { return __builtin_bit_cast(float, (e + 127) << 23); }
 __device__ inline int clamp_exp(int e) { return e < -126 ? -126 : (e > 127 ? 127 : e); }
 
+__device__ inline f32x4 load4_dword_aligned(const float* p) {
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+  return *reinterpret_cast<const f32x4u*>(p);
+}
+
+__device__ inline float abs_max4(const f32x4& v) {
+  return fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+}
+// Four values scaled by `up` as f16 high parts at dst and low parts at dst + n_in.
+__device__ inline void split_store4(const f32x4& x, float up, _Float16* dst, int n_in) {
+  f16x4v hv, lv;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float v = x[j] * up;
+    const _Float16 h = static_cast<_Float16>(v);
+    hv[j] = h;
+    lv[j] = static_cast<_Float16>(v - static_cast<float>(h));
+  }
+  *reinterpret_cast<f16x4v*>(dst) = hv;
+  *reinterpret_cast<f16x4v*>(dst + n_in) = lv;
+}
+
+template <int kCached, bool kLn>
 __global__ __launch_bounds__(256) void linear_split_rows(const float* x, int64_t x_rs,
                                                          int n_tokens, int n_in,
-                                                         _Float16* xs, float* row_scale) {
+                                                         const float* gamma, const float* beta,
+                                                         float eps, _Float16* xs,
+                                                         float* row_scale) {
+  static_assert(!kLn || kCached > 0, "normalized rows are held in registers");
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (t >= n_tokens) return;
   const float* xr = x + static_cast<int64_t>(t) * x_rs;
+  _Float16* dst = xs + static_cast<int64_t>(t) * kSplitParts * n_in;
   float amax = 0.0f;
-  for (int k = lane; k < n_in; k += 64) amax = fmaxf(amax, fabsf(xr[k]));
-  for (int o = 32; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+  f32x4 v[kCached > 0 ? kCached : 1];
+  if constexpr (kCached > 0) {
+    f32x4 gv[kLn ? kCached : 1], bv[kLn ? kCached : 1];
+#pragma unroll
+    for (int i = 0; i < kCached; ++i) {
+      const int k = 4 * lane + 256 * i;
+      const bool in = k < n_in;
+      const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+      v[i] = in ? load4_dword_aligned(xr + k) : z;
+      if constexpr (kLn) {
+        gv[i] = in ? *reinterpret_cast<const f32x4*>(gamma + k) : z;
+        bv[i] = in ? *reinterpret_cast<const f32x4*>(beta + k) : z;
+      }
+    }
+    if constexpr (kLn) {
+      float s = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kCached; ++i) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
+      const float mean = wave_sum64(s) / static_cast<float>(n_in);
+      float q = 0.0f;
+#pragma unroll
+      for (int i = 0; i < kCached; ++i) {
+        if (4 * lane + 256 * i >= n_in) break;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q = fmaf(v[i][j] - mean, v[i][j] - mean, q);
+      }
+      const float var = wave_sum64(q) / static_cast<float>(n_in);
+      const float inv_std = 1.0f / sqrtf(var + eps);
+#pragma unroll
+      for (int i = 0; i < kCached; ++i) {
+        if (4 * lane + 256 * i >= n_in) break;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          v[i][j] = fmaf((v[i][j] - mean) * inv_std, gv[i][j], bv[i][j]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kCached; ++i) amax = fmaxf(amax, abs_max4(v[i]));  // zeros past n_in
+  } else {
+    for (int k = 4 * lane; k < n_in; k += 256)
+      amax = fmaxf(amax, abs_max4(load4_dword_aligned(xr + k)));
+  }
+  amax = wave_max64(amax);
   const int e_max = static_cast<int>((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFF);
   const int sh = e_max == 0 ? 0 : clamp_exp(141 - e_max);
   const float up = pow2(sh);
-  _Float16* dst = xs + static_cast<int64_t>(t) * kSplitParts * n_in;
-  for (int k = lane; k < n_in; k += 64) {
-    const float v = xr[k] * up;
-    const _Float16 h = static_cast<_Float16>(v);
-    dst[k] = h;
-    dst[n_in + k] = static_cast<_Float16>(v - static_cast<float>(h));
+  if constexpr (kCached > 0) {
+#pragma unroll
+    for (int i = 0; i < kCached; ++i) {
+      const int k = 4 * lane + 256 * i;
+      if (k < n_in) split_store4(v[i], up, dst + k, n_in);
+    }
+  } else {
+    for (int k = 4 * lane; k < n_in; k += 256)
+      split_store4(load4_dword_aligned(xr + k), up, dst + k, n_in);
   }
   if (lane == 0) row_scale[t] = pow2(clamp_exp(-sh));
 }
@@ -872,10 +948,29 @@ __global__ __launch_bounds__(256) void linear_split_rows(const float* x, int64_t
 }  // namespace
 
 hipError_t launch_linear_split(const float* x, int64_t x_rs, int n_tokens, int n_in,
-                               _Float16* xs, float* row_scale, hipStream_t s) {
+                               const float* ln_g, const float* ln_b, float ln_eps, _Float16* xs,
+                               float* row_scale, hipStream_t s) {
   if (n_tokens <= 0) return hipSuccess;
-  hipLaunchKernelGGL(linear_split_rows, dim3((n_tokens + 3) / 4), dim3(256), 0, s, x, x_rs,
-                     n_tokens, n_in, xs, row_scale);
+  if (ln_g && n_in > kSplitLnMax) return hipErrorInvalidValue;
+  const dim3 grid((n_tokens + 3) / 4), block(256);
+#define WRS_SPLIT(C, LN)                                                                     \
+  hipLaunchKernelGGL((linear_split_rows<C, LN>), grid, block, 0, s, x, x_rs, n_tokens, n_in, \
+                     ln_g, ln_b, ln_eps, xs, row_scale)
+  if (ln_g) {
+    if (n_in <= 1280)
+      WRS_SPLIT(5, true);
+    else
+      WRS_SPLIT(8, true);
+  } else if (n_in <= 512) {
+    WRS_SPLIT(2, false);
+  } else if (n_in <= 1280) {
+    WRS_SPLIT(5, false);
+  } else if (n_in <= 5120) {
+    WRS_SPLIT(20, false);
+  } else {
+    WRS_SPLIT(0, false);
+  }
+#undef WRS_SPLIT
   return hipGetLastError();
 }
 

@@ -46,7 +46,7 @@ struct wrs_attn_ctx {
   size_t cap_part_bytes = 0;
   void* lin_x = nullptr;  // projections: split f16 rows of f32 activations + row scales
   size_t lin_x_bytes = 0;
-  float* ln_x = nullptr;  // fused projections above the weight-stream size: normalized rows
+  float* ln_x = nullptr;  // fused projections of rows too long for the split: normalized rows
   size_t ln_x_bytes = 0;
   float* exact_scores = nullptr;  // f32 arena attention: full score rows
   size_t exact_scores_bytes = 0;
@@ -642,9 +642,11 @@ int wrs_attn_reserve(wrs_attn_ctx* c, const wrs_reserve* r) {
         align_up(r->linear_tokens * wrs::kSplitParts * r->linear_n_in * 2, 256);
     rc = grow(c, &c->lin_x, &c->lin_x_bytes, split_bytes + r->linear_tokens * 4, false);
     if (rc) return rc;
-    rc = grow(c, reinterpret_cast<void**>(&c->ln_x), &c->ln_x_bytes,
-              r->linear_tokens * r->linear_n_in * sizeof(float), false);
-    if (rc) return rc;
+    if (r->linear_n_in > static_cast<size_t>(wrs::kSplitLnMax)) {
+      rc = grow(c, reinterpret_cast<void**>(&c->ln_x), &c->ln_x_bytes,
+                r->linear_tokens * r->linear_n_in * sizeof(float), false);
+      if (rc) return rc;
+    }
   }
   WRS_HIP(c, hipStreamSynchronize(c->stream));
   return WRS_OK;
@@ -1447,10 +1449,12 @@ int wrs_attn_capture_cross_heads_lse(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, 
 namespace {
 
 // Shared front half of the projection entry points: validates x and the
-// shape, splits f32 rows into the context scratch, and fills the x part of
-// the launch arguments. Caller holds c->mu and the device guard.
+// shape, splits f32 rows (normalized first with ln_g) into the context
+// scratch, and fills the x part of the launch arguments. Caller holds c->mu
+// and the device guard.
 int linear_prepare(wrs_attn_ctx* c, int x_dtype, const void* x, int64_t x_rs, size_t n_tokens,
-                   size_t n_in, size_t n_out, wrs::LinearArgs& a) {
+                   size_t n_in, size_t n_out, wrs::LinearArgs& a, const float* ln_g = nullptr,
+                   const float* ln_b = nullptr, float ln_eps = 0.f) {
   if (n_in == 0 || n_in % wrs::kLinearK != 0)
     return fail(c, WRS_EUNSUPPORTED, "n_in must be a positive multiple of 64");
   if (n_out % 4 != 0) return fail(c, WRS_EUNSUPPORTED, "n_out must be a multiple of 4");
@@ -1482,8 +1486,8 @@ int linear_prepare(wrs_attn_ctx* c, int x_dtype, const void* x, int64_t x_rs, si
   if (rc) return rc;
   auto* xs = static_cast<_Float16*>(c->lin_x);
   auto* scale = reinterpret_cast<float*>(static_cast<char*>(c->lin_x) + split_bytes);
-  WRS_HIP(c, wrs::launch_linear_split(static_cast<const float*>(x), x_rs, a.n_tokens, a.n_in, xs,
-                                      scale, c->stream));
+  WRS_HIP(c, wrs::launch_linear_split(static_cast<const float*>(x), x_rs, a.n_tokens, a.n_in,
+                                      ln_g, ln_b, ln_eps, xs, scale, c->stream));
   a.x = xs;
   a.x_rs = wrs::kSplitParts * static_cast<int64_t>(n_in);
   a.row_scale = scale;
@@ -1566,10 +1570,11 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
     if (!aligned_out(out[gi], out_dtype, out_row_stride, out_head_stride) ||
         (bias && bias[gi] && (reinterpret_cast<uintptr_t>(bias[gi]) & 15)))
       return fail(c, WRS_EUNSUPPORTED, "bias needs 16-byte, out 4-element alignment");
-  if (ln_g) {
-    // Larger batches: the LayerNorm runs as its own launch into scratch rows.
-    if (x_row_stride != static_cast<int64_t>(n_in))
-      return fail(c, WRS_EUNSUPPORTED, "a fused layer norm over more than 8 rows needs packed x rows");
+  if (ln_g && x_row_stride != static_cast<int64_t>(n_in))
+    return fail(c, WRS_EUNSUPPORTED, "a fused layer norm over more than 8 rows needs packed x rows");
+  if (ln_g && n_in > static_cast<size_t>(wrs::kSplitLnMax)) {
+    // Rows too long for the split's registers: the LayerNorm runs as its own
+    // launch into scratch rows.
     int rc = grow(c, reinterpret_cast<void**>(&c->ln_x), &c->ln_x_bytes,
                   n_tokens * n_in * sizeof(float), false);
     if (rc) return rc;
@@ -1577,10 +1582,11 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
                                       static_cast<int>(n_tokens), static_cast<int>(n_in),
                                       wrs::kF32, c->ln_x, c->stream));
     x = c->ln_x;
-    x_row_stride = static_cast<int64_t>(n_in);
+    ln_g = ln_b = nullptr;
   }
   wrs::LinearArgs a{};
-  int rc = linear_prepare(c, x_dtype, x, x_row_stride, n_tokens, n_in, n_out, a);
+  int rc = linear_prepare(c, x_dtype, x, x_row_stride, n_tokens, n_in, n_out, a, ln_g, ln_b,
+                          ln_eps);
   if (rc) return rc;
   a.act = act;
   a.n_groups = n_groups;

@@ -233,9 +233,13 @@ struct GemvArgs {
   void* out[kMaxLinearGroups];
 };
 hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s);
-// f32 rows -> [hi | lo] f16 rows (kSplitParts n_in each) and per-row 2^-shift.
+// f32 rows -> [hi | lo] f16 rows (kSplitParts n_in each) and per-row 2^-shift,
+// normalized first when ln_g is set (n_in <= kSplitLnMax; gamma and beta
+// 16-byte aligned).
+constexpr int kSplitLnMax = 2048;
 hipError_t launch_linear_split(const float* x, int64_t x_rs, int n_tokens, int n_in,
-                               _Float16* xs, float* row_scale, hipStream_t s);
+                               const float* ln_g, const float* ln_b, float ln_eps, _Float16* xs,
+                               float* row_scale, hipStream_t s);
 
 // LayerNorm over f32 rows (norm.rs:116-143), output f32/f16/bf16 rows of d;
 // d % 4 == 0, rows 16-byte aligned.
