@@ -97,7 +97,10 @@ const char *wrs_attn_status_string(int status);
  * 16-bit prefill grids of fewer 128-query blocks than half the CUs merge
  * blocks split over two workgroups through a fixed context buffer (~9 MB on
  * 256 CUs), allocated by the first such call outside capture; during capture
- * before then, the call takes another schedule instead. Switching streams
+ * before then, the call takes another schedule instead. Projections of more
+ * than 8 rows over n_in >= 2048 whose tiles cover less than half the CUs split
+ * k through the same buffer, under the same rule (reserving linear_tokens
+ * allocates it). Switching streams
  * (wrs_attn_set_stream) drains the old stream unless either stream is
  * recording a graph. Zero fields are ignored; reserving never shrinks.
  * Synchronous. */

@@ -423,3 +423,76 @@ def test_linear_split_row_widths(wrs, ctx, n_in):
     wrs.layer_norm(xd, gamma, beta, 1e-5, normed, ctx=ctx)
     wrs.linear(normed, wd, None, ref, ctx=ctx)
     assert torch.equal(out, ref)
+
+
+# Rows and features that take each tile shape of the projection (64 x 64 to
+# 256 x 256) with ragged last tiles, and the k splits (n_in >= 2048).
+@pytest.mark.parametrize("x_dt", ["f16", "f32"])
+@pytest.mark.parametrize("n_tokens,n_in,n_out", [
+    (9, 64, 4), (65, 192, 260), (450, 192, 1284), (1500, 192, 1284), (1501, 192, 3844),
+    (3001, 192, 1284), (5990, 192, 1284), (5990, 192, 3844), (5990, 192, 5124),
+    (9, 2048, 68), (37, 5120, 1284), (65, 5184, 100), (129, 3072, 772)])
+def test_linear_tile_shapes(wrs, ctx, n_tokens, n_in, n_out, x_dt):
+    """Every tile shape against float64 (the accumulation bound), a grouped call
+    bit for bit the separate ones (whatever shape the larger grid takes), and
+    16-bit output bit for bit the rounded f32 output."""
+    note(f"linear tiles T={n_tokens} K={n_in} N={n_out} x={x_dt}")
+    gen = torch.Generator(device="cuda").manual_seed(n_tokens + n_in + n_out)
+    x = torch.randn((n_tokens, n_in), generator=gen, device="cuda")
+    if x_dt == "f16":
+        x = x.half()
+    ws = [(torch.randn((n_out, n_in), generator=gen, device="cuda") * n_in ** -0.5).half()
+          for _ in range(3)]
+    bs = [torch.randn(n_out, generator=gen, device="cuda"), None,
+          torch.randn(n_out, generator=gen, device="cuda")]
+    outs = [torch.full((n_tokens, n_out), float("nan"), device="cuda") for _ in range(3)]
+    wrs.linear_group(x, ws, bs, outs, ctx=ctx)
+    for w, b, o in zip(ws, bs, outs):
+        one = torch.full_like(o, float("nan"))
+        wrs.linear(x, w, b, one, ctx=ctx)
+        assert torch.equal(o, one)
+        xd, wd = x.double(), w.double().T.contiguous()
+        exact = xd @ wd + (0 if b is None else b.double())
+        bound = n_in * 2.0 ** -23 * (xd.abs() @ wd.abs())
+        bound += 0 if b is None else 2.0 ** -23 * b.double().abs()
+        assert bool(((one.double() - exact).abs() <= bound).all())
+    half = torch.full((n_tokens, n_out), float("nan"), dtype=torch.float16, device="cuda")
+    wrs.linear(x, ws[0], bs[0], half, ctx=ctx)
+    assert torch.equal(half, outs[0].half())
+
+
+def test_linear_split_k_under_capture(wrs):
+    """A k-split projection captured before the context's scratch exists (no
+    split) and after it does: replays with eager calls between them match."""
+    note("linear split k capture")
+    c = wrs.Context(0)
+    c.use_torch_stream()
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.randn((37, 5120), generator=gen, device="cuda").half()
+    w = (torch.randn((1280, 5120), generator=gen, device="cuda") * 5120 ** -0.5).half()
+    out, eager = (torch.zeros((37, 1280), device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+
+    def capture():
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            c.use_torch_stream()
+            wrs.linear(x, w, None, out, ctx=c)
+        c.use_torch_stream()
+        return g
+
+    early = capture()
+    wrs.linear(x, w, None, eager, ctx=c)  # allocates the scratch
+    late = capture()
+    bound = 5120 * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T.contiguous())
+    for i in range(4):
+        for g, same in ((early, False), (late, True)):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            if same:
+                assert torch.equal(out, eager)
+            else:
+                assert bool(((out - eager).double().abs() <= bound).all())
+            wrs.linear(x, w, None, eager, ctx=c)
+    c.close()

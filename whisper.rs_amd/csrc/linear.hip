@@ -6,34 +6,44 @@
 //
 // K6 (linear_f16w): D^T = W X^T on v_mfma_f32_32x32x16_f16. Both operands are
 //   "k-contiguous" rows as stored (W [n_out][n_in] f16, X [n_tokens][k] f16),
-//   so neither needs a transpose. A workgroup of 8 waves owns a tile of 256
-//   output features x 256 tokens; wave (wm, wn) owns 128 x 64 of it as 4 x 2
-//   MFMA tiles (6 operand reads per 8 MFMAs). k advances 64 per LDS stage
-//   through two stages (128 KB): tiles move global -> LDS with
-//   buffer_load ... lds (no staging registers), one stage ahead of the
-//   MFMAs, and rows past the matrix edge read as zero through the buffer
-//   range check; one barrier per stage (64-k stages halved the barriers of
-//   the earlier 32-k, three-stage ring: 0.285 -> 0.267 ms). LDS rows (128
-//   bytes) keep their 16-byte chunks XOR-permuted by the row index, so the 32
-//   rows read by one operand fetch spread over the banks (swz_f). Workgroups are ordered so
-//   that each XCD runs a compact block of 4 feature x 8 token tiles at a time.
-//   Measured on the large-v3 fused QKV shape (24000 x 1280 x 3840): this
-//   shape of tile reaches ~85% of the library GEMM on the same box.
+//   so neither needs a transpose. A workgroup owns a tile of output features x
+//   tokens (LinTile: 64 x 64 up to 256 x 256, picked by grid size in
+//   launch_parts); k advances 32 or 64 per LDS stage through a ring of 2 to 4
+//   stages: tiles move global -> LDS with buffer_load ... lds (no staging
+//   registers), rows past the matrix edge read as zero through the buffer range
+//   check, and one barrier separates stages. Inside a stage every 16-k step
+//   issues one MFMA per slot, with the LDS reads of the next step's operands
+//   and a share of the tile loads between them: left to itself the compiler
+//   reads two operands, waits, multiplies, and a wave alone on its SIMD idles
+//   for the LDS latency six times a stage (256 x 256 tiles, one round: 31 ->
+//   25 us at n_in 1280, 208 -> 171 us at 5120 with two parts). LDS rows keep
+//   their 16-byte chunks XOR-permuted by the row index, so the 32 rows read by
+//   one operand fetch spread over the banks (swz). Every tile shape adds k in
+//   the same order, so the shape does not change a result's bits.
+//   Bound: the larger tiles by LDS reads and DMA writes against the MFMAs (a
+//   128 x 64 wave reads 6 operands per 8 MFMAs) and by the f32 output, which
+//   one workgroup per CU does not overlap (6000 x 5120: 24 of 89 us); the
+//   small ones by the memory latency of a few stages.
 //   f32 activations go to the f16 matrix pipe through a pre-pass
 //   (linear_split_rows): each row is scaled by a power of two so that its
 //   largest element lies in [2^14, 2^15), then split into two f16 parts
 //   hi + lo that sum to it within 2^-22 relative (2^-25 of the row maximum
-//   where lo is subnormal). The GEMM then runs over k' = 2 n_in with the
-//   weight column k' mod n_in; each product carries at most that 2^-22
+//   where lo is subnormal). Both parts meet each W operand in turn (read once
+//   for the two); each product carries at most that 2^-22
 //   relative error, below what one f32 addition of the accumulation
 //   (dot_f16_f32, simd.rs:593-700) already rounds away. The epilogue multiplies by
 //   the row's 2^-shift (exact), adds the f32 bias and writes the output type
 //   at out + t * out_rs + (r / 64) * out_hs + r % 64: token-major rows
-//   (out_hs = 64) or the arena's [head][token][64] planes. A 16-bit tile
-//   passes through the freed stage buffers first and leaves as whole 512-byte
-//   token rows, 16 bytes per lane: stored straight from the MFMA layout (8
-//   bytes of 32 different rows per instruction) the same bytes took 2.2x as
-//   long to write. f32 output is stored straight from the MFMA layout.
+//   (out_hs = 64) or the arena's [head][token][64] planes. Each wave passes its
+//   tile through the freed stage buffers and stores 64- to 512-byte pieces of
+//   output rows, 16 bytes per lane: stored straight from the MFMA layout (pieces
+//   of 32 different rows per instruction) a 16-bit tile took 2.2x as long.
+//   Few rows over long k (37 x 5120 -> 1280) leave too few tiles for the chip:
+//   32 x 64 tiles then split k over workgroups, merged through memory.
+//   Measured (f32 x, f32 output, pre-pass included, against one 256 x 256 shape
+//   for every call): 37 x 1280 x 1280 54 -> 11.4 us, 1500 x 1280 x 1280 65 ->
+//   23 us, 1500 x 5120 -> 1280 208 -> 57 us, 37 x 5120 -> 1280 192 -> 16 us,
+//   6000 x 1280 -> 5120 166 -> 153 us.
 #include "wrs_internal.hpp"
 
 #include <algorithm>
@@ -49,24 +59,41 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kWaves = 8;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kBM = 256;          // output features per workgroup (MFMA M)
-constexpr int kBN = 256;          // tokens per workgroup (MFMA N)
-constexpr int kBK = 64;           // k per LDS stage: one 128-byte row per feature/token
-constexpr int kStages = 2;        // LDS ring
-constexpr int kStageA = kBM * kBK;  // f16 elements per stage
-constexpr int kStageB = kBN * kBK;
-constexpr int kDmaA = kBM / kWaves / 8;  // 1 KB DMA instructions per wave per stage (4)
-constexpr int kDmaB = kBN / kWaves / 8;  // (4)
+// Tile shape of one workgroup: FT output features x TT tokens, WM x WN of it per
+// wave in 32 x 32 MFMA tiles; k advances BK per LDS stage through NS stages; P
+// f16 parts of every x row share each W stage.
+template <int FT_, int TT_, int WM_, int WN_, int BK_, int NS_, int P_, bool kSlots_ = true>
+struct LinTile {
+  static constexpr bool kSlots = kSlots_;  // 16-k steps in hand-placed slots
+  static constexpr int FT = FT_, TT = TT_, WM = WM_, WN = WN_, BK = BK_, NS = NS_, P = P_;
+  static constexpr int MI = WM / 32, NJ = WN / 32;       // MFMA tiles of a wave
+  static constexpr int kWavesM = FT / WM;
+  static constexpr int kWaves = kWavesM * (TT / WN), kThreads = 64 * kWaves;
+  static constexpr int KS = BK / 16;                     // 16-k steps per stage
+  static constexpr int kStage = (FT + P * TT) * BK;      // f16 elements of a stage: W rows, x rows
+  static constexpr int kChunks = BK / 8;                 // 16-byte chunks of an LDS row
+  static constexpr int kDmaRows = 64 / kChunks;          // rows one 1 KB DMA instruction moves
+  static constexpr int kDmaA = FT / kDmaRows / kWaves;   // DMA instructions per wave and stage
+  static constexpr int kDmaB = P * TT / kDmaRows / kWaves;
+  static constexpr int kDma = kDmaA + kDmaB;
+  static constexpr int kMfmas = P * MI * NJ, kReads = MI + P * NJ;  // of one 16-k step
+  static constexpr int kGroupM = FT >= 256 ? 4 : 1024 / FT;  // feature tiles an XCD walks at a time
+  static_assert(kDmaA * kDmaRows * kWaves == FT && kDmaB * kDmaRows * kWaves == P * TT,
+                "every wave moves whole DMA instructions");
+  static_assert(BK == 32 || BK == 64, "swizzles for 64- and 128-byte rows");
+  static_assert(KS % 2 == 0, "operands alternate between two register sets");
+  static_assert(kWaves * WM * 128 <= NS * kStage * 2, "32 staged f32 token rows per wave fit");
+};
 
-// 16-byte chunk c of LDS row r sits at slot c ^ f(r), f(r) = (r >> 1) & 7.
-// An operand fetch reads one chunk of 32 consecutive rows; 16 lanes at a time
-// cover 256 bytes of banks, i.e. two 128-byte rows per bank line, so the 8
-// even (and the 8 odd) rows of every 16 must land in distinct slots; f does
+// 16-byte chunk c of LDS row r sits at slot c ^ f(r). An operand fetch reads
+// one chunk of 32 consecutive rows; 16 lanes at a time cover the 256 bytes of
+// banks, i.e. two 128-byte (four 64-byte) rows per bank line, so the rows of
+// every 16 that share a place in the line must land in distinct slots; f does
 // that.
-__device__ inline int swz_f(int row) { return (row >> 1) & 7; }
-__device__ inline int swz(int row, int chunk) { return chunk ^ swz_f(row); }
+template <int BK>
+__device__ inline int swz(int row, int chunk) {
+  return BK == 64 ? chunk ^ ((row >> 1) & 7) : chunk ^ ((row >> 2) & 3);
+}
 
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
@@ -76,6 +103,11 @@ __device__ inline int swz(int row, int chunk) { return chunk ^ swz_f(row); }
 // it with explicit vmcnt waits and barriers. m0 is used by nothing else here.
 __device__ inline void dma16(u32x4 rsrc, uint32_t lds, uint32_t voff) {
   asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+               :: "v"(voff), "s"(rsrc), "s"(lds) : "memory", "m0");
+}
+// The same with 4 bytes per lane, at m0 + 4 * lane.
+__device__ inline void dma4(u32x4 rsrc, uint32_t lds, uint32_t voff) {
+  asm volatile("s_mov_b32 m0, %2\n\tbuffer_load_dword %0, %1, 0 offen lds"
                :: "v"(voff), "s"(rsrc), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
@@ -95,25 +127,20 @@ __device__ inline uint32_t lds_addr(const void* p) {
       reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p));
 }
 
-// This wave's stage landed (no DMA load left in flight) and its LDS writes are
-// done, then all waves meet.
+// At most N of this wave's DMA loads are still in flight and its LDS accesses
+// are done, then all waves meet.
+template <int N>
 __device__ inline void stage_barrier() {
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
 
-// Physical workgroup id -> tile. The hardware hands linear ids round-robin to
-// the 8 XCDs; each XCD is given a contiguous range of logical ids instead, and
-// logical ids walk groups of kGroupM feature tiles with the token tiles
-// outermost inside a group, so the ~32 workgroups an XCD runs at once cover
-// 4 feature x 8 token tiles and share their operand stages in its L2.
-constexpr int kGroupM = 4;
-__device__ inline void tile_of(int pid, int n_fm, int n_tn, int& fm, int& tn) {
-  const int nwg = n_fm * n_tn;
-  const int xcd = pid & 7, k = pid >> 3;
-  const int per = nwg >> 3, rem = nwg & 7;
-  const int id = xcd < rem ? xcd * (per + 1) + k : rem * (per + 1) + (xcd - rem) * per + k;
+// Tile id -> feature and token tile: ids walk groups of kGroupM feature tiles
+// with the token tiles outermost inside a group, so that the workgroups an XCD
+// runs at once (a contiguous range of ids) share their operand stages in its L2.
+template <int kGroupM>
+__device__ inline void tile_of(int id, int n_fm, int n_tn, int& fm, int& tn) {
   const int group = id / (kGroupM * n_tn);
   const int gm = min(kGroupM, n_fm - group * kGroupM);
   const int in = id - group * kGroupM * n_tn;
@@ -121,210 +148,304 @@ __device__ inline void tile_of(int pid, int n_fm, int n_tn, int& fm, int& tn) {
   tn = in / gm;
 }
 
-template <typename OutT>
-__global__ __launch_bounds__(kThreads) void linear_f16w(LinearArgs a) {
-  __shared__ __attribute__((aligned(16))) _Float16 lds_ab[kStages * (kStageA + kStageB)];
-  __shared__ __attribute__((aligned(16))) float bias_s[kBM];  // this tile's bias
-  _Float16* const lds_a = lds_ab;
-  _Float16* const lds_b = lds_ab + kStages * kStageA;
+constexpr int kLinCounterStride = 32;  // words between merge counters (one 128-byte line)
+constexpr int kLinMaxSplits = 8;
+constexpr int kLinPartFloats = 2048;   // partial sums of one 32 x 64 tile
+
+template <typename OutT, class C>
+__global__ __launch_bounds__(C::kThreads, 1) void linear_f16w(LinearArgs a, int n_splits) {
+  constexpr int MI = C::MI, NJ = C::NJ, P = C::P, BK = C::BK, NS = C::NS, KS = C::KS;
+  __shared__ __attribute__((aligned(128))) _Float16 lds[NS * C::kStage];
+  __shared__ __attribute__((aligned(16))) float bias_s[(C::FT + 63) / 64 * 64];
+  __shared__ int merger;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int wm = wave & 1, wn = wave >> 1;  // 128-feature and 64-token block of this wave
-  const int n_fm = (a.n_out + kBM - 1) / kBM, n_tn = (a.n_tokens + kBN - 1) / kBN;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = wave % C::kWavesM, wn = wave / C::kWavesM;
+  const int n_fm = (a.n_out + C::FT - 1) / C::FT, n_tn = (a.n_tokens + C::TT - 1) / C::TT;
+  // Workgroup ids run over (group, k split, tile); each XCD takes a contiguous
+  // range of them.
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int tiles = n_fm * n_tn;
+  const int grp = id / (tiles * n_splits);
+  const int split = (id / tiles) % n_splits;
   int fm, tn;
-  tile_of(blockIdx.x, n_fm, n_tn, fm, tn);
-  const int m0 = fm * kBM;  // first output feature
-  const int n0 = tn * kBN;  // first token
-  const int grp = blockIdx.z;
+  tile_of<C::kGroupM>(id % tiles, n_fm, n_tn, fm, tn);
+  const int m0 = fm * C::FT;  // first output feature
+  const int n0 = tn * C::TT;  // first token
 
-  // DMA sources. A wave moves rows 32*wave.. of the A and of the B tile, 16
-  // rows per instruction; lane i lands at slot i%4 of row i/4 and so fetches
-  // logical chunk swz(row, i%4). Rows past n_out / n_tokens fall
-  // outside the buffer ranges and read as zero.
+  // Row scales of this lane's tokens, requested before the stages.
+  const int orow = lane & 31, kgrp = lane >> 5;
+  float rs[NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    const int t = n0 + wn * C::WN + 32 * j + orow;
+    rs[j] = (a.row_scale && t < a.n_tokens) ? a.row_scale[t] : 1.0f;
+  }
+
+  // DMA sources. An instruction moves kDmaRows LDS rows; lane i lands at slot
+  // i % kChunks of row i / kChunks and so fetches logical chunk swz(row, slot).
+  // Rows past n_out / n_tokens fall outside the buffer ranges and read as zero.
   const u32x4 wrs = buffer_rsrc(a.w[grp], static_cast<uint32_t>(
                                               static_cast<int64_t>(a.n_out) * a.n_in * 2));
   const u32x4 xrs = buffer_rsrc(
-      a.x, static_cast<uint32_t>(((static_cast<int64_t>(a.n_tokens) - 1) * a.x_rs + a.k_total) *
-                                 2));
-  uint32_t aoff[kDmaA], boff[kDmaB];
+      a.x, static_cast<uint32_t>(((static_cast<int64_t>(a.n_tokens) - 1) * a.x_rs +
+                                  static_cast<int64_t>(P) * a.n_in) * 2));
+  uint32_t aoff[C::kDmaA], boff[C::kDmaB];
 #pragma unroll
-  for (int j = 0; j < kDmaA; ++j) {
-    const int row = wave * (kBM / kWaves) + 8 * j + (lane >> 3);
-    const int ch = swz(row, lane & 7);
+  for (int j = 0; j < C::kDmaA; ++j) {
+    const int row = (wave * C::kDmaA + j) * C::kDmaRows + lane / C::kChunks;
+    const int ch = swz<BK>(row, lane % C::kChunks);
     aoff[j] = static_cast<uint32_t>((static_cast<int64_t>(m0 + row) * a.n_in + ch * 8) * 2);
   }
 #pragma unroll
-  for (int j = 0; j < kDmaB; ++j) {
-    const int row = wave * (kBN / kWaves) + 8 * j + (lane >> 3);
-    const int ch = swz(row, lane & 7);
-    boff[j] = static_cast<uint32_t>((static_cast<int64_t>(n0 + row) * a.x_rs + ch * 8) * 2);
+  for (int j = 0; j < C::kDmaB; ++j) {
+    const int row = (wave * C::kDmaB + j) * C::kDmaRows + lane / C::kChunks;
+    const int ch = swz<BK>(row, lane % C::kChunks);
+    boff[j] = static_cast<uint32_t>((static_cast<int64_t>(n0 + row % C::TT) * a.x_rs +
+                                     static_cast<int64_t>(row / C::TT) * a.n_in + ch * 8) * 2);
   }
-  const uint32_t a_lds = lds_addr(lds_a) + wave * (kBM / kWaves) * kBK * 2;
-  const uint32_t b_lds = lds_addr(lds_b) + wave * (kBN / kWaves) * kBK * 2;
-  auto issue_stage = [&](int kt) {
-    const uint32_t kx = static_cast<uint32_t>(kt * kBK * 2);             // x' column, bytes
-    const uint32_t kw = static_cast<uint32_t>((kt * kBK) % a.n_in * 2);  // W column, bytes
-    const int s = kt % kStages;
-    const uint32_t ab = __builtin_amdgcn_readfirstlane(a_lds + s * kStageA * 2);
-    const uint32_t bb = __builtin_amdgcn_readfirstlane(b_lds + s * kStageB * 2);
-#pragma unroll
-    for (int j = 0; j < kDmaA; ++j) dma16(wrs, ab + j * 1024, aoff[j] + kw);
-#pragma unroll
-    for (int j = 0; j < kDmaB; ++j) dma16(xrs, bb + j * 1024, boff[j] + kx);
+  const uint32_t a_lds = lds_addr(lds) + wave * C::kDmaA * 1024;
+  const uint32_t b_lds = lds_addr(lds) + C::FT * BK * 2 + wave * C::kDmaB * 1024;
+  const int n_kt = a.n_in / BK;
+  const int kt0 = n_kt * split / n_splits, kt1 = n_kt * (split + 1) / n_splits;
+  // DMA instruction d of stage kt into ring slot `slot`. Stages past the last
+  // are issued too, out of the buffers' ranges (spans stay below 2^31): they
+  // touch no memory, and every step has the same number in flight.
+  auto dma = [&](int d, int kt, int slot) __attribute__((always_inline)) {
+    const uint32_t ko = kt < kt1 ? static_cast<uint32_t>(kt * BK * 2) : 0x80000000u;
+    const uint32_t so = __builtin_amdgcn_readfirstlane(slot * C::kStage * 2);
+    if (d < C::kDmaA)
+      dma16(wrs, a_lds + so + d * 1024, aoff[d] + ko);
+    else
+      dma16(xrs, b_lds + so + (d - C::kDmaA) * 1024, boff[d - C::kDmaA] + ko);
   };
 
-  f32x16 acc[4][2];
+  f32x16 acc[MI][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < NJ; ++j)
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
 
-  // Operand rows of this lane: feature/token l % 32 of each 32-row MFMA tile,
-  // k-group l / 32 (8 consecutive k) of each 16-k step.
-  const int orow = lane & 31, kgrp = lane >> 5;
-  int aread[4][kBK / 16], bread[2][kBK / 16];
+  // Operand reads: row l % 32 of each 32-row MFMA tile (32 rows on, the same
+  // swizzle), k-group l / 32 (8 consecutive k) of a 16-k step.
+  const char* const ldsb = reinterpret_cast<const char*>(lds);
+  int aaddr[KS], baddr[KS];
 #pragma unroll
-  for (int ks = 0; ks < kBK / 16; ++ks) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ra = wm * 128 + i * 32 + orow;
-      aread[i][ks] = ra * kBK + swz(ra, 2 * ks + kgrp) * 8;
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int rb = wn * 64 + j * 32 + orow;
-      bread[j][ks] = rb * kBK + swz(rb, 2 * ks + kgrp) * 8;
-    }
+  for (int ks = 0; ks < KS; ++ks) {
+    const int ch = swz<BK>(orow, 2 * ks + kgrp) * 16;
+    aaddr[ks] = (wm * C::WM + orow) * BK * 2 + ch;
+    baddr[ks] = (C::FT + wn * C::WN + orow) * BK * 2 + ch;
   }
+  struct Frag {
+    f16x8 a[MI], b[P][NJ];
+  };
+  auto read = [&](Frag& f, int r, int slot, int ks) __attribute__((always_inline)) {
+    const char* const st = ldsb + slot * (C::kStage * 2);
+    if (r < MI)
+      f.a[r] = *reinterpret_cast<const f16x8*>(st + aaddr[ks] + r * (32 * BK * 2));
+    else
+      f.b[(r - MI) / NJ][(r - MI) % NJ] = *reinterpret_cast<const f16x8*>(
+          st + baddr[ks] + ((r - MI) / NJ * C::TT + (r - MI) % NJ * 32) * (BK * 2));
+  };
 
-  const int n_kt = a.k_total / kBK;
-  issue_stage(0);
-  // The tile's bias goes to LDS while the first stage is in flight (the loop's
-  // barriers order the write before the epilogue's reads): the epilogue then
-  // reads it without a global-memory round trip per store.
+  // The tile's bias goes to LDS (zeros without one) ahead of the first stage:
+  // the stage barriers cover it, and the epilogue reads it without a round trip.
   {
-    const float* bias_g = a.bias[grp];
-    if (threadIdx.x < kBM)
-      bias_s[threadIdx.x] =
-          (bias_g && m0 + static_cast<int>(threadIdx.x) < a.n_out) ? bias_g[m0 + threadIdx.x] : 0.0f;
+    const u32x4 brs = buffer_rsrc(a.bias[grp] ? a.bias[grp] : reinterpret_cast<const float*>(a.x),
+                                  a.bias[grp] ? static_cast<uint32_t>(a.n_out * 4) : 0u);
+    if (wave < (C::FT + 63) / 64)
+      dma4(brs, lds_addr(bias_s) + wave * 256, static_cast<uint32_t>((m0 + wave * 64 + lane) * 4));
   }
-  for (int kt = 0; kt < n_kt; ++kt) {
-    stage_barrier();
-    if (kt + 1 < n_kt) issue_stage(kt + 1);  // its buffer was last read in step kt - 1
-    const _Float16* as = lds_a + (kt % kStages) * kStageA;
-    const _Float16* bs = lds_b + (kt % kStages) * kStageB;
-    f16x8 av[kBK / 16][4], bv[kBK / 16][2];
 #pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks) {
+  for (int s = 0; s < NS - 1; ++s)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[ks][i] = *reinterpret_cast<const f16x8*>(as + aread[i][ks]);
+    for (int d = 0; d < C::kDma; ++d) dma(d, kt0 + s, s);
+
+  // One 16-k step: its MFMAs, one per slot, with the operand reads of the next
+  // step and a share of the tile loads dealt between them, so that a wave alone
+  // on its SIMD keeps the matrix pipe fed. The order of the sums is k steps
+  // ascending, high part before low.
+  constexpr int kM = C::kMfmas, kR = C::kReads;
+  auto kstep = [&](const Frag& cur, Frag& nxt, int slot, int ks, int d0, int d1, int kt_dma,
+                   int slot_dma) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j) bv[ks][j] = *reinterpret_cast<const f16x8*>(bs + bread[j][ks]);
+    for (int n = 0; n < kM; ++n) {
+#pragma unroll
+      for (int r = 0; r < kR; ++r)
+        if (r * kM / kR == n) read(nxt, r, slot, ks);
+#pragma unroll
+      for (int d = 0; d < C::kDma; ++d)
+        if (d >= d0 && d < d1 && (d - d0) * kM / (d1 - d0) == n) dma(d, kt_dma, slot_dma);
+      const int p = n / (MI * NJ), i = n / NJ % MI, j = n % NJ;
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(cur.a[i], cur.b[p][j], acc[i][j], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
     }
+  };
+  if constexpr (C::kSlots) {
+    Frag f0, f1;
+    stage_barrier<(NS - 2) * C::kDma>();
+  #pragma unroll
+    for (int r = 0; r < kR; ++r) read(f0, r, 0, 0);
+    // The first share of stage kt0 + NS - 1, which a step before kt0 would issue.
+  #pragma unroll
+    for (int d = 0; d < C::kDma / KS; ++d) dma(d, kt0 + NS - 1, NS - 1);
+    int slot = 0;
+    // Stage kt, whose first operands are in `f`. In its last step stage kt + 1
+    // has landed and nobody reads stage kt any more, whose buffer takes stage
+    // kt + NS: its loads are dealt over that step and the next stage's others.
+    auto stage = [&](int kt, Frag& f, Frag& g) __attribute__((always_inline)) {
+  #pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        Frag& cur = ks % 2 == 0 ? f : g;
+        Frag& nxt = ks % 2 == 0 ? g : f;
+        if (ks + 1 < KS) {
+          kstep(cur, nxt, slot, ks + 1, C::kDma * (ks + 1) / KS, C::kDma * (ks + 2) / KS,
+                kt + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+        } else {
+          stage_barrier<(NS - 2) * C::kDma>();
+          const int freed = slot;
+          slot = slot + 1 == NS ? 0 : slot + 1;
+          kstep(cur, nxt, slot, 0, 0, C::kDma / KS, kt + NS, freed);
+        }
+      }
+    };
+    for (int kt = kt0; kt < kt1; ++kt) stage(kt, f0, f1);
+  } else {
+    // A stage at a time, in the compiler's order.
+    int slot = 0;
+    for (int kt = kt0; kt < kt1; ++kt) {
+      stage_barrier<(NS - 2) * C::kDma>();
 #pragma unroll
-    for (int ks = 0; ks < kBK / 16; ++ks)
+      for (int d = 0; d < C::kDma; ++d) dma(d, kt + NS - 1, slot == 0 ? NS - 1 : slot - 1);
+      Frag f[KS];
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[ks][i], bv[ks][j], acc[i][j], 0, 0, 0);
+        for (int r = 0; r < kR; ++r) read(f[ks], r, slot, ks);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+        for (int n = 0; n < kM; ++n) {
+          const int p = n / (MI * NJ), i = n / NJ % MI, j = n % NJ;
+          acc[i][j] =
+              __builtin_amdgcn_mfma_f32_32x32x16_f16(f[ks].a[i], f[ks].b[p][j], acc[i][j], 0, 0, 0);
+        }
+      slot = slot + 1 == NS ? 0 : slot + 1;
+    }
+  }
+  stage_barrier<0>();  // no load in flight, nobody reads a stage any more
+
+  if constexpr (C::FT == 32 && C::TT == 64) {
+    if (n_splits > 1) {
+      // Split k: every wave publishes its sums lane by lane with agent-scope
+      // stores and waits for them; the workgroup that counts in last adds the
+      // splits in split order (the bits do not depend on the arrival order),
+      // re-arms the tile's counter and writes the tile.
+      static_assert(MI == 1 && NJ == 1, "one MFMA tile per wave");
+      const int unit = grp * tiles + id % tiles;
+      const bool valid = n0 + wn * C::WN + orow < a.n_tokens;
+      float* const base = a.part + static_cast<int64_t>(unit) * n_splits * kLinPartFloats +
+                          wave * 1024 + lane;
+      float* const mine = base + split * kLinPartFloats;
+      if (valid) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) st_agent(mine + e * 64, acc[0][0][e]);
+      }
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      unsigned* const counter = a.counters + static_cast<int64_t>(unit) * kLinCounterStride;
+      if (tid == 0)
+        merger = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+                 static_cast<unsigned>(n_splits - 1);
+      __syncthreads();
+      if (!merger) return;
+      float px[kLinMaxSplits][16];
+#pragma unroll
+      for (int s = 0; s < kLinMaxSplits; ++s) {
+        if (s >= n_splits) break;
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          px[s][e] = valid && s != split ? ld_agent(base + s * kLinPartFloats + e * 64) : 0.f;
+      }
+      f32x16 sum = {};
+#pragma unroll
+      for (int s = 0; s < kLinMaxSplits; ++s) {
+        if (s >= n_splits) break;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sum[e] += s == split ? acc[0][0][e] : px[s][e];
+      }
+      acc[0][0] = sum;
+      if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 
-  // Epilogue: acc[i][j][e] is feature m0 + 64 wm + 32 i + 8 (e / 4) + 4 kgrp + e % 4
-  // of token n0 + 64 wn + 32 j + orow.
-  OutT* out = reinterpret_cast<OutT*>(a.out[grp]);
-  const float* bias = a.bias[grp];
-  if constexpr (sizeof(OutT) == 2) {
-    // 16-bit output: the tile goes through LDS (the stage buffers, 128 KB:
-    // 256 token rows of 512 bytes, 16-byte chunk c of row t at c ^ (t % 32)),
-    // then leaves as whole rows: 64 lanes store 2 rows of 512 bytes.
-    char* ot = reinterpret_cast<char*>(lds_a);  // lds_a and lds_b are one 128 KB span
-    // this lane's 64 bias values, read before any LDS write of the tile, so
-    // that no read waits behind the writes
-    f32x4 bv[4][4];
+  // Epilogue: acc[i][j][e] is feature 32 i + 8 (e / 4) + 4 kgrp + e % 4 of the
+  // wave's part, token 32 j + orow. A wave passes 32 tokens at a time through
+  // its part of the stage buffers, as rows of its WM features (16-byte chunk c
+  // of row t at c ^ (t mod chunks)), and stores whole pieces of output rows.
+  constexpr int kRowBytes = C::WM * static_cast<int>(sizeof(OutT));
+  constexpr int kCh = kRowBytes / 16;
+  constexpr int kPer = 16 / static_cast<int>(sizeof(OutT));  // values of a chunk
+  char* const ot = reinterpret_cast<char*>(lds) + wave * (32 * kRowBytes);
+  OutT* const out = reinterpret_cast<OutT*>(a.out[grp]);
+  const bool v16 =
+      sizeof(OutT) == 4 ||
+      ((reinterpret_cast<uintptr_t>(out) | (a.out_rs * 2) | (a.out_hs * 2)) & 15) == 0;
+  auto wave_sync = [] {
+    // LDS operations of one wave complete in order: only the compiler must keep it.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < NJ; ++j) {
+    wave_sync();
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        bv[i][g] = bias ? *reinterpret_cast<const f32x4*>(&bias_s[wm * 128 + i * 32 + 8 * g + 4 * kgrp])
-                        : f32x4{0.f, 0.f, 0.f, 0.f};
-    __syncthreads();                             // every wave is done with the last stage
+    for (int i = 0; i < MI; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int tl = wn * 64 + j * 32 + orow;
-      const int t = n0 + tl;
-      const float rs = (a.row_scale && t < a.n_tokens) ? a.row_scale[t] : 1.0f;
+      for (int g = 0; g < 4; ++g) {
+        const int fl = i * 32 + 8 * g + 4 * kgrp;  // feature within the staged row
+        const f32x16& s = acc[i][j];
+        f32x4 v = {s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
+        v *= rs[j];
+        v += *reinterpret_cast<const f32x4*>(&bias_s[wm * C::WM + fl]);
+        if (a.act == kActGelu) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int fl = wm * 128 + i * 32 + 8 * g + 4 * kgrp;  // feature within the tile
-          f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
-                     acc[i][j][4 * g + 3]};
-          v *= rs;
-          v += bv[i][g];
-          if (a.act == kActGelu) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
-          }
-          u32x2 h;
-          if constexpr (__is_same(OutT, __bf16)) {
-            typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-            h = __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
-          } else {
-            typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-            h = __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4));
-          }
-          const int chunk = (fl >> 3) ^ (tl & 31);
-          *reinterpret_cast<u32x2*>(ot + tl * 512 + chunk * 16 + (fl & 4) * 2) = h;
+          for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
         }
-    }
-    __syncthreads();
-    const bool v16 = ((reinterpret_cast<uintptr_t>(out) | (a.out_rs * 2) | (a.out_hs * 2)) & 15) == 0;
-    const int c = lane & 31;  // 16-byte chunk: features 8c .. 8c + 7 of the row
-    const int r = m0 + 8 * c;
-    OutT* ocol = out + static_cast<int64_t>(r >> 6) * a.out_hs + (r & 63);
+        const int at = orow * kRowBytes + (((fl / kPer) ^ (orow & (kCh - 1))) * 16);
+        if constexpr (sizeof(OutT) == 4) {
+          *reinterpret_cast<f32x4*>(ot + at) = v;
+        } else if constexpr (__is_same(OutT, __bf16)) {
+          typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+          *reinterpret_cast<u32x2*>(ot + at + (fl & 4) * 2) =
+              __builtin_bit_cast(u32x2, __builtin_convertvector(v, bf16x4));
+        } else {
+          *reinterpret_cast<u32x2*>(ot + at + (fl & 4) * 2) =
+              __builtin_bit_cast(u32x2, __builtin_convertvector(v, f16x4v));
+        }
+      }
+    wave_sync();
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const int tl = wave * 32 + 2 * q + (lane >> 5);
-      const int t = n0 + tl;
-      const u32x4 h = *reinterpret_cast<const u32x4*>(ot + tl * 512 + ((c ^ (tl & 31)) * 16));
+    for (int q = 0; q < kCh / 2; ++q) {
+      const int row = (q * 64 + lane) / kCh, c = (q * 64 + lane) % kCh;
+      const int t = n0 + wn * C::WN + 32 * j + row;
+      const int r = m0 + wm * C::WM + c * kPer;
+      const u32x4 h =
+          *reinterpret_cast<const u32x4*>(ot + row * kRowBytes + ((c ^ (row & (kCh - 1))) * 16));
       if (t < a.n_tokens && r < a.n_out) {
-        OutT* p = ocol + static_cast<int64_t>(t) * a.out_rs;
-        if (v16 && r + 8 <= a.n_out) {
+        OutT* p = out + static_cast<int64_t>(t) * a.out_rs +
+                  static_cast<int64_t>(r >> 6) * a.out_hs + (r & 63);
+        if (sizeof(OutT) == 4 || (v16 && r + 8 <= a.n_out)) {
           *reinterpret_cast<u32x4*>(p) = h;
         } else {
           *reinterpret_cast<u32x2*>(p) = u32x2{h[0], h[1]};
           if (r + 8 <= a.n_out) *reinterpret_cast<u32x2*>(p + 4) = u32x2{h[2], h[3]};
         }
       }
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int t = n0 + wn * 64 + j * 32 + orow;
-      if (t >= a.n_tokens) continue;
-      const float rs = a.row_scale ? a.row_scale[t] : 1.0f;
-      OutT* orow_p = out + static_cast<int64_t>(t) * a.out_rs;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int r = m0 + wm * 128 + i * 32 + 8 * g + 4 * kgrp;
-          if (r >= a.n_out) continue;
-          f32x4 v = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
-                     acc[i][j][4 * g + 3]};
-          v *= rs;
-          if (bias) v += *reinterpret_cast<const f32x4*>(&bias_s[r - m0]);
-          if (a.act == kActGelu) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = gelu_tanh(v[e]);
-          }
-          *reinterpret_cast<f32x4*>(orow_p + static_cast<int64_t>(r >> 6) * a.out_hs + (r & 63)) = v;
-        }
     }
   }
 }
@@ -1091,16 +1212,151 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
   return hipGetLastError();
 }
 
+namespace {
+
+// CUs of the current device, read once.
+int linear_cus() {
+  static const int cus = [] {
+    int dev = 0, n = 256;
+    if (hipGetDevice(&dev) == hipSuccess)
+      (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    return n;
+  }();
+  return cus;
+}
+
+int64_t n_tiles(const LinearArgs& a, int ft, int tt) {
+  return static_cast<int64_t>((a.n_out + ft - 1) / ft) * ((a.n_tokens + tt - 1) / tt);
+}
+
+// k splits of 32 x 64 tiles: as many as fill the CUs once, each of at least 1024
+// k. The merge costs a chain of memory round trips: 37 rows, f32: 5120 -> 1280
+// takes 16.0 us in 5 splits, 29.6 in one pass of 64 x 64 tiles; 1280 -> 1280
+// 11.6 in 6 splits and 11.4 without. By the shape of one group, so that a
+// grouped call sums in the order of separate calls.
+int linear_splits(const LinearArgs& a) {
+  const int64_t t = n_tiles(a, 32, 64);
+  const int64_t s = std::min<int64_t>({linear_cus() / std::max<int64_t>(t, 1), a.n_in / 1024,
+                                       kLinMaxSplits});
+  return static_cast<int>(std::max<int64_t>(s, 1));
+}
+
+template <typename OutT, class C>
+hipError_t launch_tile(const LinearArgs& a, int splits, hipStream_t s) {
+  const int64_t wgs = n_tiles(a, C::FT, C::TT) * splits * a.n_groups;
+  if (wgs > 0x7fffffff) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL((linear_f16w<OutT, C>), dim3(static_cast<unsigned>(wgs)), dim3(C::kThreads),
+                     0, s, a, splits);
+  return hipGetLastError();
+}
+
+// A tile shape's time over `tiles` workgroups: fixed + per256 for every started
+// round of one workgroup per CU, in units of us at n_in = 1280 (every shape
+// grows alike with n_in, so one fit serves all), measured at 37 to 6000 rows
+// and 384 to 5120 features, f32 output.
+struct TileCost {
+  int ft, tt;
+  float fixed, round, tile;
+};
+float tile_cost(const LinearArgs& a, const TileCost& c) {
+  const int64_t n = n_tiles(a, c.ft, c.tt) * a.n_groups, cus = linear_cus();
+  return c.fixed + c.round * static_cast<float>((n + cus - 1) / cus) +
+         c.tile * static_cast<float>(n);
+}
+template <size_t N>
+int cheapest(const LinearArgs& a, const TileCost (&t)[N]) {
+  int best = 0;
+  for (size_t i = 1; i < N; ++i)
+    if (tile_cost(a, t[i]) < tile_cost(a, t[best])) best = static_cast<int>(i);
+  return best;
+}
+
+// Large tiles read the LDS least per MFMA but leave CUs idle on small grids: the
+// 256 x 256 tile alone took 31 us for any call of up to 3000 x 1280 outputs over
+// 1280 k (f16 x; 8 to 19 us with the shapes below).
+template <typename OutT>
+hipError_t launch_parts(const LinearArgs& a, int splits, hipStream_t s) {
+  if (a.parts == 2) {
+    if (splits > 1) return launch_tile<OutT, LinTile<32, 64, 32, 32, 64, 3, 2>>(a, splits, s);
+    static constexpr TileCost kCosts[] = {{64, 64, 6.f, 9.3f, 0.f},
+                                          {128, 64, 10.f, 13.f, 0.f},
+                                          {128, 64, 12.f, 11.5f, 0.f},
+                                          {256, 128, 18.f, 36.f, 0.f},
+                                          {256, 256, 0.f, 42.f, 0.14f}};
+    switch (cheapest(a, kCosts)) {
+      case 0: return launch_tile<OutT, LinTile<64, 64, 32, 32, 64, 3, 2>>(a, 1, s);
+      case 1: return launch_tile<OutT, LinTile<128, 64, 64, 32, 64, 4, 2>>(a, 1, s);
+      case 2: return launch_tile<OutT, LinTile<128, 64, 64, 32, 64, 2, 2>>(a, 1, s);
+      case 3: return launch_tile<OutT, LinTile<256, 128, 128, 64, 32, 2, 2>>(a, 1, s);
+      default: return launch_tile<OutT, LinTile<256, 256, 128, 64, 32, 3, 2>>(a, 1, s);
+    }
+  }
+  if (splits > 1) return launch_tile<OutT, LinTile<32, 64, 32, 32, 64, 4, 1>>(a, splits, s);
+  static constexpr TileCost kCosts[] = {{64, 64, 3.f, 5.f, 0.f},
+                                        {128, 64, 4.5f, 7.8f, 0.f},
+                                        {128, 128, 8.5f, 11.5f, 0.f},
+                                        {256, 256, 0.f, 24.f, 0.077f}};
+  switch (cheapest(a, kCosts)) {
+    case 0: return launch_tile<OutT, LinTile<64, 64, 32, 32, 64, 4, 1>>(a, 1, s);
+    case 1: return launch_tile<OutT, LinTile<128, 64, 64, 32, 64, 3, 1>>(a, 1, s);
+    case 2: return launch_tile<OutT, LinTile<128, 128, 64, 64, 64, 2, 1>>(a, 1, s);
+    default:
+      // Past one workgroup per CU the compiler's own order of a stage (all its
+      // reads, then the MFMAs) keeps the two waves of a SIMD further apart:
+      // 24000 x 3840 over 1280 k 246 against 277 us; 3000 x 3840, one round, 44.2
+      // against 42.7 with slots.
+      if (n_tiles(a, 256, 256) * a.n_groups > linear_cus())
+        return launch_tile<OutT, LinTile<256, 256, 128, 64, 64, 2, 1, false>>(a, 1, s);
+      return launch_tile<OutT, LinTile<256, 256, 128, 64, 64, 2, 1>>(a, 1, s);
+  }
+}
+
+template <typename OutT>
+hipError_t launch_groups(const LinearArgs& a, hipStream_t s) {
+  const int splits = a.part ? linear_splits(a) : 1;
+  // Groups that fit the split's scratch run together.
+  int per = a.n_groups;
+  if (splits > 1) {
+    const int64_t t = n_tiles(a, 32, 64);
+    per = static_cast<int>(std::min<int64_t>(
+        {a.n_groups, static_cast<int64_t>(a.part_floats) / (t * splits * kLinPartFloats),
+         static_cast<int64_t>(a.counter_words) / (t * kLinCounterStride)}));
+    if (per < 1) return hipErrorInvalidValue;
+  }
+  if (per == a.n_groups) return launch_parts<OutT>(a, splits, s);
+  for (int g0 = 0; g0 < a.n_groups; g0 += per) {
+    LinearArgs b = a;
+    b.n_groups = std::min(per, a.n_groups - g0);
+    for (int g = 0; g < b.n_groups; ++g) {
+      b.w[g] = a.w[g0 + g];
+      b.bias[g] = a.bias[g0 + g];
+      b.out[g] = a.out[g0 + g];
+    }
+    const hipError_t e = launch_parts<OutT>(b, splits, s);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+}  // namespace
+
 hipError_t launch_linear_f16w(const LinearArgs& a, DType out_dt, hipStream_t s) {
   if (a.n_tokens <= 0 || a.n_out <= 0 || a.n_groups <= 0) return hipSuccess;
-  dim3 grid(((a.n_out + kBM - 1) / kBM) * ((a.n_tokens + kBN - 1) / kBN), 1, a.n_groups);
   switch (out_dt) {
-    case kF32: hipLaunchKernelGGL(linear_f16w<float>, grid, dim3(kThreads), 0, s, a); break;
-    case kF16: hipLaunchKernelGGL(linear_f16w<_Float16>, grid, dim3(kThreads), 0, s, a); break;
-    case kBF16: hipLaunchKernelGGL(linear_f16w<__bf16>, grid, dim3(kThreads), 0, s, a); break;
+    case kF32: return launch_groups<float>(a, s);
+    case kF16: return launch_groups<_Float16>(a, s);
+    case kBF16: return launch_groups<__bf16>(a, s);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
+}
+
+bool linear_needs_split(const LinearArgs& a) { return linear_splits(a) > 1; }
+// t tiles in s splits with t * s <= CUs and s >= 2, for four groups at once.
+size_t linear_split_floats() {
+  return static_cast<size_t>(4) * linear_cus() * kLinPartFloats;
+}
+size_t linear_split_words() {
+  return static_cast<size_t>(4) * (linear_cus() / 2) * kLinCounterStride;
 }
 
 }  // namespace wrs

@@ -224,26 +224,29 @@ int run_exact(wrs_attn_ctx* c, const float* q, size_t q_floats, const float* k, 
   return WRS_OK;
 }
 
-// Scratch for a prefill schedule that splits blocks over workgroups (pf
-// floats of partials, cw counter words; 0 when it needs none). Outside capture
-// it is allocated here, at least the size every default split needs (so that
-// graphs captured later keep valid pointers), or grown for a forced schedule
-// on a larger grid; during capture the kernels take another schedule when
-// what exists does not fit. Hands the buffers to `a`.
-int split_scratch(wrs_attn_ctx* c, size_t pf, size_t cw, wrs::PrefillArgs& a) {
-  if (pf && !capturing(c)) {
-    int rc = grow(c, reinterpret_cast<void**>(&c->split_part), &c->split_part_bytes,
-                  std::max(pf, wrs::prefill_split_floats_min()) * sizeof(float), false);
-    if (rc) return rc;
-    rc = grow(c, reinterpret_cast<void**>(&c->split_counters), &c->split_counter_bytes,
-              std::max(cw, wrs::prefill_split_words_min()) * sizeof(unsigned), true);
-    if (rc) return rc;
-  }
+// Context scratch for launches that split a block or tile over workgroups (pf
+// floats of partials, cw counter words; 0 when the launch needs none). Outside
+// capture it is allocated here, at least the size that every default split of
+// either kind needs (so that graphs captured later keep valid pointers), or
+// grown for a forced prefill schedule on a larger grid; during capture the
+// kernels take another schedule when what exists does not fit.
+int split_scratch(wrs_attn_ctx* c, size_t pf, size_t cw) {
+  if (!pf || capturing(c)) return WRS_OK;
+  int rc = grow(c, reinterpret_cast<void**>(&c->split_part), &c->split_part_bytes,
+                std::max({pf, wrs::prefill_split_floats_min(), wrs::linear_split_floats()}) *
+                    sizeof(float),
+                false);
+  if (rc) return rc;
+  return grow(c, reinterpret_cast<void**>(&c->split_counters), &c->split_counter_bytes,
+              std::max({cw, wrs::prefill_split_words_min(), wrs::linear_split_words()}) *
+                  sizeof(unsigned),
+              true);
+}
+void give_scratch(wrs_attn_ctx* c, wrs::PrefillArgs& a) {
   a.split_part = c->split_part;
   a.split_part_floats = c->split_part_bytes / sizeof(float);
   a.split_counters = c->split_counters;
   a.split_counter_words = c->split_counter_bytes / sizeof(unsigned);
-  return WRS_OK;
 }
 
 int prefill_impl(wrs_attn_ctx* c, int q_dtype, const void* q, const wrs_layout& lq, int kv_dtype,
@@ -298,16 +301,18 @@ int prefill_impl(wrs_attn_ctx* c, int q_dtype, const void* q, const wrs_layout& 
       aligned16(v, lv, 8) && aligned16(out, lo, 4) && wrs::prefill_mfma16_supports(a)) {
     size_t pf = 0, cw = 0;
     wrs::prefill_mfma16_scratch(a, &pf, &cw);
-    const int rc = split_scratch(c, pf, cw, a);
+    const int rc = split_scratch(c, pf, cw);
     if (rc) return rc;
+    give_scratch(c, a);
     WRS_HIP(c, wrs::launch_prefill_mfma16(a, q_dtype == WRS_F16 ? wrs::kF16 : wrs::kBF16,
                                           c->stream));
     return WRS_OK;
   }
   size_t pf = 0, cw = 0;
   wrs::prefill_f32_scratch(a, &pf, &cw);
-  const int rc = split_scratch(c, pf, cw, a);
+  const int rc = split_scratch(c, pf, cw);
   if (rc) return rc;
+  give_scratch(c, a);
   WRS_HIP(c, wrs::launch_prefill_f32(a, static_cast<DType>(q_dtype), static_cast<DType>(kv_dtype),
                                      c->stream));
   return WRS_OK;
@@ -639,8 +644,10 @@ int wrs_attn_reserve(wrs_attn_ctx* c, const wrs_reserve* r) {
   }
   if (r->linear_tokens > static_cast<size_t>(wrs::kGemvMaxRows) && r->linear_n_in) {
     const size_t split_bytes =
-        align_up(r->linear_tokens * wrs::kSplitParts * r->linear_n_in * 2, 256);
+        align_up(r->linear_tokens * wrs::kSplitParts * static_cast<int64_t>(r->linear_n_in) * 2, 256);
     rc = grow(c, &c->lin_x, &c->lin_x_bytes, split_bytes + r->linear_tokens * 4, false);
+    if (rc) return rc;
+    rc = split_scratch(c, wrs::linear_split_floats(), wrs::linear_split_words());
     if (rc) return rc;
     if (r->linear_n_in > static_cast<size_t>(wrs::kSplitLnMax)) {
       rc = grow(c, reinterpret_cast<void**>(&c->ln_x), &c->ln_x_bytes,
@@ -1448,6 +1455,11 @@ int wrs_attn_capture_cross_heads_lse(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, 
 
 namespace {
 
+// A new context's split-row scratch: one encoder window of the widest rows
+// (1500 x 5120 in two f16 parts), so that a model's first pass allocates once
+// and does not grow it (a hipFree and hipMalloc pair: ~300 us).
+constexpr size_t kMinSplitRowsBytes = size_t{32} << 20;
+
 // Shared front half of the projection entry points: validates x and the
 // shape, splits f32 rows (normalized first with ln_g) into the context
 // scratch, and fills the x part of the launch arguments. Caller holds c->mu
@@ -1477,21 +1489,22 @@ int linear_prepare(wrs_attn_ctx* c, int x_dtype, const void* x, int64_t x_rs, si
     a.x = static_cast<const _Float16*>(x);
     a.x_rs = x_rs;
     a.row_scale = nullptr;
-    a.k_total = a.n_in;
+    a.parts = 1;
     return WRS_OK;
   }
   if (x_dtype != WRS_F32) return fail(c, WRS_EUNSUPPORTED, "x must be f32 or f16");
-  const size_t split_bytes = align_up(n_tokens * wrs::kSplitParts * n_in * 2, 256);
-  int rc = grow(c, &c->lin_x, &c->lin_x_bytes, split_bytes + n_tokens * 4, false);
+  const size_t split_bytes = align_up(n_tokens * wrs::kSplitParts * static_cast<int64_t>(n_in) * 2, 256);
+  int rc = grow(c, &c->lin_x, &c->lin_x_bytes,
+                std::max(split_bytes + n_tokens * 4, kMinSplitRowsBytes), false);
   if (rc) return rc;
   auto* xs = static_cast<_Float16*>(c->lin_x);
   auto* scale = reinterpret_cast<float*>(static_cast<char*>(c->lin_x) + split_bytes);
+  a.x_rs = wrs::kSplitParts * static_cast<int64_t>(n_in);
   WRS_HIP(c, wrs::launch_linear_split(static_cast<const float*>(x), x_rs, a.n_tokens, a.n_in,
                                       ln_g, ln_b, ln_eps, xs, scale, c->stream));
   a.x = xs;
-  a.x_rs = wrs::kSplitParts * static_cast<int64_t>(n_in);
   a.row_scale = scale;
-  a.k_total = wrs::kSplitParts * a.n_in;
+  a.parts = wrs::kSplitParts;
   return WRS_OK;
 }
 
@@ -1596,6 +1609,16 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
     a.w[gi] = static_cast<const _Float16*>(w[gi]);
     a.bias[gi] = bias ? bias[gi] : nullptr;
     a.out[gi] = out[gi];
+  }
+  if (wrs::linear_needs_split(a)) {
+    rc = split_scratch(c, wrs::linear_split_floats(), wrs::linear_split_words());
+    if (rc) return rc;
+    if (c->split_counters) {  // captured before any scratch: no split
+      a.part = c->split_part;
+      a.part_floats = c->split_part_bytes / sizeof(float);
+      a.counters = c->split_counters;
+      a.counter_words = c->split_counter_bytes / sizeof(unsigned);
+    }
   }
   WRS_HIP(c, wrs::launch_linear_f16w(a, static_cast<wrs::DType>(out_dtype), c->stream));
   return WRS_OK;

@@ -194,8 +194,8 @@ hipError_t launch_capture_cross_f32(const CaptureArgs& a, hipStream_t s);
 
 // Projections with f16 weights (quant.rs:415-473 semantics):
 // out(t, r) = row_scale[t] * (W[r] . x'[t]) + bias[r] with W [n_out][n_in] f16
-// and x' [n_tokens][k_total] f16 (k_total = n_in, or kSplitParts n_in for split
-// f32 rows, whose weight column is k' mod n_in). Element (t, r) is stored at
+// and x' [n_tokens][parts n_in] f16 (one part, or the kSplitParts parts of split
+// f32 rows, whose products with the same weights add up). Element (t, r) is stored at
 // out + t*out_rs + (r/64)*out_hs + r%64. Groups share x and differ in W, bias
 // and out (all layers' cross K and V in one launch).
 constexpr int kLinearK = 64;          // n_in must be a multiple of this
@@ -205,14 +205,25 @@ struct LinearArgs {
   const _Float16* x;
   int64_t x_rs;
   const float* row_scale;  // nullable: 1
-  int n_tokens, n_in, n_out, k_total, n_groups;
+  int n_tokens, n_in, n_out, parts, n_groups;
   int64_t out_rs, out_hs;
   int act;  // Act, applied after the bias
+  // Scratch for tiles whose k is split over workgroups (null: no split):
+  // partial sums and merge counters (zero between launches), with their sizes.
+  float* part;
+  size_t part_floats;
+  unsigned* counters;
+  size_t counter_words;
   const _Float16* w[kMaxLinearGroups];
   const float* bias[kMaxLinearGroups];  // nullable entries
   void* out[kMaxLinearGroups];
 };
 hipError_t launch_linear_f16w(const LinearArgs& a, DType out_dt, hipStream_t s);
+// Whether the launch splits k when it is given scratch, and the scratch that
+// serves every such launch.
+bool linear_needs_split(const LinearArgs& a);
+size_t linear_split_floats();
+size_t linear_split_words();
 // Decode-sized batches (n_tokens <= kGemvMaxRows) of the same product on the
 // f16 weight stream; x is f32 or f16 with row stride x_rs, no split needed.
 constexpr int kGemvMaxRows = 8;
