@@ -304,3 +304,45 @@ def test_f16_only_entry_points_refuse_f32_arenas(wrs, ctx, W):
     with pytest.raises(RuntimeError, match="unsupported"):
         arena.capture_cross_heads(0, q, [(0, 1)], 1, 0, cap, lse=lse)
     arena.close()
+
+
+@pytest.mark.parametrize("rows", [1, 9])
+@pytest.mark.parametrize("keys", [1, 15, 17, 128, 129, 256, 257, 512, 513, 577, 1500, 4100])
+def test_exact_decode_key_counts(wrs, ctx, keys, rows):
+    """Both sides of every key count the exact decode treats differently (one
+    workgroup per row up to 512 keys, 64-key chunks beyond), rows past one row
+    block, planes with unused rows: against float64, and bit for bit the
+    host-slice call on the same values, whose rows start on any dword."""
+    note(f"exact decode keys={keys} rows={rows}")
+    H = 3
+    dm = H * 64
+    rng = np.random.default_rng(keys * 10 + rows)
+    k, v = (rng.standard_normal((keys, dm)).astype(np.float32) for _ in range(2))
+    q = (2.0 * rng.standard_normal((rows, dm))).astype(np.float32)
+    arena = _arena(wrs, ctx, 1, 1, H, 16, keys + 3)
+    arena.set_cross(0, k, v)
+    out = torch.full((rows, dm), float("nan"), device="cuda")
+    for _ in range(2):  # the merge counters are re-armed
+        out.fill_(float("nan"))
+        arena.decode_cross(0, dev(q), out)
+    got = host(out)
+    qd, kd, vd = (a.astype(np.float64).reshape(-1, H, 64).transpose(1, 0, 2) for a in (q, k, v))
+    s = qd @ kd.transpose(0, 2, 1) / 8.0
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    ref = (np.where(p < 1e-7, 0.0, p) @ vd).transpose(1, 0, 2).reshape(rows, dm)
+    # f32 sums of 64 products and of `keys` weights, and weights at the 1e-7 line
+    assert np.abs(got - ref).max() <= 4e-6 + 5e-7
+    for r in range(min(rows, 2)):
+        one = np.zeros(dm, np.float32)
+        wrs.single_token_mha_d64(q[r].copy(), k.ravel(), v.ravel(), keys, H, dm, one, ctx=ctx)
+        assert np.array_equal(one, got[r])
+    wide = dm + 2  # head span inside wider rows that start on 8-byte boundaries only
+    kw, vw = (np.zeros((keys, wide), np.float32) for _ in range(2))
+    kw[:, :dm], vw[:, :dm] = k, v
+    one = np.zeros(wide, np.float32)
+    qw = np.zeros(wide, np.float32)
+    qw[:dm] = q[0]
+    wrs.single_token_mha_d64(qw, kw.ravel(), vw.ravel(), keys, H, wide, one, ctx=ctx)
+    assert np.array_equal(one[:dm], got[0])
+    arena.close()

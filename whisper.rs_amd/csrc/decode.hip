@@ -43,6 +43,8 @@
 //   group g sees keys [0, glen[g] + i * limit_step).
 #include "wrs_internal.hpp"
 
+#include <algorithm>
+
 namespace wrs {
 namespace {
 
@@ -491,6 +493,278 @@ __global__ __launch_bounds__(kThreads) void decode_exact_f32(ExactArgs a) {
   }
 }
 
+// The same arithmetic for d_head 64, coalesced: 16 lanes hold one key row, four
+// columns each (16-byte loads, or four dwords where the rows are not 16-byte
+// aligned), and add their products with DPP. Up to kOneKeys keys one workgroup
+// per (row, head) does the whole step with every K and V load in flight at once
+// (decode_exact_one); longer caches deal 64-key chunks over workgroups in two
+// launches, since the 1e-7 rule needs the row's whole sum before any value is
+// weighted: the chunk scores with their maximum and sum (decode_exact_scores),
+// then the weighted values, whose chunks meet in the workgroup that counts in
+// last and are added in chunk order (decode_exact_values). Rows of one group
+// share each chunk read, kExactRows at a time. Bound by memory latency: one
+// thread per key reading its row alone took 52 us a call on average (6 heads,
+// 61 and 1500 keys).
+constexpr int kOneKeys = 512;
+constexpr int kExactChunk = 64;
+constexpr int kExactRows = 8;
+
+// Four floats at p, of which only dword alignment is known when !kVec.
+template <bool kVec>
+__device__ inline f32x4 load4(const float* p) {
+  if constexpr (kVec) {
+    return *reinterpret_cast<const f32x4*>(p);
+  } else {
+    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+    return *reinterpret_cast<const f32x4u*>(p);
+  }
+}
+// Sum over the 16 lanes of a row (DPP), in every lane.
+__device__ inline float sum16(float x) {
+  x += dpp<0xB1>(x);
+  x += dpp<0x4E>(x);
+  x += dpp<0x141>(x);
+  return x + dpp<0x140>(x);
+}
+__device__ inline float dot4(const f32x4& a, const f32x4& b) {
+  return __builtin_fmaf(a[3], b[3], __builtin_fmaf(a[2], b[2], __builtin_fmaf(a[1], b[1], a[0] * b[0])));
+}
+// acc += w v where the reference does not skip the weight.
+__device__ inline void add_weighted(float w, const f32x4& v, f32x4& acc) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = w < 1e-7f ? acc[e] : __builtin_fmaf(w, v[e], acc[e]);
+}
+
+// kT tiles of 128 keys: key 128 t + 16 wave + 4 i + (lane / 16), i < 4.
+template <int kT, bool kVec>
+__global__ __launch_bounds__(512) void decode_exact_one(ExactArgs a) {
+  __shared__ float red[2][8];
+  __shared__ __attribute__((aligned(16))) float accs[8][64];
+  const int h = blockIdx.x, row = blockIdx.y;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int sub = lane >> 4, c = 4 * (lane & 15);
+  const int g = row / a.rows_per_group;
+  const int L = a.glen[g] + (row - g * a.rows_per_group) * a.limit_step;
+  const int64_t kv0 = a.goff[g] + h * a.kv_hs + c;
+  f32x4 kx[kT * 4], vx[kT * 4];
+  const f32x4 q = load4<kVec>(a.q + static_cast<int64_t>(row) * a.q_rs + h * 64 + c);
+#pragma unroll
+  for (int i = 0; i < kT * 4; ++i) {
+    const int j = 128 * (i >> 2) + 16 * wave + 4 * (i & 3) + sub;
+    kx[i] = load4<kVec>(a.k + kv0 + static_cast<int64_t>(min(j, L - 1)) * a.kv_rs);
+  }
+#pragma unroll
+  for (int i = 0; i < kT * 4; ++i) {
+    const int j = 128 * (i >> 2) + 16 * wave + 4 * (i & 3) + sub;
+    vx[i] = load4<kVec>(a.v + kv0 + static_cast<int64_t>(min(j, L - 1)) * a.kv_rs);
+  }
+  float s[kT * 4], mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kT * 4; ++i) {
+    const int j = 128 * (i >> 2) + 16 * wave + 4 * (i & 3) + sub;
+    s[i] = j < L ? sum16(dot4(q, kx[i])) * a.scale : -INFINITY;
+    mx = fmaxf(mx, s[i]);
+  }
+  mx = max_x16_x32(mx);
+  if (lane == 0) red[0][wave] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 8; ++w) mx = fmaxf(mx, red[0][w]);
+  float sum = 0.f;
+#pragma unroll
+  for (int i = 0; i < kT * 4; ++i) {
+    const int j = 128 * (i >> 2) + 16 * wave + 4 * (i & 3) + sub;
+    s[i] = j < L ? expf(s[i] - mx) : 0.f;
+    sum += s[i];
+  }
+  sum = sum_x16_x32(sum);
+  if (lane == 0) red[1][wave] = sum;
+  __syncthreads();
+  sum = red[1][0];
+#pragma unroll
+  for (int w = 1; w < 8; ++w) sum += red[1][w];
+  const float inv = 1.f / sum;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < kT * 4; ++i) {
+    const int j = 128 * (i >> 2) + 16 * wave + 4 * (i & 3) + sub;
+    if (j < L) add_weighted(s[i] * inv, vx[i], acc);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) acc[e] = sum_x16_x32(acc[e]);
+  if (sub == 0) *reinterpret_cast<f32x4*>(&accs[wave][c]) = acc;
+  __syncthreads();
+  if (tid < 64) {
+    float o = accs[0][tid];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) o += accs[w][tid];
+    a.o[static_cast<int64_t>(row) * a.o_rs + h * 64 + tid] = o;
+  }
+}
+
+// Rows, keys and scratch of one (chunk, head, row block) workgroup of the two
+// launches below. Chunks past the block's longest row have nothing to do.
+struct ExactBlock {
+  int g, row0, rows, chunks;  // group, first row, rows of the block, chunks it spans
+  __device__ explicit ExactBlock(const ExactArgs& a) {
+    const int per = (a.rows_per_group + kExactRows - 1) / kExactRows;
+    g = blockIdx.z / per;
+    const int r0 = (blockIdx.z - g * per) * kExactRows;
+    row0 = g * a.rows_per_group + r0;
+    rows = min(min(kExactRows, a.rows_per_group - r0), a.n_rows - row0);
+    chunks = rows > 0 ? (a.glen[g] + (r0 + rows - 1) * a.limit_step + kExactChunk - 1) / kExactChunk : 0;
+  }
+};
+__device__ inline int exact_len(const ExactArgs& a, const ExactBlock& b, int r) {
+  return a.glen[b.g] + (b.row0 + r - b.g * a.rows_per_group) * a.limit_step;
+}
+
+template <bool kVec>
+__global__ __launch_bounds__(256) void decode_exact_scores(ExactArgs a) {
+  __shared__ __attribute__((aligned(16))) float qs[kExactRows][64];
+  __shared__ float red[2][kExactRows][4];
+  const ExactBlock b(a);
+  const int chunk = blockIdx.x, h = blockIdx.y;
+  if (chunk >= b.chunks) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int sub = lane >> 4, c = 4 * (lane & 15);
+  const int last = exact_len(a, b, b.rows - 1) - 1;  // the longest row's last key
+  const int64_t kv0 = a.goff[b.g] + h * a.kv_hs + c;
+  f32x4 kx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = chunk * kExactChunk + 16 * wave + 4 * i + sub;
+    kx[i] = load4<kVec>(a.k + kv0 + static_cast<int64_t>(min(j, last)) * a.kv_rs);
+  }
+  for (int e = tid; e < b.rows * 64; e += 256)
+    qs[e >> 6][e & 63] = a.q[static_cast<int64_t>(b.row0 + (e >> 6)) * a.q_rs + h * 64 + (e & 63)];
+  __syncthreads();
+  for (int r = 0; r < b.rows; ++r) {
+    const int L = exact_len(a, b, r);
+    const f32x4 q = *reinterpret_cast<const f32x4*>(&qs[r][c]);
+    float* sc = a.scores + (static_cast<int64_t>(b.row0 + r) * a.n_heads + h) * a.scores_stride;
+    float s[4], mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = chunk * kExactChunk + 16 * wave + 4 * i + sub;
+      s[i] = j < L ? sum16(dot4(q, kx[i])) * a.scale : -INFINITY;
+      if (j < L && c == 0) sc[j] = s[i];
+      mx = fmaxf(mx, s[i]);
+    }
+    mx = max_x16_x32(mx);
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = chunk * kExactChunk + 16 * wave + 4 * i + sub;
+      if (j < L) sum += expf(s[i] - mx);
+    }
+    sum = sum_x16_x32(sum);
+    if (lane == 0) {
+      red[0][r][wave] = mx;
+      red[1][r][wave] = sum;
+    }
+  }
+  __syncthreads();
+  if (tid < b.rows) {
+    float M = red[0][tid][0], S = 0.f;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) M = fmaxf(M, red[0][tid][w]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+      S += red[0][tid][w] == -INFINITY ? 0.f : red[1][tid][w] * expf(red[0][tid][w] - M);
+    float* st = a.stats + 2 * ((static_cast<int64_t>(b.row0 + tid) * a.n_heads + h) * a.n_chunks + chunk);
+    st[0] = M;
+    st[1] = S;
+  }
+}
+
+template <bool kVec>
+__global__ __launch_bounds__(256) void decode_exact_values(ExactArgs a) {
+  __shared__ __attribute__((aligned(16))) float accs[4][kExactRows][64];
+  __shared__ float rowmax[kExactRows], rowinv[kExactRows];
+  __shared__ int merger;
+  const ExactBlock b(a);
+  const int chunk = blockIdx.x, h = blockIdx.y;
+  if (chunk >= b.chunks) return;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int sub = lane >> 4, c = 4 * (lane & 15);
+  const int last = exact_len(a, b, b.rows - 1) - 1;
+  const int64_t kv0 = a.goff[b.g] + h * a.kv_hs + c;
+  f32x4 vx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = chunk * kExactChunk + 16 * wave + 4 * i + sub;
+    vx[i] = load4<kVec>(a.v + kv0 + static_cast<int64_t>(min(j, last)) * a.kv_rs);
+  }
+  // Row r's maximum and sum over its chunks, by wave r mod 4.
+  for (int r = wave; r < b.rows; r += 4) {
+    const float* st = a.stats + 2 * (static_cast<int64_t>(b.row0 + r) * a.n_heads + h) * a.n_chunks;
+    const int n = (exact_len(a, b, r) + kExactChunk - 1) / kExactChunk;
+    float M = -INFINITY;
+    for (int i = lane; i < n; i += 64) M = fmaxf(M, st[2 * i]);
+    M = wave_max(M);
+    float S = 0.f;
+    for (int i = lane; i < n; i += 64)
+      S += st[2 * i] == -INFINITY ? 0.f : st[2 * i + 1] * expf(st[2 * i] - M);
+    S = wave_sum(S);
+    if (lane == 0) {
+      rowmax[r] = M;
+      rowinv[r] = 1.f / S;
+    }
+  }
+  __syncthreads();
+  for (int r = 0; r < b.rows; ++r) {
+    const int L = exact_len(a, b, r);
+    const float* sc = a.scores + (static_cast<int64_t>(b.row0 + r) * a.n_heads + h) * a.scores_stride;
+    const float M = rowmax[r], inv = rowinv[r];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = chunk * kExactChunk + 16 * wave + 4 * i + sub;
+      if (j < L) add_weighted(expf(sc[j] - M) * inv, vx[i], acc);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[e] = sum_x16_x32(acc[e]);
+    if (sub == 0) *reinterpret_cast<f32x4*>(&accs[wave][r][c]) = acc;
+  }
+  __syncthreads();
+  const int64_t pr = static_cast<int64_t>(a.n_heads) * a.n_chunks * 64;  // partials of a row
+  float* const part = a.part + (static_cast<int64_t>(b.row0) * a.n_heads + h) * a.n_chunks * 64;
+  for (int e = tid; e < b.rows * 64; e += 256) {
+    const int r = e >> 6, d = e & 63;
+    const float o = accs[0][r][d] + accs[1][r][d] + accs[2][r][d] + accs[3][r][d];
+    if (b.chunks == 1)
+      a.o[static_cast<int64_t>(b.row0 + r) * a.o_rs + h * 64 + d] = o;
+    else
+      st_agent(part + r * pr + chunk * 64 + d, o);
+  }
+  if (b.chunks == 1) return;
+  // Every wave's stores are performed before the chunk counts in (as K2's merge).
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  unsigned* const counter =
+      a.counters + (static_cast<int64_t>(blockIdx.z) * a.n_heads + h) * kCounterStride;
+  if (tid == 0)
+    merger = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+             static_cast<unsigned>(b.chunks - 1);
+  __syncthreads();
+  if (!merger) return;
+  for (int e = tid; e < b.rows * 64; e += 256) {
+    const int r = e >> 6, d = e & 63;
+    float o = 0.f;
+    for (int s0 = 0; s0 < b.chunks; s0 += kMaxSplitsMerge) {
+      float x[kMaxSplitsMerge];
+#pragma unroll
+      for (int i = 0; i < kMaxSplitsMerge; ++i)
+        x[i] = s0 + i < b.chunks ? ld_agent(part + r * pr + (s0 + i) * 64 + d) : 0.f;
+#pragma unroll
+      for (int i = 0; i < kMaxSplitsMerge; ++i) o += x[i];
+    }
+    a.o[static_cast<int64_t>(b.row0 + r) * a.o_rs + h * 64 + d] = o;
+  }
+  if (tid == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // Streaming read with the decode grid's shape: 512 threads x 64 bytes per
 // workgroup, every load issued before any is used; one float per workgroup
 // keeps the loads live.
@@ -637,12 +911,84 @@ hipError_t launch_decode_f16(const DecodeArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+namespace {
+int exact_max_keys(const ExactArgs& a) {
+  int keys = 1;
+  for (int g = 0; g < a.n_groups; ++g)
+    keys = std::max(keys, a.glen[g] + (a.rows_per_group - 1) * a.limit_step);
+  return keys;
+}
+int exact_blocks(int n_groups, int rows_per_group) {
+  return n_groups * ((rows_per_group + kExactRows - 1) / kExactRows);
+}
+}  // namespace
+
+// Scratch of a launch: score rows; for d_head 64 past kOneKeys keys also chunk
+// statistics and partials, and a counter for each block of rows and head.
+ExactScratch decode_exact_scratch(int n_rows, int n_heads, int d_head, int max_keys, int n_groups,
+                                  int rows_per_group) {
+  ExactScratch x{};
+  const size_t rh = static_cast<size_t>(n_rows) * n_heads;
+  if (d_head != 64 || max_keys > kOneKeys) x.scores = rh * std::max(max_keys, 1);
+  if (d_head == 64 && max_keys > kOneKeys) {
+    x.chunks = (max_keys + kExactChunk - 1) / kExactChunk;
+    x.stats = 2 * rh * x.chunks;
+    x.part = 64 * rh * x.chunks;
+    x.counter_words =
+        static_cast<size_t>(exact_blocks(n_groups, rows_per_group)) * n_heads * kCounterStride;
+  }
+  return x;
+}
+
 hipError_t launch_decode_exact_f32(const ExactArgs& a, hipStream_t s) {
   if (a.n_rows <= 0 || a.n_heads <= 0) return hipSuccess;
   if (a.rows_per_group <= 0 || a.n_groups <= 0 || a.n_groups > kMaxExactGroups ||
       static_cast<int64_t>(a.n_groups) * a.rows_per_group < a.n_rows || a.n_rows > 65535 ||
       a.d_head <= 0 || a.d_head > 128)
     return hipErrorInvalidValue;
+  if (a.d_head == 64) {
+    auto al = [](const float* p, int64_t rs) {
+      return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && rs % 4 == 0;
+    };
+    bool vec = al(a.q, a.q_rs) && al(a.k, a.kv_rs) && al(a.v, a.kv_hs);
+    for (int g = 0; g < a.n_groups; ++g) vec = vec && a.goff[g] % 4 == 0;
+    const int keys = exact_max_keys(a);
+    // One workgroup takes in a row's keys at ~50 GB/s; past 512 keys (256 KB of
+    // K and V) the second launch and the merge cost less than that.
+    if (keys <= kOneKeys) {
+      const dim3 grid(a.n_heads, a.n_rows), block(512);
+#define WRS_ONE(T)                                                                            \
+  if (vec)                                                                                    \
+    hipLaunchKernelGGL((decode_exact_one<T, true>), grid, block, 0, s, a);                    \
+  else                                                                                        \
+    hipLaunchKernelGGL((decode_exact_one<T, false>), grid, block, 0, s, a);
+      if (keys <= 128) {
+        WRS_ONE(1)
+      } else if (keys <= 256) {
+        WRS_ONE(2)
+      } else {
+        WRS_ONE(4)
+      }
+#undef WRS_ONE
+      return hipGetLastError();
+    }
+    if (!a.stats || !a.part || !a.counters) return hipErrorInvalidValue;
+    const int blocks = exact_blocks(a.n_groups, a.rows_per_group);
+    if (blocks > 65535) return hipErrorInvalidConfiguration;
+    const dim3 grid(a.n_chunks, a.n_heads, blocks), block(256);
+    if (vec) {
+      hipLaunchKernelGGL(decode_exact_scores<true>, grid, block, 0, s, a);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(decode_exact_values<true>, grid, block, 0, s, a);
+    } else {
+      hipLaunchKernelGGL(decode_exact_scores<false>, grid, block, 0, s, a);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      hipLaunchKernelGGL(decode_exact_values<false>, grid, block, 0, s, a);
+    }
+    return hipGetLastError();
+  }
   const dim3 grid(a.n_heads, a.n_rows), block(kThreads);
   hipLaunchKernelGGL(decode_exact_f32, grid, block, 0, s, a);
   return hipGetLastError();

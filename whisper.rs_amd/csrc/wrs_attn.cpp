@@ -188,8 +188,14 @@ int run_exact(wrs_attn_ctx* c, const float* q, size_t q_floats, const float* k, 
   Stage st;
   const size_t iq = st.add(q_floats), ik = st.add(kv_floats), iv = st.add(kv_floats);
   const size_t io = st.add(out_floats);
-  const size_t is = st.add(static_cast<size_t>(n_rows) * n_heads * std::max<size_t>(max_keys, 1));
+  if (!fits_int(max_keys)) return fail(c, WRS_EINVAL, "dimension exceeds 2^31");
+  const wrs::ExactScratch x = wrs::decode_exact_scratch(n_rows, n_heads, d_head,
+                                                        static_cast<int>(max_keys), 1, n_rows);
+  const size_t is = st.add(x.scores), it = st.add(x.stats), ip = st.add(x.part);
   int rc = grow(c, &c->stage, &c->stage_bytes, st.total, false);
+  if (rc) return rc;
+  rc = grow(c, reinterpret_cast<void**>(&c->counters), &c->counter_bytes,
+            x.counter_words * sizeof(unsigned), true);
   if (rc) return rc;
   float *dq = stage_ptr(c, st, iq), *dk = stage_ptr(c, st, ik), *dv = stage_ptr(c, st, iv);
   float *dout = stage_ptr(c, st, io), *ds = stage_ptr(c, st, is);
@@ -218,6 +224,10 @@ int run_exact(wrs_attn_ctx* c, const float* q, size_t q_floats, const float* k, 
   a.scale = 1.0f / std::sqrt(static_cast<float>(d_head));
   a.scores = ds;
   a.scores_stride = static_cast<int64_t>(std::max<size_t>(max_keys, 1));
+  a.n_chunks = x.chunks;
+  a.stats = stage_ptr(c, st, it);
+  a.part = stage_ptr(c, st, ip);
+  a.counters = c->counters;
   WRS_HIP(c, wrs::launch_decode_exact_f32(a, c->stream));
   WRS_HIP(c, hipMemcpyAsync(out, dout, out_floats * 4, hipMemcpyDeviceToHost, c->stream));
   WRS_HIP(c, hipStreamSynchronize(c->stream));
@@ -814,10 +824,14 @@ int exact_arena(wrs_attn_ctx* c, wrs_kv* kv, const float* q, float* out, void* k
   int max_len = 1;
   for (size_t g = 0; g < groups; ++g)
     max_len = std::max(max_len, glen[g] + (rows_per_group - 1) * limit_step);
-  const size_t bytes =
-      static_cast<size_t>(n_rows) * kv->n_heads * static_cast<size_t>(max_len) * sizeof(float);
-  int rc = grow(c, reinterpret_cast<void**>(&c->exact_scores), &c->exact_scores_bytes, bytes,
-                false);
+  const wrs::ExactScratch x =
+      wrs::decode_exact_scratch(n_rows, static_cast<int>(kv->n_heads), 64, max_len,
+                                static_cast<int>(groups), rows_per_group);
+  int rc = grow(c, reinterpret_cast<void**>(&c->exact_scores), &c->exact_scores_bytes,
+                (x.scores + x.stats + x.part) * sizeof(float), false);
+  if (rc) return rc;
+  rc = grow(c, reinterpret_cast<void**>(&c->counters), &c->counter_bytes,
+            x.counter_words * sizeof(unsigned), true);
   if (rc) return rc;
   wrs::ExactArgs a{};
   a.q = q;
@@ -837,6 +851,10 @@ int exact_arena(wrs_attn_ctx* c, wrs_kv* kv, const float* q, float* out, void* k
   a.scale = 0.125f;  // 1/sqrt(64) (attention.rs:255, decoder.rs:857)
   a.scores = c->exact_scores;
   a.scores_stride = max_len;
+  a.n_chunks = x.chunks;
+  a.stats = c->exact_scores + x.scores;
+  a.part = a.stats + x.stats;
+  a.counters = c->counters;
   for (size_t g = 0; g < groups; ++g) {
     a.goff[g] = goff[g];
     a.glen[g] = glen[g];

@@ -115,11 +115,22 @@ struct ExactArgs {
   int n_rows, n_heads, d_head;
   int rows_per_group, n_groups, limit_step;
   float scale;
-  float* scores;  // scratch [n_rows][n_heads][scores_stride]
+  // Scratch, as decode_exact_scratch sizes it.
+  float* scores;  // [n_rows][n_heads][scores_stride]
   int64_t scores_stride;
+  int n_chunks;
+  float* stats;        // [n_rows][n_heads][n_chunks] (max, sum)
+  float* part;         // [n_rows][n_heads][n_chunks][64]
+  unsigned* counters;  // zero between launches
   int64_t goff[kMaxExactGroups];
   int glen[kMaxExactGroups];
 };
+struct ExactScratch {
+  size_t scores, stats, part, counter_words;  // floats, floats, floats, words
+  int chunks;
+};
+ExactScratch decode_exact_scratch(int n_rows, int n_heads, int d_head, int max_keys, int n_groups,
+                                  int rows_per_group);
 hipError_t launch_decode_exact_f32(const ExactArgs& a, hipStream_t s);
 
 // Split-K decode over an f16 KV cache: one query row per (group, row),
