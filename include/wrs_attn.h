@@ -68,7 +68,7 @@ int wrs_attn_set_stream(wrs_attn_ctx *ctx, void *hip_stream);
 void *wrs_attn_get_stream(wrs_attn_ctx *ctx);
 int wrs_attn_synchronize(wrs_attn_ctx *ctx);
 /* Work decomposition of this context's prefill calls (wrs_attn_prefill, the
- * host-slice drop-ins and the prompt-row entry points); results do not depend
+ * host-slice drop-ins and the prompt rows of f32 arenas); results do not depend
  * on it beyond floating-point summation order. No reference counterpart: the
  * reference's tiling is fixed (Q_TILE = KV_TILE = 128, attention.rs:13,26).
  * prefill_queries: queries per workgroup of the f16/bf16 kernel: 256 or 128
@@ -270,9 +270,11 @@ int wrs_attn_decode_cross_noalloc(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, c
                                   size_t n_beams, float *out);
 /* Multi-token rows (prompt prefill): decoder.rs:857-891 self-attention with
  * offset t_past = slot_len(slot) over the slot's f16 cache (rows appended),
- * and attention.rs:107-243 cross-attention with t_q = n_tokens (the rows run
- * on the split-K decode kernel in groups of 8 that share each read of the
- * plane, with its numerics: f16 keys and values, q split into two f16 parts). */
+ * and attention.rs:107-243 cross-attention with t_q = n_tokens. f16 keys and
+ * values on the f16 matrix pipe, with q and the weights split into f16 parts:
+ * two for cross-attention (up to 24 rows on the split-K decode kernel in groups
+ * of 8 that share each read of the plane), three, which hold all 24 bits, for
+ * the cached self-attention. */
 int wrs_attn_prefill_self(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, size_t slot,
                           const float *q, size_t n_tokens, float *out);
 int wrs_attn_prefill_cross(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, const float *q,

@@ -1,0 +1,111 @@
+"""Prompt rows over the f16 arena (K10): cached self-attention with a causal
+offset (decoder.rs:857-891) and cross-attention of more rows than a decode
+group (attention.rs:107-243), at the edges of its row blocks, and key steps, against float64 over the f16 cache values."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_util import dev, host, note
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx(wrs):
+    c = wrs.Context(0)
+    c.use_torch_stream()
+    return c
+
+
+def _f16(a):
+    return a.astype(np.float16).astype(np.float32)
+
+
+def _attend(q, k, v, heads, pos0=None):
+    """Rows and row statistics (max, sum of 2^(s - max)) in float64."""
+    qd, kd, vd = (a.astype(np.float64).reshape(a.shape[0], heads, 64).transpose(1, 0, 2)
+                  for a in (q, k, v))
+    s = (qd @ kd.transpose(0, 2, 1)) * (0.125 * np.log2(np.e))
+    if pos0 is not None:
+        s = np.where(np.arange(k.shape[0])[None, :] > pos0 + np.arange(q.shape[0])[:, None],
+                     -np.inf, s)
+    m = s.max(-1, keepdims=True)
+    p = np.exp2(s - m)
+    out = (p @ vd) / p.sum(-1, keepdims=True)
+    return out.transpose(1, 0, 2).reshape(q.shape), m[..., 0], p.sum(-1)
+
+
+def _bound(q, k, v, heads):
+    """Largest error of each output row: its scores err by at most
+    (64 2^-24 + 2^-21) max_j |q||k_j| / 8 (a sum of 64 products in f32, operands
+    and scaling to 2^-22), so every normalized weight by twice that relative to
+    itself, and the weighted sum adds 2^-20 max |v| (exp2, split weights, f32 sums)."""
+    qa, ka, va = (np.abs(a.astype(np.float64)).reshape(a.shape[0], heads, 64).transpose(1, 0, 2)
+                  for a in (q, k, v))
+    ds = (64 * 2.0 ** -24 + 2.0 ** -21) * (qa @ ka.transpose(0, 2, 1)).max(-1) / 8.0
+    b = (2.0 * np.expm1(ds) + 2.0 ** -20) * va.max((1, 2))[:, None]  # [head][row]
+    return np.repeat(b.T[:, :, None], 64, axis=2).reshape(q.shape)
+
+
+@pytest.mark.parametrize("heads,rows,keys", [
+    (1, 9, 1), (6, 9, 1500), (3, 17, 200), (6, 24, 700), (1, 25, 1), (2, 31, 31), (2, 32, 33), (3, 33, 64), (20, 37, 1500), (20, 128, 1500),
+    (6, 65, 511), (6, 64, 513), (1, 25, 4097), (20, 448, 300), (2, 26, 767), (2, 26, 768)])
+def test_cross_rows(wrs, ctx, heads, rows, keys):
+    note(f"cross rows heads={heads} rows={rows} keys={keys}")
+    rng = np.random.default_rng(heads * 1000 + rows + keys)
+    d = heads * 64
+    k, v = (_f16(rng.standard_normal((keys, d))) for _ in range(2))
+    q = rng.standard_normal((rows, d)).astype(np.float32)
+    q[0] *= 30.0   # a peaked row
+    q[1] *= 1e-30  # a flat one
+    q[2] = 0.0
+    arena = wrs.KvArena(1, 1, heads, 16, keys + 5, ctx=ctx)
+    arena.set_cross(0, k, v)
+    out = torch.full((rows + 1, d), float("nan"), device="cuda")
+    lse = torch.full((heads * rows * 2 + 2,), float("nan"), device="cuda")
+    ref, m, l = _attend(q, k, v, heads)
+    tol = _bound(q, k, v, heads)
+    arena.prefill_cross(0, dev(q), out[:rows], lse=lse)
+    got = host(out)
+    assert (np.abs(got[:rows] - ref) <= tol).all()
+    assert np.isnan(got[rows]).all()
+    st = host(lse)
+    assert np.isnan(st[-2:]).all()
+    st = st[:-2].reshape(heads, rows, 2).astype(np.float64)
+    lg, lr = st[..., 0] + np.log2(st[..., 1]), m + np.log2(l)
+    assert np.abs(lg - lr).max() <= 1e-5 * max(1.0, np.abs(lr).max())
+    plain = torch.empty((rows, d), device="cuda")
+    arena.prefill_cross(0, dev(q), plain)
+    assert torch.equal(plain, out[:rows])
+    arena.close()
+
+
+@pytest.mark.parametrize("heads,rows,past", [
+    (1, 2, 0), (2, 31, 0), (2, 32, 1), (3, 33, 30), (20, 37, 0), (20, 224, 224), (6, 2, 445),
+    (1, 100, 1900), (4, 448, 0)])
+def test_cached_self_rows(wrs, ctx, heads, rows, past):
+    note(f"self rows heads={heads} rows={rows} past={past}")
+    rng = np.random.default_rng(heads * 1000 + rows + past)
+    d = heads * 64
+    n = past + rows
+    k, v = (_f16(rng.standard_normal((n, d))) for _ in range(2))
+    buf = torch.zeros(rows * d + 1, device="cuda")
+    q = buf[1:].view(rows, d)  # rows that start on any dword
+    qh = rng.standard_normal((rows, d)).astype(np.float32)
+    qh[-1] *= 30.0
+    q.copy_(dev(qh))
+    arena = wrs.KvArena(1, 2, heads, n + 3, 0, ctx=ctx)
+    if past:
+        arena.append(0, 1, k[:past], v[:past])
+        arena.advance(1, past)
+    arena.append(0, 1, np.ascontiguousarray(k[past:]), np.ascontiguousarray(v[past:]))
+    out = torch.full((rows + 1, d), float("nan"), device="cuda")
+    ref, _, _ = _attend(qh, k, v, heads, past)
+    tol = _bound(qh, k, v, heads)
+    arena.prefill_self(0, 1, q, out[:rows])
+    got = host(out)
+    assert (np.abs(got[:rows] - ref) <= tol).all()
+    assert np.isnan(got[rows]).all()
+    arena.close()

@@ -147,6 +147,7 @@ struct DecodeArgs {
   int64_t goff[kMaxDecodeGroups];  // per-group plane offset (elements)
   int len[kMaxDecodeGroups];       // keys visible to group g
   int n_groups, rows_per_group, n_heads;
+  int n_rows;    // query rows: the last group may hold fewer than rows_per_group
   int chunk;     // keys per workgroup (kDecodeChunk or kDecodeChunkLong)
   int n_splits;  // workgroups per (group, head) = ceil(max len / chunk)
   float scale_log2;  // (1/8) * log2(e)
@@ -162,6 +163,25 @@ constexpr int kDecodeChunkLong = 256;  // one workgroup per (group, head) up to 
 hipError_t launch_decode_f16(const DecodeArgs& a, hipStream_t s);
 size_t decode_part_floats(int n_groups, int n_heads, int n_splits, int rows);
 size_t decode_counter_words(int n_groups, int n_heads);
+
+// Prompt rows over the f16 cache: query row i, head h at q + i*q_rs + h*64 (any
+// dword) against n_keys keys of plane k + h*kv_hs (key j at +j*64). With causal,
+// row i sees keys j < pos0 + i + 1 (the cached self-attention: three-part
+// operands); without, every key (two parts, like the split-K decode).
+struct RowsArgs {
+  const float* q;
+  float* o;  // same indexing with o_rs
+  const _Float16* k;
+  const _Float16* v;
+  int64_t q_rs, o_rs, kv_hs;
+  int n_rows, n_heads, n_keys;
+  int causal, pos0;
+  float scale_log2;  // (1/8) * log2(e)
+  float* lse;        // optional: (max, sum of exp2(s - max)) at lse[2 * (h * n_rows + row)]
+};
+hipError_t launch_attend_rows(const RowsArgs& a, hipStream_t s);
+// One past the keys a launch takes (32-bit plane offsets).
+constexpr size_t kRowsMaxKeys = (size_t{1} << 24) - 4095;
 
 // Measurement: a streaming read of `bytes` (multiple of 16, 16-byte aligned)
 // with the split-K decode's grid shape (512 threads x 64 bytes per
