@@ -496,3 +496,37 @@ def test_linear_split_k_under_capture(wrs):
                 assert bool(((out - eager).double().abs() <= bound).all())
             wrs.linear(x, w, None, eager, ctx=c)
     c.close()
+
+
+@pytest.mark.parametrize("n_tokens", [3, 4, 7, 8])
+@pytest.mark.parametrize("n_in,n_out", [(1344, 5), (1536, 384), (2112, 130), (5120, 1280),
+                                        (5120, 4100)])
+def test_decode_rows_long(wrs, ctx, n_tokens, n_in, n_out):
+    """Three to eight f32 rows past the register width: rows and column batches
+    of very different magnitude, k steps that do not divide over the waves, one
+    and several tiles per workgroup; and with a fused LayerNorm bit for bit the
+    separate calls."""
+    note(f"decode rows long T={n_tokens} K={n_in} N={n_out}")
+    rng = np.random.default_rng(n_in + n_out + n_tokens)
+    x = rng.standard_normal((n_tokens, n_in)).astype(np.float32)
+    x *= 10.0 ** rng.uniform(-6, 6, (n_tokens, 1)).astype(np.float32)
+    x[:, :256] *= np.float32(1e-4)
+    x[-1, 512:] = 0.0
+    w = _weights(n_out, n_in, n_in + 7)
+    b = rng.standard_normal(n_out).astype(np.float32)
+    buf = torch.zeros((n_tokens, n_in + 4), device="cuda")
+    buf[:, :n_in] = dev(x)
+    wd, bd = torch.from_numpy(w).cuda(), dev(b)
+    out = torch.full((n_tokens, n_out), float("nan"), device="cuda")
+    wrs.linear(buf[:, :n_in], wd, bd, out, ctx=ctx)
+    bound = _gamma_bound(x, w) + 2.0 ** -23 * np.abs(b)
+    assert (np.abs(host(out) - _exact(x, w, b)) <= bound).all()
+    gamma = dev((1.0 + 0.1 * rng.standard_normal(n_in)).astype(np.float32))
+    beta = dev((0.1 * rng.standard_normal(n_in)).astype(np.float32))
+    xd = dev(x)
+    wrs.linear_fused(xd, [wd], [bd], [out], ln=(gamma, beta, 1e-5), act="gelu", ctx=ctx)
+    normed, ref = torch.empty_like(xd), torch.empty_like(out)
+    wrs.layer_norm(xd, gamma, beta, 1e-5, normed, ctx=ctx)
+    wrs.linear(normed, wd, bd, ref, ctx=ctx)
+    wrs.gelu_inplace(ref, ctx=ctx)
+    assert torch.equal(out, ref)

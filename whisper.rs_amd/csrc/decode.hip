@@ -97,35 +97,6 @@ __device__ inline void store_lse(const DecodeArgs& a, int row, int h, float m, f
 }
 __device__ inline int clamp_exp(int e) { return e < -126 ? -126 : (e > 127 ? 127 : e); }
 
-// x op x[lane ^ 32] and x op x[lane ^ 16] with the gfx950 lane-swap VALU
-// instructions (no LDS round trip). Issued as inline asm on two distinct
-// registers: the swap writes both operands.
-__device__ inline void swap32(float& a, float& b) {
-  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-__device__ inline void swap16(float& a, float& b) {
-  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-}
-__device__ inline float max_x16_x32(float x) {
-  float a = x, b = x;
-  swap16(a, b);  // a, b: x of this row and of the row 16 lanes away
-  x = fmaxf(a, b);
-  a = x;
-  b = x;
-  swap32(a, b);
-  return fmaxf(a, b);
-}
-__device__ inline float sum_x16_x32(float x) {
-  float a = x, b = x;
-  swap16(a, b);
-  x = a + b;
-  a = x;
-  b = x;
-  swap32(a, b);
-  return a + b;
-}
-
-
 // kMWaves waves of kTiles 16-key tiles each: 8 waves of one tile (128 keys,
 // kDecodeChunk) in general, 8 waves of two (kDecodeChunkLong = 256 keys) when
 // that covers the whole sequence, which then needs no split-K merge. Tile t of

@@ -798,7 +798,7 @@ __global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_mfma(GemvArgs a, int 
   // both.
   int tile = blockIdx.x;
   u32x4 wv[kGmKB];
-  const bool reg_row = kSplit && n_in <= 256 * kLnCache;
+  constexpr bool reg_row = kSplit;  // n_in <= 256 * kLnCache: longer f32 rows run on K7l
   f32x4 xv[kLnCache], gg[kLnCache], bb[kLnCache];
   const float* xr32 = static_cast<const float*>(a.x) + static_cast<int64_t>(wave) * a.x_rs;
   if (reg_row && wave < nt)
@@ -837,73 +837,13 @@ __global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_mfma(GemvArgs a, int 
     }
     if (lane == 0) dn[wave] = gm_pow2(gm_clamp_exp(-sh));
   }
-  if constexpr (kSplit) {
-    if (kLn && !reg_row && wave < nt) {
-      // Longer rows with a fused LayerNorm: statistics, then two passes.
-      const float* xr = xr32;
-      float mean, inv_std;
-      ln_row_stats(xr, n_in, a.ln_eps, mean, inv_std);
-      float amax = 0.f;
-      for (int k = 4 * lane; k < n_in; k += 256) {
-        const f32x4 y = ln_apply(xr, a.ln_g, a.ln_b, k, mean, inv_std);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fabsf(y[j]));
-      }
-      amax = wave_max64(amax);
-      const int e_max = static_cast<int>((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFF);
-      const int sh = e_max == 0 ? 0 : gm_clamp_exp(141 - e_max);
-      const float up = gm_pow2(sh);
-      for (int k = 4 * lane; k < n_in; k += 256) {
-        const f32x4 y = ln_apply(xr, a.ln_g, a.ln_b, k, mean, inv_std);
-        f16x4v hv, lv;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float v = y[j] * up;
-          const _Float16 h = static_cast<_Float16>(v);
-          hv[j] = h;
-          lv[j] = static_cast<_Float16>(v - static_cast<float>(h));
-        }
-        *reinterpret_cast<f16x4v*>(&gxs[wave * pitch + k]) = hv;
-        *reinterpret_cast<f16x4v*>(&gxs[(nt + wave) * pitch + k]) = lv;
-      }
-      if (lane == 0) dn[wave] = gm_pow2(gm_clamp_exp(-sh));
+  if constexpr (!kSplit) {
+    if (wave < nt) {
+      const XT* xr = static_cast<const XT*>(a.x) + static_cast<int64_t>(wave) * a.x_rs;
+      for (int k = 8 * lane; k < n_in; k += 512)
+        *reinterpret_cast<f16x8*>(&gxs[wave * pitch + k]) = *reinterpret_cast<const f16x8*>(xr + k);
+      if (lane == 0) dn[wave] = 1.f;
     }
-  }
-  if (wave < nt && !reg_row && !kLn) {
-    const XT* xr = static_cast<const XT*>(a.x) + static_cast<int64_t>(wave) * a.x_rs;
-    int sh = 0;
-    if constexpr (kSplit) {
-      float amax = 0.f;
-      for (int k = 8 * lane; k < n_in; k += 512) {
-        const f32x4 lo = *reinterpret_cast<const f32x4*>(xr + k);
-        const f32x4 hi = *reinterpret_cast<const f32x4*>(xr + k + 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fmaxf(fabsf(lo[j]), fabsf(hi[j])));
-      }
-      amax = wave_max64(amax);
-      const int e_max = static_cast<int>((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFF);
-      sh = e_max == 0 ? 0 : gm_clamp_exp(141 - e_max);
-    }
-    const float up = gm_pow2(sh);
-    for (int k = 8 * lane; k < n_in; k += 512) {
-      f16x8 hv, lv;
-      if constexpr (kSplit) {
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(xr + k);
-        const f32x4 x1 = *reinterpret_cast<const f32x4*>(xr + k + 4);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float v = (j < 4 ? x0[j] : x1[j - 4]) * up;
-          const _Float16 h = static_cast<_Float16>(v);
-          hv[j] = h;
-          lv[j] = static_cast<_Float16>(v - static_cast<float>(h));
-        }
-        *reinterpret_cast<f16x8*>(&gxs[(nt + wave) * pitch + k]) = lv;
-      } else {
-        hv = *reinterpret_cast<const f16x8*>(xr + k);
-      }
-      *reinterpret_cast<f16x8*>(&gxs[wave * pitch + k]) = hv;
-    }
-    if (lane == 0) dn[wave] = gm_pow2(gm_clamp_exp(-sh));
   }
   __syncthreads();
 
@@ -952,6 +892,192 @@ __global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_mfma(GemvArgs a, int 
         for (int w8 = 0; w8 < kGmWaves; ++w8)
           sacc += red[par][w8][r * kGmRedPitch + b] + red[par][w8][r * kGmRedPitch + b + 8];
         float v = sacc * dn[b];
+        if (bias) v += bias_v;
+        if (a.act == kActGelu) v = gelu_tanh(v);
+        out[static_cast<int64_t>(b) * a.out_rs + static_cast<int64_t>(row >> 6) * a.out_hs +
+            (row & 63)] = static_cast<OutT>(v);
+      }
+    }
+    par ^= 1;
+  }
+}
+
+// K7l (gemv_f16w_long): K7m for f32 rows longer than its registers hold (the
+//   second MLP projection). A wave needs x only at its own k-steps, so each
+//   stages batches of kGlKB k-steps of every row for itself: half a wave per row
+//   loads 128 columns, takes their largest element (a scale per row and batch),
+//   and writes the high and low parts to the wave's own LDS rows; the batch's
+//   MFMAs start from zero and are scaled back (exact) as they are added up. No
+//   barrier stands before the products and the next batch of W and x is in
+//   flight meanwhile. Rows staged whole by one wave each, in two passes, had cost
+//   most of the launch, and eight rows of 5120 did not fit the LDS: 5 rows,
+//   5120 -> 1280 12.2 -> 11.2 us, 8 rows 28.4 -> 12.4 us (FMA kernel before), 5
+//   rows 3072 -> 768 8.6 -> 7.4 us.
+//   A fused LayerNorm takes one barrier: wave b forms row b's mean and deviation.
+constexpr int kGlKB = 4;                       // k-steps per wave per batch: 128 columns
+constexpr int kGlPitch = 32 * kGlKB + 8;       // f16 elements of a staged row
+
+template <typename OutT, bool kLn>
+__global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_long(GemvArgs a, int T) {
+  __shared__ __attribute__((aligned(16))) _Float16 xs[kGmWaves][16][kGlPitch];  // hi rows, lo rows
+  __shared__ __attribute__((aligned(16))) float red[2][kGmWaves][kGmRedFloats];
+  __shared__ float dn[kGmWaves][8], row_mean[8], row_inv[8];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int col = lane & 15, kg = lane >> 4;
+  const int grp = blockIdx.y;
+  const int nt = a.n_tokens, n_in = a.n_in, n_out = a.n_out;
+  const _Float16* w = a.w[grp];
+  const float* x = static_cast<const float*>(a.x);
+  const int ks_total = n_in >> 5;
+  const int s_per = (ks_total + kGmWaves - 1) / kGmWaves;
+  const int ks0 = min(wave * s_per, ks_total), ks1 = min(ks0 + s_per, ks_total);
+  const int n_batches = (s_per + kGlKB - 1) / kGlKB;
+  const int n_tiles = (n_out + T - 1) / T;
+  const bool arow = col < T;
+
+  auto load_w = [&](int tile, int bj, u32x4 (&wv)[kGlKB]) {
+    const int r = min(tile * T + (arow ? col : 0), n_out - 1);
+    const _Float16* wr = w + static_cast<int64_t>(r) * n_in + 8 * kg;
+#pragma unroll
+    for (int u = 0; u < kGlKB; ++u)
+      wv[u] = *reinterpret_cast<const u32x4*>(wr + 32 * min(ks0 + bj * kGlKB + u, ks_total - 1));
+  };
+  // Row 2 i + (lane / 32), columns 4 (lane % 32).. of the batch (the row's last
+  // columns again past the matrix).
+  const int xrow = lane >> 5, xcol = 4 * (lane & 31);
+  const int pairs = (nt + 1) >> 1;
+  auto load_x = [&](int bj, f32x4 (&xv)[4]) {
+    const int k = min(32 * (ks0 + bj * kGlKB) + xcol, n_in - 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < pairs)
+        xv[i] = *reinterpret_cast<const f32x4*>(
+            x + static_cast<int64_t>(min(2 * i + xrow, nt - 1)) * a.x_rs + k);
+  };
+
+  u32x4 wv[kGlKB];
+  f32x4 xv[4], gv, bv;
+  auto load_norm = [&](int bj) {
+    const int k = min(32 * (ks0 + bj * kGlKB) + xcol, n_in - 4);
+    gv = *reinterpret_cast<const f32x4*>(a.ln_g + k);
+    bv = *reinterpret_cast<const f32x4*>(a.ln_b + k);
+  };
+  int tile = blockIdx.x;
+  load_x(0, xv);
+  if constexpr (kLn) load_norm(0);
+  load_w(tile, 0, wv);
+  if constexpr (kLn) {
+    if (wave < nt) {
+      float m, iv;
+      ln_row_stats(x + static_cast<int64_t>(wave) * a.x_rs, n_in, a.ln_eps, m, iv);
+      if (lane == 0) {
+        row_mean[wave] = m;
+        row_inv[wave] = iv;
+      }
+    }
+    __syncthreads();
+  }
+  auto wave_sync = [] {
+    // LDS operations of one wave complete in order: only the compiler must keep it.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // The batch's rows into this wave's LDS rows.
+  auto stage = [&](int bj) __attribute__((always_inline)) {
+    const bool in = 32 * (ks0 + bj * kGlKB) + xcol < 32 * ks1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (i >= pairs) break;
+      const int row = 2 * i + xrow;
+      f32x4 v = xv[i];
+      if constexpr (kLn) {
+        const float mean = row_mean[min(row, nt - 1)], inv_std = row_inv[min(row, nt - 1)];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = fmaf((v[j] - mean) * inv_std, gv[j], bv[j]);
+      }
+      if (!in) v = f32x4{0.f, 0.f, 0.f, 0.f};
+      float amax = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+      amax = fmaxf(amax, dpp<0xB1>(amax));
+      amax = fmaxf(amax, dpp<0x4E>(amax));
+      amax = fmaxf(amax, dpp<0x141>(amax));
+      amax = fmaxf(amax, dpp<0x140>(amax));
+      float p = amax, q = amax;
+      swap16(p, q);  // the other 16 lanes of this half
+      amax = fmaxf(p, q);
+      const int e_max = static_cast<int>((__builtin_bit_cast(uint32_t, amax) >> 23) & 0xFF);
+      const int sh = e_max == 0 ? 0 : gm_clamp_exp(141 - e_max);
+      const float up = gm_pow2(sh);
+      f16x4v hv, lv;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float s = v[j] * up;
+        const _Float16 h = static_cast<_Float16>(s);
+        hv[j] = h;
+        lv[j] = static_cast<_Float16>(s - static_cast<float>(h));
+      }
+      if (row < nt) {
+        *reinterpret_cast<f16x4v*>(&xs[wave][row][xcol]) = hv;
+        *reinterpret_cast<f16x4v*>(&xs[wave][8 + row][xcol]) = lv;
+        if ((lane & 31) == 0) dn[wave][row] = gm_pow2(gm_clamp_exp(-sh));
+      }
+    }
+  };
+
+  const int beam = col & 7;
+  const bool bvalid = beam < nt;
+  const _Float16* const xb = &xs[wave][bvalid ? col : 0][8 * kg];
+  OutT* out = reinterpret_cast<OutT*>(a.out[grp]);
+  const float* bias = a.bias[grp];
+  const f16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+  const u32x4 zero4 = {0, 0, 0, 0};
+  int par = 0;
+  for (; tile < n_tiles; tile += gridDim.x) {
+    float bias_v = 0.f;
+    if (bias && tid < 128) bias_v = bias[min(tile * T + min(tid >> 3, T - 1), n_out - 1)];
+    const bool more = tile + static_cast<int>(gridDim.x) < n_tiles;
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int bj = 0; bj < n_batches; ++bj) {
+      u32x4 cur[kGlKB];
+#pragma unroll
+      for (int u = 0; u < kGlKB; ++u) cur[u] = arow ? wv[u] : zero4;
+      wave_sync();  // the last batch's operand reads are done
+      stage(bj);
+      const bool last = bj + 1 == n_batches;
+      if (!last || more) {
+        const int nb = last ? 0 : bj + 1;
+        load_x(nb, xv);
+        if constexpr (kLn) load_norm(nb);
+        load_w(last ? tile + gridDim.x : tile, nb, wv);
+      }
+      wave_sync();
+      const float down = bvalid ? dn[wave][beam] : 0.f;
+      f32x4 part = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < kGlKB; ++u) {
+        if (ks0 + bj * kGlKB + u < ks1) {  // wave-uniform
+          const f16x8 bx = bvalid ? *reinterpret_cast<const f16x8*>(xb + 32 * u) : zero8;
+          part = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, cur[u]), bx, part,
+                                                        0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = fmaf(part[i], down, acc[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[par][wave][(4 * kg + i) * kGmRedPitch + col] = acc[i];
+    // LDS only: the next tile's loads stay in flight.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tid < 128) {
+      const int r = tid >> 3, b = tid & 7;
+      const int row = tile * T + r;
+      if (r < T && b < nt && row < n_out) {
+        float v = 0.f;
+#pragma unroll
+        for (int w8 = 0; w8 < kGmWaves; ++w8)
+          v += red[par][w8][r * kGmRedPitch + b] + red[par][w8][r * kGmRedPitch + b + 8];
         if (bias) v += bias_v;
         if (a.act == kActGelu) v = gelu_tanh(v);
         out[static_cast<int64_t>(b) * a.out_rs + static_cast<int64_t>(row >> 6) * a.out_hs +
@@ -1102,11 +1228,11 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
   int dev = 0, n_cu = 256;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
-  // Three or more x rows: the matrix-pipe kernel (one or two rows read the
+  // Three or more x rows: the matrix-pipe kernels (one or two rows read the
   // staged x cheaply enough that the FMA kernel's wider spread wins).
   const size_t gm_lds = static_cast<size_t>(x_dt == kF32 ? 2 : 1) * a.n_tokens * (a.n_in + 8) * 2;
-  if (a.n_tokens >= 3 && (a.n_in & 31) == 0 && gm_lds <= kGmMaxDynLds &&
-      (x_dt == kF32 || x_dt == kF16)) {
+  const bool long_rows = x_dt == kF32 && a.n_in > 256 * kLnCache;
+  if (a.n_tokens >= 3 && (long_rows || (gm_lds <= kGmMaxDynLds && (x_dt == kF32 || x_dt == kF16)))) {
     // Tiles of T features, T chosen so that the tiles of all groups just
     // cover one workgroup per CU (a d x d matrix measured fastest that way:
     // two smaller tiles per CU stage x twice), or exactly k per CU when one
@@ -1114,56 +1240,48 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
     // tiles gave 64 CUs two tiles and the rest one. Up to as many workgroups
     // as fit at once (LDS and registers decide) share the tiles, looping.
     const dim3 gblock(64 * kGmWaves);
-#define WRS_GM_L(XT, OT, LN)                                                                  \
+    const int64_t rows = static_cast<int64_t>(a.n_out) * a.n_groups;
+    const int64_t per_cu_tiles = (rows + 16 * n_cu - 1) / (16 * n_cu);
+    const int T = static_cast<int>(std::max<int64_t>(
+        1, std::min<int64_t>(16, (rows + per_cu_tiles * n_cu - 1) / (per_cu_tiles * n_cu))));
+    const int n_tiles = (a.n_out + T - 1) / T;
+#define WRS_GM_K(KERNEL, LDS)                                                                 \
   {                                                                                           \
-    const void* fn = reinterpret_cast<const void*>(&gemv_f16w_mfma<XT, OT, LN>);              \
+    const void* fn = reinterpret_cast<const void*>(&KERNEL);                                  \
     static std::atomic<uint64_t> attr_set{0};  /* one bit per device */                       \
-    if (dev < 64 && !(attr_set.load(std::memory_order_acquire) & (uint64_t{1} << dev))) {     \
+    if (LDS > 0 && dev < 64 &&                                                                \
+        !(attr_set.load(std::memory_order_acquire) & (uint64_t{1} << dev))) {                 \
       const hipError_t e = hipFuncSetAttribute(                                               \
           fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGmMaxDynLds));    \
       if (e != hipSuccess) return e;                                                          \
       attr_set.fetch_or(uint64_t{1} << dev, std::memory_order_acq_rel);                       \
     }                                                                                         \
     int per_cu = 1;                                                                           \
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, gblock.x, gm_lds) !=         \
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, gblock.x, LDS) !=           \
             hipSuccess ||                                                                     \
         per_cu < 1)                                                                           \
       per_cu = 1;                                                                             \
-    const int64_t rows = static_cast<int64_t>(a.n_out) * a.n_groups;                         \
-    const int64_t per_cu_tiles = (rows + 16 * n_cu - 1) / (16 * n_cu);                      \
-    const int T = static_cast<int>(std::max<int64_t>(                                        \
-        1, std::min<int64_t>(16, (rows + per_cu_tiles * n_cu - 1) / (per_cu_tiles * n_cu)))); \
-    const int n_tiles = (a.n_out + T - 1) / T;                                                \
     const dim3 ggrid(std::min(n_tiles, n_cu * std::min(per_cu, 2)), a.n_groups);              \
-    hipLaunchKernelGGL((gemv_f16w_mfma<XT, OT, LN>), ggrid, gblock, gm_lds, s, a, T);         \
+    hipLaunchKernelGGL((KERNEL), ggrid, gblock, LDS, s, a, T);                                \
+    return hipGetLastError();                                                                 \
   }
-#define WRS_GM(XT, OT)                 \
-  if (a.ln_g) {                        \
-    WRS_GM_L(XT, OT, true)             \
-  } else {                             \
-    WRS_GM_L(XT, OT, false)            \
-  }
-#define WRS_GM16(XT, OT) WRS_GM_L(XT, OT, false)
-    if (x_dt == kF32) {
-      switch (out_dt) {
-        case kF32: WRS_GM(float, float); break;
-        case kF16: WRS_GM(float, _Float16); break;
-        case kBF16: WRS_GM(float, __bf16); break;
-        default: return hipErrorInvalidValue;
-      }
-    } else {
-      if (a.ln_g) return hipErrorInvalidValue;  // the fused LayerNorm takes f32 rows
-      switch (out_dt) {
-        case kF32: WRS_GM16(_Float16, float); break;
-        case kF16: WRS_GM16(_Float16, _Float16); break;
-        case kBF16: WRS_GM16(_Float16, __bf16); break;
-        default: return hipErrorInvalidValue;
-      }
+#define WRS_GM(OT)                                                              \
+  if (x_dt == kF16) {                                                           \
+    if (a.ln_g) return hipErrorInvalidValue;  /* a fused LayerNorm takes f32 */ \
+    WRS_GM_K((gemv_f16w_mfma<_Float16, OT, false>), gm_lds)                     \
+  }                                                                             \
+  if (long_rows && a.ln_g) WRS_GM_K((gemv_f16w_long<OT, true>), 0)              \
+  if (long_rows) WRS_GM_K((gemv_f16w_long<OT, false>), 0)                       \
+  if (a.ln_g) WRS_GM_K((gemv_f16w_mfma<float, OT, true>), gm_lds)               \
+  WRS_GM_K((gemv_f16w_mfma<float, OT, false>), gm_lds)
+    switch (out_dt) {
+      case kF32: WRS_GM(float)
+      case kF16: WRS_GM(_Float16)
+      case kBF16: WRS_GM(__bf16)
+      default: return hipErrorInvalidValue;
     }
-#undef WRS_GM16
 #undef WRS_GM
-#undef WRS_GM_L
-    return hipGetLastError();
+#undef WRS_GM_K
   }
   // Up to kGemvSmallOut features: one feature per wave, so that the matrix
   // spreads over ~n_out / 8 CUs; beyond it 4 features per wave share each

@@ -53,6 +53,34 @@ __device__ inline float ld_agent(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// x op x[lane ^ 32] and x op x[lane ^ 16] with the gfx950 lane-swap VALU
+// instructions (no LDS round trip). Issued as inline asm on two distinct
+// registers: the swap writes both operands.
+__device__ inline void swap32(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+__device__ inline void swap16(float& a, float& b) {
+  asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+}
+__device__ inline float max_x16_x32(float x) {
+  float a = x, b = x;
+  swap16(a, b);  // a, b: x of this row and of the row 16 lanes away
+  x = fmaxf(a, b);
+  a = x;
+  b = x;
+  swap32(a, b);
+  return fmaxf(a, b);
+}
+__device__ inline float sum_x16_x32(float x) {
+  float a = x, b = x;
+  swap16(a, b);
+  x = a + b;
+  a = x;
+  b = x;
+  swap32(a, b);
+  return a + b;
+}
+
 // Flash-attention prefill over full query/key sequences
 // (crates/tensor/src/ops/attention.rs:68-243 semantics).
 struct PrefillArgs {
