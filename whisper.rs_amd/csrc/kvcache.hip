@@ -16,12 +16,17 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// One thread per 8 values: row i, head h, 8-column group c.
-__global__ void kv_write_rows(const float* src, int64_t src_rs, int n, int n_heads,
-                              _Float16* dst, int64_t dst_hs, int pos) {
+// K (blockIdx.y == 0) and V rows in one launch: a step's append is bound by its
+// launches (five slots of a 12-layer step: 120 -> 60, ~2 us each).
+// One thread per 8 values: row i, head h, 8-column group c. The source rows need
+// only 4-byte alignment.
+__global__ void kv_write_rows(KvRows rows, int64_t src_rs, int n, int n_heads, int64_t dst_hs,
+                              int pos) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t total = static_cast<int64_t>(n) * n_heads * 8;
   if (t >= total) return;
+  const float* src = blockIdx.y ? rows.v_src : rows.k_src;
+  _Float16* dst = static_cast<_Float16*>(blockIdx.y ? rows.v_dst : rows.k_dst);
   const int c = static_cast<int>(t & 7);
   const int64_t ih = t >> 3;
   const int h = static_cast<int>(ih % n_heads);
@@ -36,11 +41,13 @@ __global__ void kv_write_rows(const float* src, int64_t src_rs, int n, int n_hea
 
 // f32 planes: one thread per 4 values (row i, head h, 4-column group c). The
 // source rows need only 4-byte alignment; the plane rows are 256-byte aligned.
-__global__ void kv_write_rows_f32(const float* src, int64_t src_rs, int n, int n_heads,
-                                  float* dst, int64_t dst_hs, int pos) {
+__global__ void kv_write_rows_f32(KvRows rows, int64_t src_rs, int n, int n_heads, int64_t dst_hs,
+                                  int pos) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   const int64_t total = static_cast<int64_t>(n) * n_heads * 16;
   if (t >= total) return;
+  const float* src = blockIdx.y ? rows.v_src : rows.k_src;
+  float* dst = static_cast<float*>(blockIdx.y ? rows.v_dst : rows.k_dst);
   const int c = static_cast<int>(t & 15);
   const int64_t ih = t >> 4;
   const int h = static_cast<int>(ih % n_heads);
@@ -54,9 +61,9 @@ __global__ void kv_write_rows_f32(const float* src, int64_t src_rs, int n, int n
 // 8 halves); every block is read before any thread writes it, and later blocks
 // only read rows above everything written so far, so the in-place move is safe
 // for any drop >= 1.
-__global__ __launch_bounds__(256) void kv_slide(_Float16* base, int64_t layer_stride,
+__global__ __launch_bounds__(256) void kv_slide(_Float16* k, _Float16* v, int64_t layer_stride,
                                                 int64_t plane_stride, int len, int drop) {
-  _Float16* p = base + blockIdx.y * layer_stride + blockIdx.x * plane_stride;
+  _Float16* p = (blockIdx.z ? v : k) + blockIdx.y * layer_stride + blockIdx.x * plane_stride;
   const int keep = len - drop;
   const int tid = threadIdx.x;
   for (int r0 = 0; r0 < keep; r0 += 32) {
@@ -70,15 +77,30 @@ __global__ __launch_bounds__(256) void kv_slide(_Float16* base, int64_t layer_st
   }
 }
 
-// Copy rows [0, len) of every (layer, head) plane from one slot to another.
-__global__ __launch_bounds__(256) void kv_copy_planes(const _Float16* src, _Float16* dst,
-                                                      int64_t layer_stride,
-                                                      int64_t plane_stride, int len) {
+// Copy rows [0, len) of every (layer, head) plane of K and V from one slot to
+// another, kCopyUnits 16-byte units per workgroup, all read before any is written
+// (a workgroup that walked a whole plane waited out a round trip per 4 KB).
+constexpr int kCopyUnits = 1024;
+__global__ __launch_bounds__(256) void kv_copy_planes(const _Float16* k_src, _Float16* k_dst,
+                                                      const _Float16* v_src, _Float16* v_dst,
+                                                      int64_t layer_stride, int64_t plane_stride,
+                                                      int len, int parts) {
+  const int which = blockIdx.z / parts, part = blockIdx.z - which * parts;
   const int64_t off = blockIdx.y * layer_stride + blockIdx.x * plane_stride;
-  const u32x4* s = reinterpret_cast<const u32x4*>(src + off);
-  u32x4* d = reinterpret_cast<u32x4*>(dst + off);
+  const u32x4* s = reinterpret_cast<const u32x4*>((which ? v_src : k_src) + off);
+  u32x4* d = reinterpret_cast<u32x4*>((which ? v_dst : k_dst) + off);
   const int n = len * 8;  // 16-byte units
-  for (int i = threadIdx.x; i < n; i += 256) d[i] = s[i];
+  u32x4 x[kCopyUnits / 256];
+#pragma unroll
+  for (int u = 0; u < kCopyUnits / 256; ++u) {
+    const int i = part * kCopyUnits + 256 * u + threadIdx.x;
+    x[u] = s[i < n ? i : 0];
+  }
+#pragma unroll
+  for (int u = 0; u < kCopyUnits / 256; ++u) {
+    const int i = part * kCopyUnits + 256 * u + threadIdx.x;
+    if (i < n) d[i] = x[u];
+  }
 }
 
 // Zero fill of a strided [batch][head][row][cols] f32 region (replaces
@@ -125,42 +147,37 @@ hipError_t launch_fill_zero_u32(unsigned* p, int64_t n, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_kv_write_rows(const float* src, int64_t src_rs, int n, int n_heads,
-                                _Float16* dst, int64_t dst_hs, int pos, hipStream_t s) {
-  const int64_t total = static_cast<int64_t>(n) * n_heads * 8;
+hipError_t launch_kv_write_rows(const KvRows& rows, bool f32, int64_t src_rs, int n, int n_heads,
+                                int64_t dst_hs, int pos, hipStream_t s) {
+  const int64_t total = static_cast<int64_t>(n) * n_heads * (f32 ? 16 : 8);
   if (total <= 0) return hipSuccess;
   const int64_t blocks = (total + 255) / 256;
   if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(kv_write_rows, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, src,
-                     src_rs, n, n_heads, dst, dst_hs, pos);
+  const dim3 grid(static_cast<unsigned>(blocks), 2);
+  if (f32)
+    hipLaunchKernelGGL(kv_write_rows_f32, grid, dim3(256), 0, s, rows, src_rs, n, n_heads, dst_hs, pos);
+  else
+    hipLaunchKernelGGL(kv_write_rows, grid, dim3(256), 0, s, rows, src_rs, n, n_heads, dst_hs, pos);
   return hipGetLastError();
 }
 
-hipError_t launch_kv_write_rows_f32(const float* src, int64_t src_rs, int n, int n_heads,
-                                    float* dst, int64_t dst_hs, int pos, hipStream_t s) {
-  const int64_t total = static_cast<int64_t>(n) * n_heads * 16;
-  if (total <= 0) return hipSuccess;
-  const int64_t blocks = (total + 255) / 256;
-  if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
-  hipLaunchKernelGGL(kv_write_rows_f32, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, src,
-                     src_rs, n, n_heads, dst, dst_hs, pos);
-  return hipGetLastError();
-}
-
-hipError_t launch_kv_slide(_Float16* base, int64_t layer_stride, int64_t plane_stride,
+hipError_t launch_kv_slide(_Float16* k, _Float16* v, int64_t layer_stride, int64_t plane_stride,
                            int n_layers, int n_heads, int len, int drop, hipStream_t s) {
   if (n_layers <= 0 || n_heads <= 0 || drop <= 0 || len <= drop) return hipSuccess;
-  hipLaunchKernelGGL(kv_slide, dim3(n_heads, n_layers), dim3(256), 0, s, base, layer_stride,
+  hipLaunchKernelGGL(kv_slide, dim3(n_heads, n_layers, 2), dim3(256), 0, s, k, v, layer_stride,
                      plane_stride, len, drop);
   return hipGetLastError();
 }
 
-hipError_t launch_kv_copy_planes(const _Float16* src, _Float16* dst, int64_t layer_stride,
-                                 int64_t plane_stride, int n_layers, int n_heads, int len,
-                                 hipStream_t s) {
+hipError_t launch_kv_copy_planes(const _Float16* k_src, _Float16* k_dst, const _Float16* v_src,
+                                 _Float16* v_dst, int64_t layer_stride, int64_t plane_stride,
+                                 int n_layers, int n_heads, int len, hipStream_t s) {
   if (n_layers <= 0 || n_heads <= 0 || len <= 0) return hipSuccess;
-  hipLaunchKernelGGL(kv_copy_planes, dim3(n_heads, n_layers), dim3(256), 0, s, src, dst,
-                     layer_stride, plane_stride, len);
+  const int64_t parts = (static_cast<int64_t>(len) * 8 + kCopyUnits - 1) / kCopyUnits;
+  if (len > (1 << 27) || 2 * parts > 65535) return hipErrorInvalidConfiguration;
+  hipLaunchKernelGGL(kv_copy_planes, dim3(n_heads, n_layers, static_cast<unsigned>(2 * parts)),
+                     dim3(256), 0, s, k_src, k_dst, v_src, v_dst, layer_stride, plane_stride, len,
+                     static_cast<int>(parts));
   return hipGetLastError();
 }
 

@@ -796,19 +796,15 @@ int wrs_attn_prefill(wrs_attn_ctx* c, int q_dtype, const void* q, const wrs_layo
 
 namespace {
 
-// Rows [pos, pos + n) of every head plane of one plane set (element `off`
-// on), from n f32 rows of d_model: converted to f16, or copied for f32 arenas.
-int write_rows(wrs_attn_ctx* c, wrs_kv* kv, const float* src, int64_t src_rs, size_t n,
-               void* base, size_t off, int64_t plane, size_t pos) {
-  const int nh = static_cast<int>(kv->n_heads);
-  if (kv->f32())
-    WRS_HIP(c, wrs::launch_kv_write_rows_f32(src, src_rs, static_cast<int>(n), nh,
-                                             wrs_kv::f32p(base, off), plane,
-                                             static_cast<int>(pos), c->stream));
-  else
-    WRS_HIP(c, wrs::launch_kv_write_rows(src, src_rs, static_cast<int>(n), nh,
-                                         static_cast<_Float16*>(base) + off, plane,
-                                         static_cast<int>(pos), c->stream));
+// Rows [pos, pos + n) of every head plane of K and V (element `off` on), from n
+// f32 rows of d_model each: converted to f16, or copied for f32 arenas.
+int write_rows(wrs_attn_ctx* c, wrs_kv* kv, const float* k_src, const float* v_src, size_t n,
+               void* k, void* v, size_t off, size_t plane, size_t pos) {
+  const wrs::KvRows rows{k_src, v_src, kv->words(k, off), kv->words(v, off)};
+  WRS_HIP(c, wrs::launch_kv_write_rows(rows, kv->f32(), static_cast<int64_t>(kv->d_model()),
+                                       static_cast<int>(n), static_cast<int>(kv->n_heads),
+                                       static_cast<int64_t>(plane), static_cast<int>(pos),
+                                       c->stream));
   return WRS_OK;
 }
 
@@ -1001,14 +997,11 @@ int wrs_kv_copy_slot(wrs_kv* kv, size_t dst, size_t src) {
       static_cast<int64_t>(kv->n_slots * kv->n_heads * kv->plane() * w);
   const int64_t plane = static_cast<int64_t>(kv->plane() * w);
   const int n = static_cast<int>(kv->len[src] * w);
-  WRS_HIP(c, wrs::launch_kv_copy_planes(kv->words(kv->k_self, kv->self_off(0, src)),
-                                        kv->words(kv->k_self, kv->self_off(0, dst)), layer_stride,
-                                        plane, static_cast<int>(kv->n_layers),
-                                        static_cast<int>(kv->n_heads), n, c->stream));
-  WRS_HIP(c, wrs::launch_kv_copy_planes(kv->words(kv->v_self, kv->self_off(0, src)),
-                                        kv->words(kv->v_self, kv->self_off(0, dst)), layer_stride,
-                                        plane, static_cast<int>(kv->n_layers),
-                                        static_cast<int>(kv->n_heads), n, c->stream));
+  const size_t from = kv->self_off(0, src), to = kv->self_off(0, dst);
+  WRS_HIP(c, wrs::launch_kv_copy_planes(
+                 kv->words(kv->k_self, from), kv->words(kv->k_self, to),
+                 kv->words(kv->v_self, from), kv->words(kv->v_self, to), layer_stride, plane,
+                 static_cast<int>(kv->n_layers), static_cast<int>(kv->n_heads), n, c->stream));
   kv->len[dst] = kv->len[src];
   return WRS_OK;
 }
@@ -1045,11 +1038,11 @@ int wrs_kv_slide_to_fit(wrs_kv* kv, size_t slot, size_t n_new, size_t max_ctx, s
     const int64_t layer_stride =
         static_cast<int64_t>(kv->n_slots * kv->n_heads * kv->plane() * w);
     const int64_t plane = static_cast<int64_t>(kv->plane() * w);
-    for (void* base : {kv->k_self, kv->v_self})
-      WRS_HIP(c, wrs::launch_kv_slide(kv->words(base, kv->self_off(0, slot)), layer_stride, plane,
-                                      static_cast<int>(kv->n_layers),
-                                      static_cast<int>(kv->n_heads), static_cast<int>(t_past * w),
-                                      static_cast<int>(drop * w), c->stream));
+    const size_t at = kv->self_off(0, slot);
+    WRS_HIP(c, wrs::launch_kv_slide(kv->words(kv->k_self, at), kv->words(kv->v_self, at),
+                                    layer_stride, plane, static_cast<int>(kv->n_layers),
+                                    static_cast<int>(kv->n_heads), static_cast<int>(t_past * w),
+                                    static_cast<int>(drop * w), c->stream));
     t_past -= drop;
     kv->len[slot] = t_past;
   }
@@ -1078,12 +1071,8 @@ int wrs_kv_append(wrs_kv* kv, size_t layer, size_t slot, const float* k_rows,
   if (rc) return rc;
   const float* dv = to_device_f32(c, v_rows, floats, src_on_host, align_up(floats * 4, 256), &rc);
   if (rc) return rc;
-  const int64_t dm = static_cast<int64_t>(kv->d_model());
-  const int64_t plane = static_cast<int64_t>(kv->plane());
-  const size_t off = kv->self_off(layer, slot);
-  rc = write_rows(c, kv, dk, dm, n, kv->k_self, off, plane, pos);
-  if (rc) return rc;
-  rc = write_rows(c, kv, dv, dm, n, kv->v_self, off, plane, pos);
+  rc = write_rows(c, kv, dk, dv, n, kv->k_self, kv->v_self, kv->self_off(layer, slot),
+                  kv->plane(), pos);
   if (rc) return rc;
   if (src_on_host) WRS_HIP(c, hipStreamSynchronize(c->stream));
   return WRS_OK;
@@ -1118,11 +1107,8 @@ int wrs_kv_set_cross(wrs_kv* kv, size_t layer, const float* k, const float* v, s
     if (rc) return rc;
     const float* dv = to_device_f32(c, v, floats, src_on_host, align_up(floats * 4, 256), &rc);
     if (rc) return rc;
-    const int64_t dm = static_cast<int64_t>(kv->d_model());
-    const int64_t plane = static_cast<int64_t>(kv->n_audio_max * 64);
-    rc = write_rows(c, kv, dk, dm, n_audio, kv->k_cross, kv->cross_off(layer), plane, 0);
-    if (rc) return rc;
-    rc = write_rows(c, kv, dv, dm, n_audio, kv->v_cross, kv->cross_off(layer), plane, 0);
+    rc = write_rows(c, kv, dk, dv, n_audio, kv->k_cross, kv->v_cross, kv->cross_off(layer),
+                    kv->n_audio_max * 64, 0);
     if (rc) return rc;
     if (src_on_host) WRS_HIP(c, hipStreamSynchronize(c->stream));
   }

@@ -326,21 +326,23 @@ hipError_t launch_fill_zero_rows(float* base, int64_t bs, int64_t hs, int64_t rs
 hipError_t launch_fill_zero_u32(unsigned* p, int64_t n, hipStream_t s);
 
 // KV arena kernels.
-// f32 rows [n][d_model] (row stride src_rs) -> f16 planes: head h, row i at
-// dst + h*dst_hs + (pos + i)*64.
-hipError_t launch_kv_write_rows(const float* src, int64_t src_rs, int n, int n_heads,
-                                _Float16* dst, int64_t dst_hs, int pos, hipStream_t s);
-// The same into f32 planes (a copy).
-hipError_t launch_kv_write_rows_f32(const float* src, int64_t src_rs, int n, int n_heads,
-                                    float* dst, int64_t dst_hs, int pos, hipStream_t s);
-// Planes of one slot: plane (l, h) at base + l*layer_stride + h*plane_stride,
-// in rows of 64 f16 (an f32 plane is passed as twice the rows and strides).
+// f32 rows [n][d_model] of K and of V (row stride src_rs) -> planes, f16 or f32:
+// head h, row i at dst + h*dst_hs + (pos + i)*64.
+struct KvRows {
+  const float *k_src, *v_src;
+  void *k_dst, *v_dst;
+};
+hipError_t launch_kv_write_rows(const KvRows& rows, bool f32, int64_t src_rs, int n, int n_heads,
+                                int64_t dst_hs, int pos, hipStream_t s);
+// K and V planes of one slot: plane (l, h) at base + l*layer_stride +
+// h*plane_stride, in rows of 64 f16 (an f32 plane is passed as twice the rows
+// and strides).
 // Move rows [drop, len) of every plane down to [0, len - drop).
-hipError_t launch_kv_slide(_Float16* base, int64_t layer_stride, int64_t plane_stride,
+hipError_t launch_kv_slide(_Float16* k, _Float16* v, int64_t layer_stride, int64_t plane_stride,
                            int n_layers, int n_heads, int len, int drop, hipStream_t s);
 // Copy rows [0, len) of every plane from src to dst (same plane geometry).
-hipError_t launch_kv_copy_planes(const _Float16* src, _Float16* dst, int64_t layer_stride,
-                                 int64_t plane_stride, int n_layers, int n_heads, int len,
-                                 hipStream_t s);
+hipError_t launch_kv_copy_planes(const _Float16* k_src, _Float16* k_dst, const _Float16* v_src,
+                                 _Float16* v_dst, int64_t layer_stride, int64_t plane_stride,
+                                 int n_layers, int n_heads, int len, hipStream_t s);
 
 }  // namespace wrs
