@@ -530,3 +530,22 @@ def test_decode_rows_long(wrs, ctx, n_tokens, n_in, n_out):
     wrs.linear(normed, wd, bd, ref, ctx=ctx)
     wrs.gelu_inplace(ref, ctx=ctx)
     assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("n_tokens", [2, 5])
+@pytest.mark.parametrize("n_groups", [8, 9, 17, 64])
+def test_linear_group_counts(wrs, ctx, n_tokens, n_groups):
+    """Group counts at and past one launch's weight groups, up to the most a
+    call takes, with and without biases: each group equals its own call."""
+    note(f"linear group counts T={n_tokens} G={n_groups}")
+    rng = np.random.default_rng(n_groups + n_tokens)
+    x = dev(rng.standard_normal((n_tokens, 192)).astype(np.float32))
+    ws = [torch.from_numpy(_weights(70, 192, 500 + g)).cuda() for g in range(n_groups)]
+    bs = [dev(rng.standard_normal(70).astype(np.float32)) if g % 3 else None
+          for g in range(n_groups)]
+    outs = [torch.full((n_tokens, 70), float("nan"), device="cuda") for _ in ws]
+    wrs.linear_group(x, ws, bs, outs, ctx=ctx)
+    for w, b, o in zip(ws, bs, outs):
+        ref = torch.empty_like(o)
+        wrs.linear(x, w, b, ref, ctx=ctx)
+        assert torch.equal(o, ref)

@@ -759,7 +759,7 @@ __device__ inline float wave_max64(float v) {
 }
 
 template <typename XT, typename OutT, bool kLn>
-__global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_mfma(GemvArgs a, int T) {
+__global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_mfma(GemvArgs a, int T) {
   extern __shared__ __attribute__((aligned(16))) _Float16 gxs[];  // [parts * nt][n_in + 8]
   __shared__ __attribute__((aligned(16))) float red[2][kGmWaves][kGmRedFloats];
   __shared__ float dn[8];
@@ -918,7 +918,7 @@ constexpr int kGlKB = 4;                       // k-steps per wave per batch: 12
 constexpr int kGlPitch = 32 * kGlKB + 8;       // f16 elements of a staged row
 
 template <typename OutT, bool kLn>
-__global__ __launch_bounds__(64 * kGmWaves) void gemv_f16w_long(GemvArgs a, int T) {
+__global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_long(GemvArgs a, int T) {
   __shared__ __attribute__((aligned(16))) _Float16 xs[kGmWaves][16][kGlPitch];  // hi rows, lo rows
   __shared__ __attribute__((aligned(16))) float red[2][kGmWaves][kGmRedFloats];
   __shared__ float dn[kGmWaves][8], row_mean[8], row_inv[8];
@@ -1194,6 +1194,22 @@ __global__ __launch_bounds__(256) void linear_split_rows(const float* x, int64_t
 
 }  // namespace
 
+namespace {
+
+// CUs of the current device, read once: asked for at each launch, this and the
+// occupancy of the kernel cost 0.35 us of a 6.7 us call.
+int linear_cus() {
+  static const int cus = [] {
+    int dev = 0, n = 256;
+    if (hipGetDevice(&dev) == hipSuccess)
+      (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
+    return n;
+  }();
+  return cus;
+}
+
+}  // namespace
+
 hipError_t launch_linear_split(const float* x, int64_t x_rs, int n_tokens, int n_in,
                                const float* ln_g, const float* ln_b, float ln_eps, _Float16* xs,
                                float* row_scale, hipStream_t s) {
@@ -1225,9 +1241,9 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
   if (a.n_tokens <= 0 || a.n_out <= 0 || a.n_groups <= 0) return hipSuccess;
   if (a.n_tokens > kGemvMaxRows) return hipErrorInvalidValue;
   if (a.n_tokens * a.n_in > kGemvXFloats) return hipErrorInvalidValue;
-  int dev = 0, n_cu = 256;
-  if (hipGetDevice(&dev) == hipSuccess)
-    (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
+  const int n_cu = linear_cus();
+  int dev = 0;
+  (void)hipGetDevice(&dev);
   // Three or more x rows: the matrix-pipe kernels (one or two rows read the
   // staged x cheaply enough that the FMA kernel's wider spread wins).
   const size_t gm_lds = static_cast<size_t>(x_dt == kF32 ? 2 : 1) * a.n_tokens * (a.n_in + 8) * 2;
@@ -1245,6 +1261,10 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
     const int T = static_cast<int>(std::max<int64_t>(
         1, std::min<int64_t>(16, (rows + per_cu_tiles * n_cu - 1) / (per_cu_tiles * n_cu))));
     const int n_tiles = (a.n_out + T - 1) / T;
+    // Two workgroups of 8 waves fit a CU where their LDS does (the launch bounds
+    // hold their registers to 128).
+    const size_t lds = kGmStaticLds + (long_rows ? 0 : gm_lds);
+    const int per_cu = long_rows || 2 * lds <= 160 * 1024 ? 2 : 1;
 #define WRS_GM_K(KERNEL, LDS)                                                                 \
   {                                                                                           \
     const void* fn = reinterpret_cast<const void*>(&KERNEL);                                  \
@@ -1256,12 +1276,7 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
       if (e != hipSuccess) return e;                                                          \
       attr_set.fetch_or(uint64_t{1} << dev, std::memory_order_acq_rel);                       \
     }                                                                                         \
-    int per_cu = 1;                                                                           \
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, gblock.x, LDS) !=           \
-            hipSuccess ||                                                                     \
-        per_cu < 1)                                                                           \
-      per_cu = 1;                                                                             \
-    const dim3 ggrid(std::min(n_tiles, n_cu * std::min(per_cu, 2)), a.n_groups);              \
+    const dim3 ggrid(std::min(n_tiles, n_cu * per_cu), a.n_groups);                            \
     hipLaunchKernelGGL((KERNEL), ggrid, gblock, LDS, s, a, T);                                \
     return hipGetLastError();                                                                 \
   }
@@ -1331,17 +1346,6 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
 }
 
 namespace {
-
-// CUs of the current device, read once.
-int linear_cus() {
-  static const int cus = [] {
-    int dev = 0, n = 256;
-    if (hipGetDevice(&dev) == hipSuccess)
-      (void)hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-    return n;
-  }();
-  return cus;
-}
 
 int64_t n_tiles(const LinearArgs& a, int ft, int tt) {
   return static_cast<int64_t>((a.n_out + ft - 1) / ft) * ((a.n_tokens + tt - 1) / tt);

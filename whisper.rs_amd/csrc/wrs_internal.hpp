@@ -286,6 +286,11 @@ size_t linear_split_words();
 // Decode-sized batches (n_tokens <= kGemvMaxRows) of the same product on the
 // f16 weight stream; x is f32 or f16 with row stride x_rs, no split needed.
 constexpr int kGemvMaxRows = 8;
+// Weight groups of one launch; more take further launches. A launch copies its
+// arguments, and these launches are host-bound in a step that is not captured:
+// room for 64 groups cost 0.5 us of a 6.7 us call (5 rows 768 x 768), room for 8 is
+// what a layer's projections need (3).
+constexpr int kMaxGemvGroups = 8;
 constexpr int kGemvXFloats = 40960;  // n_tokens * n_in staged in LDS (160 KB)
 struct GemvArgs {
   const void* x;
@@ -298,9 +303,9 @@ struct GemvArgs {
   const float* ln_b;
   float ln_eps;
   int act;  // Act, applied after the bias
-  const _Float16* w[kMaxLinearGroups];
-  const float* bias[kMaxLinearGroups];
-  void* out[kMaxLinearGroups];
+  const _Float16* w[kMaxGemvGroups];
+  const float* bias[kMaxGemvGroups];
+  void* out[kMaxGemvGroups];
 };
 hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s);
 // f32 rows -> [hi | lo] f16 rows (kSplitParts n_in each) and per-row 2^-shift,
