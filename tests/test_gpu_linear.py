@@ -549,3 +549,47 @@ def test_linear_group_counts(wrs, ctx, n_tokens, n_groups):
         ref = torch.empty_like(o)
         wrs.linear(x, w, b, ref, ctx=ctx)
         assert torch.equal(o, ref)
+
+
+@pytest.mark.parametrize("n_tokens", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("n_in,n_out", [(64, 1), (192, 70), (1280, 1281), (1280, 1843),
+                                        (1280, 1844), (1344, 1280), (3136, 1281), (5120, 9)])
+def test_decode_rows_by_fma(wrs, ctx, n_tokens, n_in, n_out):
+    """f32 rows on both sides of the line between FMAs and the matrix pipe: a
+    last slice of columns that is part empty, one and several slices a wave, a
+    last tile of features that is part empty; infinite weights and rows stay in
+    their own outputs; and a fused LayerNorm and GELU, alone and as one of three
+    groups, give the separate calls' bits."""
+    note(f"decode rows by fma T={n_tokens} K={n_in} N={n_out}")
+    rng = np.random.default_rng(n_in + n_out + n_tokens)
+    x = rng.standard_normal((n_tokens, n_in)).astype(np.float32)
+    x *= 10.0 ** rng.uniform(-6, 6, (n_tokens, 1)).astype(np.float32)
+    w = _weights(n_out, n_in, n_in + 11)
+    b = rng.standard_normal(n_out).astype(np.float32)
+    buf = torch.full((n_tokens, n_in + 4), float("nan"), device="cuda")
+    buf[:, :n_in] = dev(x)
+    wd, bd = torch.from_numpy(w).cuda(), dev(b)
+    out = torch.full((n_tokens, n_out), float("nan"), device="cuda")
+    wrs.linear(buf[:, :n_in], wd, bd, out, ctx=ctx)
+    bound = _gamma_bound(x, w) + 2.0 ** -23 * np.abs(b)
+    assert (np.abs(host(out) - _exact(x, w, b)) <= bound).all()
+    gamma = dev((1.0 + 0.1 * rng.standard_normal(n_in)).astype(np.float32))
+    beta = dev((0.1 * rng.standard_normal(n_in)).astype(np.float32))
+    xd = dev(x)
+    outs = [torch.full((n_tokens, n_out), float("nan"), device="cuda") for _ in range(3)]
+    wrs.linear_fused(xd, [wd] * 3, [bd, None, bd], outs, ln=(gamma, beta, 1e-5), act="gelu",
+                     ctx=ctx)
+    wrs.linear_fused(xd, [wd], [bd], [out], ln=(gamma, beta, 1e-5), act="gelu", ctx=ctx)
+    normed, ref = torch.empty_like(xd), torch.empty_like(out)
+    wrs.layer_norm(xd, gamma, beta, 1e-5, normed, ctx=ctx)
+    wrs.linear(normed, wd, bd, ref, ctx=ctx)
+    wrs.gelu_inplace(ref, ctx=ctx)
+    assert torch.equal(out, ref) and torch.equal(outs[0], ref) and torch.equal(outs[2], ref)
+    if n_out > 1:
+        wd[0, -1] = float("inf")
+        xd[-1, 0] = float("inf")
+        got = torch.empty_like(out)
+        wrs.linear(xd, wd, bd, got, ctx=ctx)
+        wrs.linear(dev(x), torch.from_numpy(w).cuda(), bd, out, ctx=ctx)
+        assert torch.equal(got[:-1, 1:], out[:-1, 1:])
+        assert not torch.isfinite(got[-1]).any() and not torch.isfinite(got[:, 0]).any()

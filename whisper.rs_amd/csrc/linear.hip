@@ -450,19 +450,19 @@ __global__ __launch_bounds__(C::kThreads, 1) void linear_f16w(LinearArgs a, int 
   }
 }
 
-// K7 (gemv_f16w): decode-sized batches (n_tokens <= 8: the beams of one step)
-//   against f16 weights, f16_gemv_parallel semantics (quant.rs:343-413). The
-//   weight stream is the whole cost, so every 16-byte chunk of W is read once
-//   for all rows. One persistent workgroup of 8 waves per CU stages all of x
-//   in LDS once (f32; f16 x widened exactly; at most kGemvXFloats values),
-//   then its waves walk groups of 4 output features (1 when n_out <= 4096, so
-//   that a d x d matrix still spreads over ~n_out / 8 CUs) across the matrix: lane l
-//   multiplies W[r][k..k+8) for k = 8 l + 512 m by the staged x of every row
-//   with f32 FMAs (the products dot_f16_f32 forms). The 16-byte loads of the
-//   next 2048-column batch (or of the next group) are in flight while a batch
-//   is multiplied. The row count is a template parameter (1..8), so no FMA is
-//   issued for absent rows; the 64 lane partials reduce with DPP and two
-//   cross-row moves, and lane b stores row b.
+// Decode-sized batches (n_tokens <= 8: the beams of one step) against f16 weights,
+// f16_gemv_parallel semantics (quant.rs:343-413). The weight stream is the whole
+// traffic, so every kernel below reads each 16-byte chunk of W once for all rows.
+//
+// K7 (gemv_f16w): one or two f16 rows.
+//   One persistent workgroup of 8 waves per CU stages all of x in LDS once,
+//   widened exactly, then its waves walk groups of 4 output features (1 when
+//   n_out <= 4096, so that a d x d matrix still spreads over ~n_out / 8 CUs)
+//   across the matrix: lane l multiplies W[r][k..k+8) for k = 8 l + 512 m by the
+//   staged x of every row with f32 FMAs (the products dot_f16_f32 forms). The
+//   16-byte loads of the next 2048-column batch (or of the next group) are in
+//   flight while a batch is multiplied. The 64 lane partials reduce with DPP and
+//   two cross-row moves, and lane b stores row b.
 constexpr int kGemvWaves = 8;
 constexpr int kGemvChunk = 2048;                // W columns per load batch
 constexpr int kGemvSmallOut = 4096;             // one feature per wave up to this n_out
@@ -506,21 +506,10 @@ __device__ inline void ln_row_stats(const float* xr, int d, float eps, float& me
   const float var = wave_sum64(q) / static_cast<float>(d);
   inv_std = 1.0f / sqrtf(var + eps);
 }
-__device__ inline f32x4 ln_apply(const float* xr, const float* g, const float* b, int k,
-                                 float mean, float inv_std) {
-  const f32x4 v = *reinterpret_cast<const f32x4*>(xr + k);
-  const f32x4 gg = *reinterpret_cast<const f32x4*>(g + k);
-  const f32x4 bb = *reinterpret_cast<const f32x4*>(b + k);
-  f32x4 o;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) o[j] = fmaf((v[j] - mean) * inv_std, gg[j], bb[j]);
-  return o;
-}
-
 // Rows of up to 256 * kLnCache values live in registers: lane l holds
 // columns 4 l + 256 i in v[i] (zeros past d). The loads are issued first
 // (ln_row_load), the arithmetic follows (ln_row_norm), with the arithmetic
-// of ln_row_stats / ln_apply exactly.
+// of ln_row_stats exactly.
 constexpr int kLnCache = 5;  // 1280 columns: every Whisper d_model
 __device__ inline void ln_row_load(const float* xr, const float* g, const float* b, int d,
                                    f32x4 (&v)[kLnCache], f32x4 (&gg)[kLnCache],
@@ -538,13 +527,13 @@ __device__ inline void ln_row_load(const float* xr, const float* g, const float*
     }
   }
 }
-__device__ inline void ln_row_norm(int d, float eps, f32x4 (&v)[kLnCache],
-                                   const f32x4 (&gg)[kLnCache], const f32x4 (&bb)[kLnCache]) {
+__device__ inline void ln_reg_stats(int d, float eps, const f32x4 (&v)[kLnCache], float& mean,
+                                    float& inv_std) {
   const int lane = threadIdx.x & 63;
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < kLnCache; ++i) s += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-  const float mean = wave_sum64(s) / static_cast<float>(d);
+  mean = wave_sum64(s) / static_cast<float>(d);
   float q = 0.0f;
 #pragma unroll
   for (int i = 0; i < kLnCache; ++i) {
@@ -553,14 +542,19 @@ __device__ inline void ln_row_norm(int d, float eps, f32x4 (&v)[kLnCache],
     for (int j = 0; j < 4; ++j) q = fmaf(v[i][j] - mean, v[i][j] - mean, q);
   }
   const float var = wave_sum64(q) / static_cast<float>(d);
-  const float inv_std = 1.0f / sqrtf(var + eps);
+  inv_std = 1.0f / sqrtf(var + eps);
+}
+__device__ inline void ln_row_norm(int d, float eps, f32x4 (&v)[kLnCache],
+                                   const f32x4 (&gg)[kLnCache], const f32x4 (&bb)[kLnCache]) {
+  float mean, inv_std;
+  ln_reg_stats(d, eps, v, mean, inv_std);
 #pragma unroll
   for (int i = 0; i < kLnCache; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[i][j] = fmaf((v[i][j] - mean) * inv_std, gg[i][j], bb[i][j]);
 }
 
-template <int NT, int kGemvRowsPerWave, typename XT, typename OutT>
+template <int NT, int kGemvRowsPerWave, typename OutT>
 __global__ __launch_bounds__(64 * kGemvWaves) void gemv_f16w(GemvArgs a) {
   __shared__ __attribute__((aligned(16))) float xs[kGemvXFloats];
   const int tid = threadIdx.x;
@@ -591,60 +585,25 @@ __global__ __launch_bounds__(64 * kGemvWaves) void gemv_f16w(GemvArgs a) {
   if (g4 < n_groups4) load_w(g4, 0, wv);  // in flight while x is staged
 
   // Stage x: row b at xs[b * n_in ..], 8 columns per thread and step, the
-  // 16-byte loads of 4 steps in flight before their stores. With a fused
-  // LayerNorm, wave b normalizes row b instead.
-  if constexpr (sizeof(XT) == 4) {
-    if (a.ln_g) {
-      if (wave < NT) {
-        const float* xr = static_cast<const float*>(a.x) + static_cast<int64_t>(wave) * a.x_rs;
-        if (n_in <= 256 * kLnCache) {
-          f32x4 y[kLnCache], gg[kLnCache], bb[kLnCache];
-          ln_row_load(xr, a.ln_g, a.ln_b, n_in, y, gg, bb);
-          ln_row_norm(n_in, a.ln_eps, y, gg, bb);
+  // 16-byte loads of 4 steps in flight before their stores.
+  const int n8 = NT * n_in / 8;
+  for (int e0 = tid; e0 < n8; e0 += 4 * 64 * kGemvWaves) {
+    uint4 v[4];
 #pragma unroll
-          for (int i = 0; i < kLnCache; ++i) {
-            const int k = 4 * lane + 256 * i;
-            if (k < n_in) *reinterpret_cast<f32x4*>(&xs[wave * n_in + k]) = y[i];
-          }
-        } else {
-          float mean, inv_std;
-          ln_row_stats(xr, n_in, a.ln_eps, mean, inv_std);
-          for (int k = 4 * lane; k < n_in; k += 256)
-            *reinterpret_cast<f32x4*>(&xs[wave * n_in + k]) =
-                ln_apply(xr, a.ln_g, a.ln_b, k, mean, inv_std);
-        }
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + u * 64 * kGemvWaves;
+      if (e < n8) {
+        const int b = (8 * e) / n_in, k = 8 * e - b * n_in;
+        v[u] = *reinterpret_cast<const uint4*>(static_cast<const _Float16*>(a.x) + b * a.x_rs + k);
       }
     }
-  }
-  if (!a.ln_g) {
-    const int n8 = NT * n_in / 8;
-    for (int e0 = tid; e0 < n8; e0 += 4 * 64 * kGemvWaves) {
-      float v[4][8];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = e0 + u * 64 * kGemvWaves;
-        if (e < n8) {
-          const int b = (8 * e) / n_in, k = 8 * e - b * n_in;
-          const XT* src = static_cast<const XT*>(a.x) + b * a.x_rs + k;
-          if constexpr (sizeof(XT) == 4) {
-            const float4 lo = *reinterpret_cast<const float4*>(src);
-            const float4 hi = *reinterpret_cast<const float4*>(src + 4);
-            v[u][0] = lo.x; v[u][1] = lo.y; v[u][2] = lo.z; v[u][3] = lo.w;
-            v[u][4] = hi.x; v[u][5] = hi.y; v[u][6] = hi.z; v[u][7] = hi.w;
-          } else {
-            const f16x8 h = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(src));
+    for (int u = 0; u < 4; ++u) {
+      const int e = e0 + u * 64 * kGemvWaves;
+      if (e < n8) {
+        const f16x8 h = __builtin_bit_cast(f16x8, v[u]);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) v[u][j] = static_cast<float>(h[j]);
-          }
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int e = e0 + u * 64 * kGemvWaves;
-        if (e < n8) {
-          *reinterpret_cast<float4*>(&xs[8 * e]) = float4{v[u][0], v[u][1], v[u][2], v[u][3]};
-          *reinterpret_cast<float4*>(&xs[8 * e + 4]) = float4{v[u][4], v[u][5], v[u][6], v[u][7]};
-        }
+        for (int j = 0; j < 8; ++j) xs[8 * e + j] = static_cast<float>(h[j]);
       }
     }
   }
@@ -722,7 +681,8 @@ __global__ __launch_bounds__(64 * kGemvWaves) void gemv_f16w(GemvArgs a) {
   }
 }
 
-// K7m (gemv_f16w_mfma): the same product for 3..8 x rows on the matrix pipe.
+// K7m (gemv_f16w_mfma): the same product on the matrix pipe, for 3..8 f16 rows and
+//   the f32 rows that K7f does not take.
 //   W is read in tiles of T <= 16 features: lane (c, g) of a wave loads 16
 //   bytes of feature c (columns 32 s + 8 g ..) per 32-column k-step s, which is
 //   the A operand of a 16x16x32 f16 MFMA as loaded; lanes c >= T repeat the
@@ -1088,6 +1048,189 @@ __global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_long(GemvArgs a, i
   }
 }
 
+// K7f (gemv_f16w_rows): few f32 rows, by f32 FMAs on the registers the loads fill.
+//   A launch of this size is a chain of waits with little arithmetic between them,
+//   and what K7m and K7l add to the chain is the staging of x: timed inside the
+//   kernels (5 rows), 1.1 of the 4.6 us of a 1280 x 1280 product went into scaling,
+//   splitting and storing the rows and its barrier, 1 us into the matrix pipe's
+//   serial k steps, and at 5120 columns 1.2 us into each of the five staged batches:
+//   every workgroup stages all rows, 70 instructions a wave for four columns a lane,
+//   for a tile of five features. The products themselves are 25 FMAs a lane and four
+//   columns. So nothing is staged: a wave takes slices of 256 columns, lane l the
+//   columns 4 l .. of each feature (8 bytes) and row (16 bytes), as loaded; both
+//   slices of up to 24 are in flight from the start (kDeep). The sums over lanes are
+//   formed four to a register, those over waves in LDS behind the only barrier. A
+//   fused LayerNorm has wave b form row b's mean and deviation (one more barrier) and
+//   every lane normalize what it holds.
+//   FMAs and the LayerNorm are repeated per tile of T features and row, so rows and
+//   features set where the matrix pipe wins. us, K7f / before (K7 for 1-2 rows, K7l
+//   for 5120 columns, else K7m), 1, 2, 3, 5 and 8 rows:
+//     1280 -> 1280       3.1/3.3  3.3/4.4  3.6/4.4  4.0/4.7  4.7/4.7
+//     1280 -> 3 x 1280, LN  4.9/7.5  5.4/10.1  6.0/8.0  7.8/8.8  11.4/9.0
+//     1280 -> 5120, LN   5.8/7.6  6.5/8.7  7.2/8.3  9.2/9.0  13.6/9.2
+//     768 -> 3 x 768, LN  3.9/5.7  4.3/7.3  4.2/5.9  5.1/6.5  6.2/6.7
+//     768 -> 3072, LN    4.3/5.2  4.8/6.2  5.0/5.4  6.1/5.7  9.1/5.6
+//     512 -> 3 x 512, LN (3, 5, 8 rows)  4.1/5.4  5.1/5.7  7.8/6.0
+//     5120 -> 1280       5.5/6.5  5.7/9.6  6.4/9.8  7.0/11.0  8.4/12.1
+//     5120 -> 2560 (3, 5, 8 rows)  8.5/10.9  12.4/12.7  15.1/13.9
+//     5120 -> 5120 (3, 5, 8 rows)  17.3/16.0  22.2/19.1  28.0/21.2
+//     1280 -> 51866, LN  27.7/32.4  32.8/34.2  44.9/32.2  62.9/33.1  -
+//   Error against 64 bits 0.6 to 0.95 of theirs.
+constexpr int gf_rows(int n_tokens) { return n_tokens <= 2 ? 8 : 5; }  // features of a workgroup
+constexpr int kGfWaves = 12;  // waves of a workgroup, at most
+
+template <int NT, int kGfRows, bool kLn, bool kDeep>
+__global__ __launch_bounds__(64 * kGfWaves) void gemv_f16w_rows(GemvArgs a, int T, int n_kw,
+                                                                DType out_dt) {
+  __shared__ float part[kGfWaves][kGfRows * NT + 3];
+  __shared__ float row_mean[NT], row_inv[NT];
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = blockIdx.y;
+  const int n_in = a.n_in, n_out = a.n_out;
+  const int n_slices = (n_in + 255) >> 8;
+  const int row0 = blockIdx.x * T;
+  const _Float16* w = a.w[grp];
+  const float* x = static_cast<const float*>(a.x);
+  const float* bias = a.bias[grp];
+  void* out = a.out[grp];
+
+  struct Slice {
+    f32x4 x[NT], g, b;
+    u32x2 w[kGfRows];
+  };
+  // Slice s of the rows: columns 256 s + 4 lane .. (the last ones again past the end).
+  auto load = [&](int s, Slice& v) __attribute__((always_inline)) {
+    const int k = min(256 * s + 4 * lane, n_in - 4);
+#pragma unroll
+    for (int b = 0; b < NT; ++b)
+      v.x[b] = *reinterpret_cast<const f32x4*>(x + static_cast<int64_t>(b) * a.x_rs + k);
+    if constexpr (kLn) {
+      v.g = *reinterpret_cast<const f32x4*>(a.ln_g + k);
+      v.b = *reinterpret_cast<const f32x4*>(a.ln_b + k);
+    }
+#pragma unroll
+    for (int i = 0; i < kGfRows; ++i) {
+      const int r = min(row0 + min(i, T - 1), n_out - 1);
+      v.w[i] = *reinterpret_cast<const u32x2*>(w + static_cast<int64_t>(r) * n_in + k);
+    }
+  };
+
+  Slice va, vb;
+  f32x4 xv[kLnCache], none[kLnCache];
+  const float* xr = x + static_cast<int64_t>(min(wave, NT - 1)) * a.x_rs;
+  const bool reg_row = n_in <= 256 * kLnCache;
+  if constexpr (kLn) {
+    if (wave < NT && reg_row) ln_row_load(xr, nullptr, nullptr, n_in, xv, none, none);
+  }
+  load(wave, va);
+  if constexpr (kDeep) load(wave + n_kw, vb);
+  const int f_row = row0 + tid / NT, f_b = tid % NT;  // the output of thread tid < T * NT
+  float bias_v = 0.f;
+  if (bias && tid < kGfRows * NT) bias_v = bias[min(f_row, n_out - 1)];
+
+  float mean[NT], inv[NT];
+  if constexpr (kLn) {
+    if (wave < NT) {
+      float m, iv;
+      if (reg_row)
+        ln_reg_stats(n_in, a.ln_eps, xv, m, iv);
+      else
+        ln_row_stats(xr, n_in, a.ln_eps, m, iv);
+      if (lane == 0) {
+        row_mean[wave] = m;
+        row_inv[wave] = iv;
+      }
+    }
+    // LDS only: the loads stay in flight.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int b = 0; b < NT; ++b) {
+      mean[b] = row_mean[b];
+      inv[b] = row_inv[b];
+    }
+  }
+
+  float acc[kGfRows * NT + 3];
+#pragma unroll
+  for (int i = 0; i < kGfRows * NT + 3; ++i) acc[i] = 0.f;
+  auto add = [&](int s, Slice& v) __attribute__((always_inline)) {
+    if constexpr (kLn) {
+#pragma unroll
+      for (int b = 0; b < NT; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          v.x[b][j] = fmaf((v.x[b][j] - mean[b]) * inv[b], v.g[j], v.b[j]);
+    }
+    if (256 * s + 4 * lane >= n_in) {  // both: an infinite weight times 0 is not 0
+#pragma unroll
+      for (int b = 0; b < NT; ++b) v.x[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < kGfRows; ++i) v.w[i] = u32x2{0, 0};
+    }
+#pragma unroll
+    for (int i = 0; i < kGfRows; ++i) {
+      if (i >= T) break;  // uniform
+      const h16x4 h = __builtin_bit_cast(h16x4, v.w[i]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float wf = static_cast<float>(h[j]);
+#pragma unroll
+        for (int b = 0; b < NT; ++b) acc[i * NT + b] = fmaf(wf, v.x[b][j], acc[i * NT + b]);
+      }
+    }
+  };
+  if (wave < n_kw) {
+    if constexpr (kDeep) {
+      for (int s = wave; s < n_slices; s += 2 * n_kw) {
+        add(s, va);
+        if (s + 2 * n_kw < n_slices) load(s + 2 * n_kw, va);
+        if (s + n_kw < n_slices) add(s + n_kw, vb);
+        if (s + 3 * n_kw < n_slices) load(s + 3 * n_kw, vb);
+      }
+    } else {
+      add(wave, va);
+    }
+    // Sums over the 64 lanes, four to a register: two swaps leave each row of 16
+    // lanes with one of four sums, which its lanes then add up.
+    constexpr int R = (kGfRows * NT + 3) / 4;
+    float mine = 0.f;
+#pragma unroll
+    for (int j = 0; j < R; ++j) {
+      swap32(acc[4 * j], acc[4 * j + 1]);
+      swap32(acc[4 * j + 2], acc[4 * j + 3]);
+      float p = acc[4 * j] + acc[4 * j + 1], q = acc[4 * j + 2] + acc[4 * j + 3];
+      swap16(p, q);
+      float v = p + q;
+      v += dpp<0x128>(v);
+      v += dpp<0x124>(v);
+      v += dpp<0x122>(v);
+      v += dpp<0x121>(v);
+      if ((lane & 15) == j) mine = v;
+    }
+    const int o = 4 * (lane & 15) + ((lane >> 5) & 1) + 2 * ((lane >> 4) & 1);
+    if (o < kGfRows * NT) part[wave][o] = mine;
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  if (tid < T * NT && f_row < n_out) {
+    float v = 0.f;
+    for (int i = 0; i < n_kw; ++i) v += part[i][tid];
+    if (bias) v += bias_v;
+    if (a.act == kActGelu) v = gelu_tanh(v);
+    const int64_t o = static_cast<int64_t>(f_b) * a.out_rs +
+                      static_cast<int64_t>(f_row >> 6) * a.out_hs + (f_row & 63);
+    if (out_dt == kF32)
+      static_cast<float*>(out)[o] = v;
+    else if (out_dt == kF16)
+      static_cast<_Float16*>(out)[o] = static_cast<_Float16>(v);
+    else
+      static_cast<__bf16*>(out)[o] = static_cast<__bf16>(v);
+  }
+}
+
 // f32 rows -> [hi | lo] f16 rows of 2 n_in, plus each row's 2^-shift; with
 // kLn the rows are normalized first (norm.rs:116-143, the layer_norm_rows
 // arithmetic exactly). One wave per row. Bound by memory (4 bytes in, 4 out a
@@ -1237,6 +1380,23 @@ hipError_t launch_linear_split(const float* x, int64_t x_rs, int n_tokens, int n
   return hipGetLastError();
 }
 
+namespace {
+
+// Which f32 products run on K7f (see there for both sides measured). Nothing but
+// the shape of one weight group decides, so that a group of a call and a call of
+// its own, and the fused and the separate LayerNorm and GELU, agree bit for bit.
+bool gemv_by_fma(int n_tokens, int n_in, int n_out) {
+  if (n_tokens <= 2) return true;
+  // Short rows, against K7m: 3 rows up to 5120 features, 4 up to 2880, 5 up to 1843.
+  // Six and more lose where a call has three groups of 512, 1024 or 1280.
+  if (n_in <= 256 * kLnCache)
+    return n_tokens <= 5 && static_cast<int64_t>(n_tokens) * n_tokens * n_out <= 9 * 5120;
+  // Long rows, against K7l: 3 rows up to 3413 features, 5 up to 2048, 8 up to 1280.
+  return static_cast<int64_t>(n_tokens) * n_out <= 10240;
+}
+
+}  // namespace
+
 hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s) {
   if (a.n_tokens <= 0 || a.n_out <= 0 || a.n_groups <= 0) return hipSuccess;
   if (a.n_tokens > kGemvMaxRows) return hipErrorInvalidValue;
@@ -1244,8 +1404,44 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
   const int n_cu = linear_cus();
   int dev = 0;
   (void)hipGetDevice(&dev);
-  // Three or more x rows: the matrix-pipe kernels (one or two rows read the
-  // staged x cheaply enough that the FMA kernel's wider spread wins).
+  // T features a workgroup: the CU's share, or an even part of it when that is more
+  // than a workgroup takes.
+  if (x_dt == kF32 && gemv_by_fma(a.n_tokens, a.n_in, a.n_out)) {
+    const int n_slices = (a.n_in + 255) / 256;
+    const int rounds = (n_slices + kGfWaves - 1) / kGfWaves;
+    const int n_kw = (n_slices + rounds - 1) / rounds;
+    const int waves = a.ln_g ? std::max(n_kw, a.n_tokens) : n_kw;
+    const int64_t rows = static_cast<int64_t>(a.n_out) * a.n_groups;
+    const int64_t share = std::max<int64_t>(1, (rows + n_cu - 1) / n_cu);
+    const int64_t per_cu = (share + gf_rows(a.n_tokens) - 1) / gf_rows(a.n_tokens);
+    const int T = static_cast<int>((share + per_cu - 1) / per_cu);
+    const dim3 fgrid((a.n_out + T - 1) / T, a.n_groups), fblock(64 * waves);
+#define WRS_GF_L(KERNEL)                                                           \
+  {                                                                                \
+    hipLaunchKernelGGL((KERNEL), fgrid, fblock, 0, s, a, T, n_kw, out_dt);         \
+    return hipGetLastError();                                                      \
+  }
+#define WRS_GF_K(NT, R)                                                            \
+  {                                                                                \
+    if (rounds > 1 && a.ln_g) WRS_GF_L((gemv_f16w_rows<NT, R, true, true>))        \
+    if (rounds > 1) WRS_GF_L((gemv_f16w_rows<NT, R, false, true>))                 \
+    if (a.ln_g) WRS_GF_L((gemv_f16w_rows<NT, R, true, false>))                     \
+    WRS_GF_L((gemv_f16w_rows<NT, R, false, false>))                                \
+  }
+    switch (a.n_tokens) {
+      case 1: if (T > 5) WRS_GF_K(1, 8) else WRS_GF_K(1, 5)
+      case 2: if (T > 5) WRS_GF_K(2, 8) else WRS_GF_K(2, 5)
+      case 3: WRS_GF_K(3, 5)
+      case 4: WRS_GF_K(4, 5)
+      case 5: WRS_GF_K(5, 5)
+      case 6: WRS_GF_K(6, 5)
+      case 7: WRS_GF_K(7, 5)
+      case 8: WRS_GF_K(8, 5)
+    }
+#undef WRS_GF_K
+#undef WRS_GF_L
+  }
+  // Three or more rows: the matrix-pipe kernels.
   const size_t gm_lds = static_cast<size_t>(x_dt == kF32 ? 2 : 1) * a.n_tokens * (a.n_in + 8) * 2;
   const bool long_rows = x_dt == kF32 && a.n_in > 256 * kLnCache;
   if (a.n_tokens >= 3 && (long_rows || (gm_lds <= kGmMaxDynLds && (x_dt == kF32 || x_dt == kF16)))) {
@@ -1298,50 +1494,31 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
 #undef WRS_GM
 #undef WRS_GM_K
   }
-  // Up to kGemvSmallOut features: one feature per wave, so that the matrix
-  // spreads over ~n_out / 8 CUs; beyond it 4 features per wave share each
-  // staged x read.
+  // What is left: one or two f16 rows. Up to kGemvSmallOut features: one feature
+  // per wave, so that the matrix spreads over ~n_out / 8 CUs; beyond it 4 features
+  // per wave share each staged x read.
+  if (x_dt != kF16 || a.n_tokens > 2) return hipErrorInvalidValue;
   const int rpw = a.n_out <= kGemvSmallOut ? 1 : 4;
   const int groups = (a.n_out + rpw - 1) / rpw;
   const int wgs = std::min(n_cu, (groups + kGemvWaves - 1) / kGemvWaves);
   dim3 grid(std::max(wgs, 1), a.n_groups);
   dim3 block(64 * kGemvWaves);
-#define WRS_GEMV_R(R, XT, OT)                                                           \
-  switch (a.n_tokens) {                                                                 \
-    case 1: hipLaunchKernelGGL((gemv_f16w<1, R, XT, OT>), grid, block, 0, s, a); break;  \
-    case 2: hipLaunchKernelGGL((gemv_f16w<2, R, XT, OT>), grid, block, 0, s, a); break;  \
-    case 3: hipLaunchKernelGGL((gemv_f16w<3, R, XT, OT>), grid, block, 0, s, a); break;  \
-    case 4: hipLaunchKernelGGL((gemv_f16w<4, R, XT, OT>), grid, block, 0, s, a); break;  \
-    case 5: hipLaunchKernelGGL((gemv_f16w<5, R, XT, OT>), grid, block, 0, s, a); break;  \
-    case 6: hipLaunchKernelGGL((gemv_f16w<6, R, XT, OT>), grid, block, 0, s, a); break;  \
-    case 7: hipLaunchKernelGGL((gemv_f16w<7, R, XT, OT>), grid, block, 0, s, a); break;  \
-    default: hipLaunchKernelGGL((gemv_f16w<8, R, XT, OT>), grid, block, 0, s, a); break; \
-  }
-#define WRS_GEMV(XT, OT)          \
-  if (rpw == 1) {                 \
-    WRS_GEMV_R(1, XT, OT)         \
-  } else {                        \
-    WRS_GEMV_R(4, XT, OT)         \
-  }
-  if (x_dt == kF32) {
-    switch (out_dt) {
-      case kF32: WRS_GEMV(float, float); break;
-      case kF16: WRS_GEMV(float, _Float16); break;
-      case kBF16: WRS_GEMV(float, __bf16); break;
-      default: return hipErrorInvalidValue;
-    }
-  } else if (x_dt == kF16) {
-    switch (out_dt) {
-      case kF32: WRS_GEMV(_Float16, float); break;
-      case kF16: WRS_GEMV(_Float16, _Float16); break;
-      case kBF16: WRS_GEMV(_Float16, __bf16); break;
-      default: return hipErrorInvalidValue;
-    }
-  } else {
-    return hipErrorInvalidValue;
+#define WRS_GEMV(OT)                                                                       \
+  if (rpw == 1 && a.n_tokens == 1)                                                         \
+    hipLaunchKernelGGL((gemv_f16w<1, 1, OT>), grid, block, 0, s, a);                       \
+  else if (rpw == 1)                                                                       \
+    hipLaunchKernelGGL((gemv_f16w<2, 1, OT>), grid, block, 0, s, a);                       \
+  else if (a.n_tokens == 1)                                                                \
+    hipLaunchKernelGGL((gemv_f16w<1, 4, OT>), grid, block, 0, s, a);                       \
+  else                                                                                     \
+    hipLaunchKernelGGL((gemv_f16w<2, 4, OT>), grid, block, 0, s, a);
+  switch (out_dt) {
+    case kF32: WRS_GEMV(float) break;
+    case kF16: WRS_GEMV(_Float16) break;
+    case kBF16: WRS_GEMV(__bf16) break;
+    default: return hipErrorInvalidValue;
   }
 #undef WRS_GEMV
-#undef WRS_GEMV_R
   return hipGetLastError();
 }
 
