@@ -870,9 +870,9 @@ __global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_mfma(GemvArgs a, i
 //   MFMAs start from zero and are scaled back (exact) as they are added up. No
 //   barrier stands before the products and the next batch of W and x is in
 //   flight meanwhile. Rows staged whole by one wave each, in two passes, had cost
-//   most of the launch, and eight rows of 5120 did not fit the LDS: 5 rows,
-//   5120 -> 1280 12.2 -> 11.2 us, 8 rows 28.4 -> 12.4 us (FMA kernel before), 5
-//   rows 3072 -> 768 8.6 -> 7.4 us.
+//   most of the launch, and eight rows of 5120 did not fit the LDS: 12.2 -> 11.2 us
+//   for 5 rows of 5120 -> 1280, a size that K7f now takes; here 5 rows of 5120 ->
+//   5120 take 19.1 us.
 //   A fused LayerNorm takes one barrier: wave b forms row b's mean and deviation.
 constexpr int kGlKB = 4;                       // k-steps per wave per batch: 128 columns
 constexpr int kGlPitch = 32 * kGlKB + 8;       // f16 elements of a staged row
