@@ -593,3 +593,28 @@ def test_decode_rows_by_fma(wrs, ctx, n_tokens, n_in, n_out):
         wrs.linear(dev(x), torch.from_numpy(w).cuda(), bd, out, ctx=ctx)
         assert torch.equal(got[:-1, 1:], out[:-1, 1:])
         assert not torch.isfinite(got[-1]).any() and not torch.isfinite(got[:, 0]).any()
+
+
+@pytest.mark.parametrize("n_tokens,n_in,n_out,n_groups", [
+    (9, 1536, 384, 1), (70, 1536, 132, 3), (200, 5120, 1280, 1),  # one k range, long ring
+    (37, 2048, 68, 1), (64, 5120, 260, 1),                        # split k, long ring
+    (37, 5120, 1280, 3),                                          # split k, more than the CUs
+])
+def test_linear_long_rows_few_tiles(wrs, ctx, n_tokens, n_in, n_out, n_groups):
+    """f32 rows over long k on grids of at most one workgroup per CU, and just
+    past it: every group against exact arithmetic, and a second call's bits."""
+    note(f"linear long rows T={n_tokens} K={n_in} N={n_out} G={n_groups}")
+    rng = np.random.default_rng(n_tokens + n_in + n_out)
+    x = rng.standard_normal((n_tokens, n_in)).astype(np.float32)
+    ws = [_weights(n_out, n_in, 900 + g) for g in range(n_groups)]
+    b = rng.standard_normal(n_out).astype(np.float32)
+    xd, bd = dev(x), dev(b)
+    wd = [torch.from_numpy(w).cuda() for w in ws]
+    outs = [torch.full((n_tokens, n_out), float("nan"), device="cuda") for _ in ws]
+    again = [torch.full((n_tokens, n_out), float("nan"), device="cuda") for _ in ws]
+    wrs.linear_group(xd, wd, [bd] * n_groups, outs, ctx=ctx)
+    wrs.linear_group(xd, wd, [bd] * n_groups, again, ctx=ctx)
+    for w, o, o2 in zip(ws, outs, again):
+        bound = _gamma_bound(x, w) + 2.0 ** -23 * np.abs(b)
+        assert (np.abs(host(o) - _exact(x, w, b)) <= bound).all()
+        assert torch.equal(o, o2)

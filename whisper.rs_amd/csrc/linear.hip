@@ -1576,6 +1576,16 @@ int cheapest(const LinearArgs& a, const TileCost (&t)[N]) {
 template <typename OutT>
 hipError_t launch_parts(const LinearArgs& a, int splits, hipStream_t s) {
   if (a.parts == 2) {
+    // Long k on at most one workgroup per CU: nothing but the ring hides a stage's
+    // way from memory, so it takes the whole LDS (weights not in any cache, us, 6
+    // stages / 3: 37 x 5120 -> 1280 17.4/18.1, 200 x 5120 -> 1280 34.4/41.6, 37 x
+    // 1536 -> 384 12.8/13.5). Up to 1280 k the longer fill costs what it gains (64 x
+    // 384 -> 384 7.3/7.0, 64 x 1280 -> 1280 12.8/12.7), with one part too.
+    const auto deep = [&](int ft, int n) {
+      return a.n_in >= 1536 && n_tiles(a, ft, 64) * n * a.n_groups <= linear_cus();
+    };
+    if (splits > 1 && deep(32, splits))
+      return launch_tile<OutT, LinTile<32, 64, 32, 32, 64, 6, 2>>(a, splits, s);
     if (splits > 1) return launch_tile<OutT, LinTile<32, 64, 32, 32, 64, 3, 2>>(a, splits, s);
     static constexpr TileCost kCosts[] = {{64, 64, 6.f, 9.3f, 0.f},
                                           {128, 64, 10.f, 13.f, 0.f},
@@ -1583,7 +1593,9 @@ hipError_t launch_parts(const LinearArgs& a, int splits, hipStream_t s) {
                                           {256, 128, 18.f, 36.f, 0.f},
                                           {256, 256, 0.f, 42.f, 0.14f}};
     switch (cheapest(a, kCosts)) {
-      case 0: return launch_tile<OutT, LinTile<64, 64, 32, 32, 64, 3, 2>>(a, 1, s);
+      case 0:
+        if (deep(64, 1)) return launch_tile<OutT, LinTile<64, 64, 32, 32, 64, 6, 2>>(a, 1, s);
+        return launch_tile<OutT, LinTile<64, 64, 32, 32, 64, 3, 2>>(a, 1, s);
       case 1: return launch_tile<OutT, LinTile<128, 64, 64, 32, 64, 4, 2>>(a, 1, s);
       case 2: return launch_tile<OutT, LinTile<128, 64, 64, 32, 64, 2, 2>>(a, 1, s);
       case 3: return launch_tile<OutT, LinTile<256, 128, 128, 64, 32, 2, 2>>(a, 1, s);
