@@ -251,3 +251,78 @@ def test_f32_workgroup_split_under_graph_capture(wrs, fresh_ctx):
         run()
         torch.cuda.synchronize()
         assert torch.equal(out, ref), f"eager call after replay {rep} differs"
+
+
+def _capture(ctx, fn):
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        ctx.use_torch_stream()
+        fn()
+    ctx.use_torch_stream()
+    return g
+
+
+@pytest.mark.parametrize("call,rows,n_in", [
+    (call, rows, n_in) for call in ("linear", "group", "fused", "cross_proj")
+    for rows, n_in in ((9, 64), (37, 1280), (37, 5120), (448, 1280))
+    if call != "cross_proj" or n_in <= 1280])
+def test_reserved_projection_allows_graph_capture(wrs, fresh_ctx, call, rows, n_in):
+    # A context that has reserved the rows records their projection as its first
+    # call: the split rows (and the k split's partials) fit what was reserved.
+    note(f"reserve + graph capture of {call} rows={rows} n_in={n_in}")
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + n_in)
+    n_out = n_in if call == "cross_proj" else 128
+    x = torch.randn((rows, n_in), generator=gen, device="cuda")
+    ws = [(torch.randn((n_out, n_in), generator=gen, device="cuda") / n_in ** 0.5).half()
+          for _ in range(2)]
+    bs = [torch.randn(n_out, generator=gen, device="cuda") for _ in range(2)]
+    ln = (torch.rand(n_in, generator=gen, device="cuda"),
+          torch.randn(n_in, generator=gen, device="cuda"), 1e-5)
+    out = torch.zeros((2, rows, n_out), device="cuda")
+    q = torch.randn((1, n_out), generator=gen, device="cuda")
+
+    def setup(ctx):
+        arena = None
+        if call == "cross_proj":
+            arena = wrs.KvArena(1, 1, n_in // 64, 4, rows, ctx=ctx)
+
+        def run():
+            if call == "linear":
+                wrs.linear(x, ws[0], bs[0], out[0], ctx=ctx)
+            elif call == "group":
+                wrs.linear_group(x, ws, bs, [out[0], out[1]], ctx=ctx)
+            elif call == "fused":
+                wrs.linear_fused(x, ws, bs, [out[0], out[1]], ln=ln, act="gelu", ctx=ctx)
+            else:
+                arena.set_cross_proj(x, [ws[0]], [ws[1]], [bs[1]])
+                arena.decode_cross(0, q, out[0, :1])
+        return run, arena
+
+    other = wrs.Context(0)
+    other.use_torch_stream()
+    run, arena = setup(other)
+    run()
+    torch.cuda.synchronize()
+    ref = out.clone()
+    assert torch.isfinite(ref).all()
+    if arena is not None:
+        arena.close()
+    other.close()
+    ctx = fresh_ctx
+    ctx.reserve(linear_tokens=rows, linear_n_in=n_in, n_heads=n_in // 64, decode_rows=1,
+                decode_keys=rows)
+    run, arena = setup(ctx)
+    out.zero_()
+    g = _capture(ctx, run)
+    for rep in range(3):
+        out.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), f"replay {rep}"
+        out.zero_()
+        run()  # eager work between replays
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), f"eager call after replay {rep}"
+    if arena is not None:
+        arena.close()

@@ -135,16 +135,17 @@ bool capturing(wrs_attn_ctx* c) {
   return hipStreamIsCapturing(c->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
-// Grows a scratch buffer to at least `bytes`. Refused while the stream is
-// capturing (a captured graph would keep the old pointer, and hipMalloc /
-// hipFree cannot be recorded): size scratch with wrs_attn_reserve first.
-// `zero` clears the new buffer with a fill kernel (never a memset node).
-int grow(wrs_attn_ctx* c, void** p, size_t* cap, size_t bytes, bool zero) {
+// Grows a scratch buffer that holds fewer than `bytes`, to `room` bytes if that
+// is more. Refused while the stream is capturing (a captured graph would keep
+// the old pointer, and hipMalloc / hipFree cannot be recorded): size scratch
+// with wrs_attn_reserve first. `zero` clears the new buffer with a fill kernel
+// (never a memset node).
+int grow(wrs_attn_ctx* c, void** p, size_t* cap, size_t bytes, bool zero, size_t room = 0) {
   if (*cap >= bytes) return WRS_OK;
   if (capturing(c))
     return fail(c, WRS_ECAPTURE,
                 "context scratch would grow during stream capture: call wrs_attn_reserve first");
-  size_t want = std::max(bytes, *cap * 2);
+  size_t want = std::max({bytes, room, *cap * 2});
   if (*p) {
     // The buffer may still be read by work queued on the stream.
     WRS_HIP(c, hipStreamSynchronize(c->stream));
@@ -1492,9 +1493,10 @@ int wrs_attn_capture_cross_heads_lse(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, 
 
 namespace {
 
-// A new context's split-row scratch: one encoder window of the widest rows
-// (1500 x 5120 in two f16 parts), so that a model's first pass allocates once
-// and does not grow it (a hipFree and hipMalloc pair: ~300 us).
+// Split-row scratch that a call allocates holds one encoder window of the widest
+// rows (1500 x 5120 in two f16 parts), so that a model's first pass allocates
+// once (a hipFree and hipMalloc pair: ~300 us). A call that fits a smaller
+// reserved buffer keeps that.
 constexpr size_t kMinSplitRowsBytes = size_t{32} << 20;
 
 // Shared front half of the projection entry points: validates x and the
@@ -1531,8 +1533,8 @@ int linear_prepare(wrs_attn_ctx* c, int x_dtype, const void* x, int64_t x_rs, si
   }
   if (x_dtype != WRS_F32) return fail(c, WRS_EUNSUPPORTED, "x must be f32 or f16");
   const size_t split_bytes = align_up(n_tokens * wrs::kSplitParts * static_cast<int64_t>(n_in) * 2, 256);
-  int rc = grow(c, &c->lin_x, &c->lin_x_bytes,
-                std::max(split_bytes + n_tokens * 4, kMinSplitRowsBytes), false);
+  int rc = grow(c, &c->lin_x, &c->lin_x_bytes, split_bytes + n_tokens * 4, false,
+                kMinSplitRowsBytes);
   if (rc) return rc;
   auto* xs = static_cast<_Float16*>(c->lin_x);
   auto* scale = reinterpret_cast<float*>(static_cast<char*>(c->lin_x) + split_bytes);
