@@ -326,3 +326,64 @@ def test_reserved_projection_allows_graph_capture(wrs, fresh_ctx, call, rows, n_
         assert torch.equal(out, ref), f"eager call after replay {rep}"
     if arena is not None:
         arena.close()
+
+
+def _replays_equal(g, out, ref, eager, n=3):
+    """n replays into a cleared `out`, with eager work between them, keep ref's bits."""
+    for rep in range(n):
+        out.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref), f"replay {rep}"
+        eager()
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("f32", [False, True])
+def test_captured_decode_outlives_exact_calls(wrs, fresh_ctx, f32):
+    # A recorded decode keeps its scratch whatever exact (f32) attention its context
+    # runs eagerly afterwards: host slices of any size, and f32 arenas of no more
+    # scores than before in more rows or slots.
+    from wrs_amd import workloads as W
+    note(f"captured decode, exact calls, replays; f32={f32}")
+    ctx = fresh_ctx
+    H, n_audio, beams = 6, 1500, 8
+    dt = wrs.WRS_F32 if f32 else wrs.WRS_F16
+    arena = wrs.KvArena(1, 1, H, 16, n_audio, ctx=ctx, dtype=dt)
+    k, v = (dev(W.normal((n_audio, H * 64), 31 + i, storage="f16")) for i in range(2))
+    arena.set_cross(0, k, v)
+    q = dev(W.normal((beams, H * 64), 33))
+    out = torch.zeros((beams, H * 64), device="cuda")
+    if not f32:
+        ctx.reserve(n_heads=H, decode_rows=beams, decode_keys=n_audio)
+    arena.decode_cross(0, q, out)
+    torch.cuda.synchronize()
+    ref = out.clone()
+    g = _capture(ctx, lambda: arena.decode_cross(0, q, out))
+
+    long = wrs.KvArena(1, 8, H, 704, 0, ctx=ctx, dtype=wrs.WRS_F32)
+    rows = torch.randn((700, H * 64), device="cuda")
+    for slot in range(8):
+        long.append(0, slot, rows, rows)
+        long.advance(slot, 600)
+    o8 = torch.zeros_like(q)
+    prompt = torch.randn((17, H * 64), device="cuda")
+    o17 = torch.zeros_like(prompt)
+    rng = np.random.default_rng(34)
+
+    def exact():
+        long.decode_self(0, list(range(8)), q, o8)  # 8 blocks of rows, 4808 scores a head
+        long.prefill_self(0, 3, prompt, o17)        # 3 blocks, 10489 scores a head
+        for heads, tokens, keys in ((8, 1, 1500), (6, 100, 600), (20, 40, 1500)):
+            d = heads * 64
+            hq, ho = (rng.standard_normal(tokens * d).astype(np.float32) for _ in range(2))
+            hk, hv = (rng.standard_normal(keys * d).astype(np.float32) for _ in range(2))
+            wrs.mha_with_cache(hq, hk, hv, tokens, keys, keys - tokens, heads, d, ho, ctx=ctx)
+        junk = [torch.full((n,), -1, dtype=torch.int32, device="cuda")
+                for n in (1 << 8, 1 << 12, 1 << 16, 1 << 20)]
+        del junk
+
+    exact()
+    _replays_equal(g, out, ref, exact)
+    long.close()
+    arena.close()

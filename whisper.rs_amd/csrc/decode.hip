@@ -477,7 +477,6 @@ __global__ __launch_bounds__(kThreads) void decode_exact_f32(ExactArgs a) {
 // share each chunk read, kExactRows at a time. Bound by memory latency: one
 // thread per key reading its row alone took 52 us a call on average (6 heads,
 // 61 and 1500 keys).
-constexpr int kOneKeys = 512;
 constexpr int kExactChunk = 64;
 constexpr int kExactRows = 8;
 
@@ -911,6 +910,14 @@ ExactScratch decode_exact_scratch(int n_rows, int n_heads, int d_head, int max_k
   }
   return x;
 }
+
+// Bytes that hold the scores, statistics and partials of any launch of up to
+// `scores` scores (rows x heads x longest row): 66 floats a chunk of 64 keys come
+// to at most 1.16 a key past kOneKeys (513 keys: 9 chunks).
+size_t exact_scratch_bytes(size_t scores) { return 9 * scores; }
+// Counters for every launch that fits `bytes` of it: no more blocks of rows than
+// rows, and more than kOneKeys scores a row.
+size_t exact_counter_words(size_t bytes) { return bytes / 9 / (kOneKeys + 1) * kCounterStride; }
 
 hipError_t launch_decode_exact_f32(const ExactArgs& a, hipStream_t s) {
   if (a.n_rows <= 0 || a.n_heads <= 0) return hipSuccess;

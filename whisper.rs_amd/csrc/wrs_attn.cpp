@@ -38,6 +38,8 @@ struct wrs_attn_ctx {
   // Device scratch, grown on demand and kept for the context's lifetime.
   void* stage = nullptr;  // host-slice staging of q/k/v/out and score rows
   size_t stage_bytes = 0;
+  unsigned* stage_counters = nullptr;  // host-slice merge counters (kept zero between launches)
+  size_t stage_counter_bytes = 0;
   float* part = nullptr;  // decode split partials
   size_t part_bytes = 0;
   unsigned* counters = nullptr;  // decode merge counters (kept zero between launches)
@@ -48,8 +50,12 @@ struct wrs_attn_ctx {
   size_t lin_x_bytes = 0;
   float* ln_x = nullptr;  // fused projections of rows too long for the split: normalized rows
   size_t ln_x_bytes = 0;
-  float* exact_scores = nullptr;  // f32 arena attention: full score rows
+  // f32 arena attention: score rows, chunk statistics and partials, and merge
+  // counters (kept zero between launches).
+  float* exact_scores = nullptr;
   size_t exact_scores_bytes = 0;
+  unsigned* exact_counters = nullptr;
+  size_t exact_counter_bytes = 0;
   // 16-bit prefill blocks whose keys split over two workgroups: partials and
   // merge counters (kept zero between launches). Allocated at their first use
   // for at least kSplitScratchBlocks blocks, so that every grid the default
@@ -197,7 +203,7 @@ int run_exact(wrs_attn_ctx* c, const float* q, size_t q_floats, const float* k, 
   const size_t is = st.add(x.scores), it = st.add(x.stats), ip = st.add(x.part);
   int rc = grow(c, &c->stage, &c->stage_bytes, st.total, false);
   if (rc) return rc;
-  rc = grow(c, reinterpret_cast<void**>(&c->counters), &c->counter_bytes,
+  rc = grow(c, reinterpret_cast<void**>(&c->stage_counters), &c->stage_counter_bytes,
             x.counter_words * sizeof(unsigned), true);
   if (rc) return rc;
   float *dq = stage_ptr(c, st, iq), *dk = stage_ptr(c, st, ik), *dv = stage_ptr(c, st, iv);
@@ -230,7 +236,7 @@ int run_exact(wrs_attn_ctx* c, const float* q, size_t q_floats, const float* k, 
   a.n_chunks = x.chunks;
   a.stats = stage_ptr(c, st, it);
   a.part = stage_ptr(c, st, ip);
-  a.counters = c->counters;
+  a.counters = c->stage_counters;
   WRS_HIP(c, wrs::launch_decode_exact_f32(a, c->stream));
   WRS_HIP(c, hipMemcpyAsync(out, dout, out_floats * 4, hipMemcpyDeviceToHost, c->stream));
   WRS_HIP(c, hipStreamSynchronize(c->stream));
@@ -526,12 +532,14 @@ void wrs_attn_destroy(wrs_attn_ctx* c) {
   DeviceGuard g(c->device);
   (void)hipStreamSynchronize(c->stream);
   if (c->stage) (void)hipFree(c->stage);
+  if (c->stage_counters) (void)hipFree(c->stage_counters);
   if (c->part) (void)hipFree(c->part);
   if (c->counters) (void)hipFree(c->counters);
   if (c->cap_part) (void)hipFree(c->cap_part);
   if (c->lin_x) (void)hipFree(c->lin_x);
   if (c->ln_x) (void)hipFree(c->ln_x);
   if (c->exact_scores) (void)hipFree(c->exact_scores);
+  if (c->exact_counters) (void)hipFree(c->exact_counters);
   if (c->split_part) (void)hipFree(c->split_part);
   if (c->split_counters) (void)hipFree(c->split_counters);
   if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
@@ -827,12 +835,20 @@ int exact_arena(wrs_attn_ctx* c, wrs_kv* kv, const float* q, float* out, void* k
   const wrs::ExactScratch x =
       wrs::decode_exact_scratch(n_rows, static_cast<int>(kv->n_heads), 64, max_len,
                                 static_cast<int>(groups), rows_per_group);
-  int rc = grow(c, reinterpret_cast<void**>(&c->exact_scores), &c->exact_scores_bytes,
-                (x.scores + x.stats + x.part) * sizeof(float), false);
-  if (rc) return rc;
-  rc = grow(c, reinterpret_cast<void**>(&c->counters), &c->counter_bytes,
-            x.counter_words * sizeof(unsigned), true);
-  if (rc) return rc;
+  // Sized by the count of scores alone, whatever their split, so that a buffer
+  // which a captured graph holds is outgrown (and freed) only by a call of more
+  // scores than any before it. Calls of up to kOneKeys keys use none of it, and
+  // are recorded whether it exists or not; made eagerly they size it too.
+  const size_t rows_heads = static_cast<size_t>(n_rows) * kv->n_heads;
+  if (x.scores || !capturing(c)) {
+    int rc = grow(c, reinterpret_cast<void**>(&c->exact_scores), &c->exact_scores_bytes,
+                  wrs::exact_scratch_bytes(rows_heads * static_cast<size_t>(max_len)), false,
+                  wrs::exact_scratch_bytes(rows_heads * wrs::kOneKeys));
+    if (rc) return rc;
+    rc = grow(c, reinterpret_cast<void**>(&c->exact_counters), &c->exact_counter_bytes,
+              wrs::exact_counter_words(c->exact_scores_bytes) * sizeof(unsigned), true);
+    if (rc) return rc;
+  }
   wrs::ExactArgs a{};
   a.q = q;
   a.k = static_cast<const float*>(kbase);
@@ -854,7 +870,7 @@ int exact_arena(wrs_attn_ctx* c, wrs_kv* kv, const float* q, float* out, void* k
   a.n_chunks = x.chunks;
   a.stats = c->exact_scores + x.scores;
   a.part = a.stats + x.stats;
-  a.counters = c->counters;
+  a.counters = c->exact_counters;
   for (size_t g = 0; g < groups; ++g) {
     a.goff[g] = goff[g];
     a.glen[g] = glen[g];

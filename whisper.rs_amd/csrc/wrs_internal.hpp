@@ -153,12 +153,15 @@ struct ExactArgs {
   int64_t goff[kMaxExactGroups];
   int glen[kMaxExactGroups];
 };
+constexpr int kOneKeys = 512;  // d_head 64: keys a row that one workgroup takes, without scratch
 struct ExactScratch {
   size_t scores, stats, part, counter_words;  // floats, floats, floats, words
   int chunks;
 };
 ExactScratch decode_exact_scratch(int n_rows, int n_heads, int d_head, int max_keys, int n_groups,
                                   int rows_per_group);
+size_t exact_scratch_bytes(size_t scores);
+size_t exact_counter_words(size_t bytes);
 hipError_t launch_decode_exact_f32(const ExactArgs& a, hipStream_t s);
 
 // Split-K decode over an f16 KV cache: one query row per (group, row),
