@@ -387,3 +387,66 @@ def test_captured_decode_outlives_exact_calls(wrs, fresh_ctx, f32):
     _replays_equal(g, out, ref, exact)
     long.close()
     arena.close()
+
+
+@pytest.mark.parametrize("rows", [9, 15, 17, 23])
+def test_reserved_cross_rows_allow_graph_capture(wrs, fresh_ctx, rows):
+    # Cross-attention rows that are no multiple of a decode group's eight fit the
+    # partials reserved for exactly that many rows.
+    from wrs_amd import workloads as W
+    note(f"reserve + graph capture of {rows} cross rows")
+    ctx = fresh_ctx
+    H, n_audio = 3, 700
+    arena = wrs.KvArena(1, 1, H, 16, n_audio, ctx=ctx)
+    k, v = (W.normal((n_audio, H * 64), 21 + i, storage="f16") for i in range(2))
+    arena.set_cross(0, dev(k), dev(v))
+    q = dev(W.normal((rows, H * 64), 23))
+    out = torch.zeros((rows, H * 64), device="cuda")
+    ctx.reserve(n_heads=H, decode_rows=rows, decode_keys=n_audio)
+    g = _capture(ctx, lambda: arena.prefill_cross(0, q, out))
+    arena.prefill_cross(0, q, out)
+    torch.cuda.synchronize()
+    ref = out.clone()
+    qd, kd, vd = (a.astype(np.float64).reshape(-1, H, 64).transpose(1, 0, 2)
+                  for a in (host(q), k, v))
+    s = qd @ kd.transpose(0, 2, 1) / 8.0
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = ((p / p.sum(-1, keepdims=True)) @ vd).transpose(1, 0, 2).reshape(rows, -1)
+    assert maxerr(host(ref), want) < 1e-5
+    _replays_equal(g, out, ref, lambda: arena.prefill_cross(0, q * 0.5, out))
+    arena.close()
+
+
+@pytest.mark.parametrize("held,rows", [(8, 9), (16, 23), (8, 23)])
+def test_captured_decode_outlives_cross_rows(wrs, fresh_ctx, held, rows):
+    # Scratch that holds a prompt's whole groups of eight rows serves its last rows
+    # too: the call replaces nothing that a recorded decode holds (the first two).
+    # One that needs more than is there (the third) is made before the recording.
+    from wrs_amd import workloads as W
+    note(f"captured decode of {held} rows, {rows} cross rows, replays")
+    ctx = fresh_ctx
+    H, n_audio = 3, 700
+    arena = wrs.KvArena(1, 1, H, 16, n_audio, ctx=ctx)
+    k, v = (W.normal((n_audio, H * 64), 41 + i, storage="f16") for i in range(2))
+    arena.set_cross(0, dev(k), dev(v))
+    q = dev(W.normal((rows, H * 64), 43))
+    out = torch.zeros((held, H * 64), device="cuda")
+    all_rows = torch.zeros((rows, H * 64), device="cuda")
+    ctx.reserve(n_heads=H, decode_rows=held, decode_keys=n_audio)
+    if rows - held >= 8:
+        arena.prefill_cross(0, q, all_rows)
+    arena.prefill_cross(0, q[:held], out)
+    torch.cuda.synchronize()
+    ref = out.clone()
+    g = _capture(ctx, lambda: arena.prefill_cross(0, q[:held], out))
+    _replays_equal(g, out, ref, lambda: arena.prefill_cross(0, q, all_rows))
+    other = wrs.Context(0)  # no scratch yet: all rows in one launch
+    other.use_torch_stream()
+    arena2 = wrs.KvArena(1, 1, H, 16, n_audio, ctx=other)
+    arena2.set_cross(0, dev(k), dev(v))
+    whole = torch.zeros_like(all_rows)
+    arena2.prefill_cross(0, q, whole)
+    assert maxerr(host(whole), host(all_rows)) < 1e-6
+    arena2.close()
+    other.close()
+    arena.close()

@@ -407,6 +407,28 @@ void noalloc_release(wrs_attn_ctx* c) {
   c->noalloc_slot = -1;
 }
 
+// Keys per workgroup of a split-K decode: sequences of 129..256 keys take one
+// 256-key workgroup per (group, head), without partials and merge; longer ones
+// split into 128-key workgroups.
+int decode_chunk(int max_len) {
+  return (max_len > wrs::kDecodeChunk && max_len <= wrs::kDecodeChunkLong) ? wrs::kDecodeChunkLong
+                                                                          : wrs::kDecodeChunk;
+}
+int decode_splits(int max_len) {
+  const int chunk = decode_chunk(max_len);
+  return std::max(1, (max_len + chunk - 1) / chunk);
+}
+
+// True if the context's scratch holds such a decode as it stands.
+bool decode_fits(const wrs_attn_ctx* c, int n_groups, int n_heads, int max_len,
+                 int rows_per_group) {
+  const int splits = decode_splits(max_len);
+  return splits == 1 ||
+         (wrs::decode_part_floats(n_groups, n_heads, splits, rows_per_group) * sizeof(float) <=
+              c->part_bytes &&
+          wrs::decode_counter_words(n_groups, n_heads) * sizeof(unsigned) <= c->counter_bytes);
+}
+
 // Split-K decode over f16 planes. `fixed` (the device address of `scratch`)
 // replaces the context's scratch and is never grown: shapes whose partials or
 // counters do not fit fail with WRS_ERANGE.
@@ -439,12 +461,8 @@ int decode_impl(wrs_attn_ctx* c, const float* q, int64_t q_rs, float* out, int64
   a.rows_per_group = rows_per_group;
   a.n_rows = n_rows;
   a.n_heads = n_heads;
-  // Sequences of 129..256 keys take one 256-key workgroup per (group, head):
-  // no partials and no merge. Longer ones split into 128-key workgroups.
-  a.chunk = (max_len > wrs::kDecodeChunk && max_len <= wrs::kDecodeChunkLong)
-                ? wrs::kDecodeChunkLong
-                : wrs::kDecodeChunk;
-  a.n_splits = std::max(1, (max_len + a.chunk - 1) / a.chunk);
+  a.chunk = decode_chunk(max_len);
+  a.n_splits = decode_splits(max_len);
   a.scale_log2 = 0.125f * 1.4426950408889634f;
   a.lse = lse;
   a.lse_rows = lse_rows;
@@ -650,8 +668,13 @@ int wrs_attn_reserve(wrs_attn_ctx* c, const wrs_reserve* r) {
         r->decode_rows, static_cast<size_t>(wrs::kMaxDecodeGroups) * wrs::kMaxRowsPerGroup));
     const int groups = std::min(rows, wrs::kMaxDecodeGroups);
     const int splits = static_cast<int>((r->decode_keys + wrs::kDecodeChunk - 1) / wrs::kDecodeChunk);
+    // Room for the last group of a prompt's rows, so that it joins the others'
+    // launch (rows of a multiple of kMaxRowsPerGroup).
+    constexpr int kGroup = wrs::kMaxRowsPerGroup;
+    const int whole = rows > kGroup ? (rows + kGroup - 1) / kGroup * kGroup : rows;
     rc = grow(c, reinterpret_cast<void**>(&c->part), &c->part_bytes,
-              wrs::decode_part_floats(rows, heads, splits, 1) * sizeof(float), false);
+              wrs::decode_part_floats(rows, heads, splits, 1) * sizeof(float), false,
+              wrs::decode_part_floats(whole, heads, splits, 1) * sizeof(float));
     if (rc) return rc;
     rc = grow(c, reinterpret_cast<void**>(&c->counters), &c->counter_bytes,
               wrs::decode_counter_words(groups, heads) * sizeof(unsigned), true);
@@ -1270,6 +1293,8 @@ int rows_impl(wrs_attn_ctx* c, wrs_kv* kv, const float* q, size_t n, float* out,
 // decode groups hold run on K10; up to that, and planes past its 32-bit offsets,
 // on the split-K decode kernel: groups of kMaxRowsPerGroup rows (the last may
 // hold fewer) share each read of the plane, up to kMaxDecodeGroups per launch.
+// Partials are laid out by whole groups; where the scratch holds the full groups'
+// but not the last one's, its rows go in a launch of their own.
 // With lse, the rows' statistics too ([head][n][2], exp2 domain).
 int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, size_t n,
                     float* out, float* lse) {
@@ -1311,15 +1336,21 @@ int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, s
                      kv->n_audio_max * 64, L, false, 0, lse);
   const int rpg = static_cast<int>(std::min<size_t>(n, wrs::kMaxRowsPerGroup));
   const size_t per_launch = static_cast<size_t>(wrs::kMaxDecodeGroups) * rpg;
-  for (size_t r0 = 0; r0 < n; r0 += per_launch) {
-    const size_t rows = std::min(per_launch, n - r0), groups = (rows + rpg - 1) / rpg;
+  for (size_t r0 = 0, rows = 0; r0 < n; r0 += rows) {
+    rows = std::min(per_launch, n - r0);
+    const int full = static_cast<int>(rows / rpg), heads = static_cast<int>(kv->n_heads);
+    const int len = static_cast<int>(L);
+    if (full > 0 && rows % rpg && decode_fits(c, full, heads, len, rpg) &&
+        !decode_fits(c, full + 1, heads, len, rpg))
+      rows = static_cast<size_t>(full) * rpg;
+    const int last = static_cast<int>(std::min<size_t>(rows, rpg));
+    const size_t groups = (rows + last - 1) / last;
     std::vector<int64_t> goff(groups, static_cast<int64_t>(kv->cross_off(layer)));
-    std::vector<int> lens(groups, static_cast<int>(L));
+    std::vector<int> lens(groups, len);
     int rc = decode_impl(c, q + r0 * dm, dm, out + r0 * dm, dm, wrs_kv::u16(kv->k_cross),
                          wrs_kv::u16(kv->v_cross), static_cast<int64_t>(kv->n_audio_max * 64),
-                         goff, lens, rpg, static_cast<int>(rows),
-                         static_cast<int>(kv->n_heads), nullptr, lse, static_cast<int>(n),
-                         static_cast<int>(r0));
+                         goff, lens, last, static_cast<int>(rows), heads, nullptr, lse,
+                         static_cast<int>(n), static_cast<int>(r0));
     if (rc) return rc;
   }
   return WRS_OK;
