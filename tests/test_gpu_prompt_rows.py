@@ -109,3 +109,81 @@ def test_cached_self_rows(wrs, ctx, heads, rows, past):
     assert (np.abs(got[:rows] - ref) <= tol).all()
     assert np.isnan(got[rows]).all()
     arena.close()
+
+
+# Rows whose output lives on weights far below the row's largest: one key, whose V
+# row is zero, scores `octaves` powers of two above the others. Only columns 0 (that
+# key alone) and 1 (the others alone) of K meet q, so a score is one product.
+def _sink(rows, keys, octaves, seed):
+    rng = np.random.default_rng(seed)
+    k = np.zeros((keys, 64), np.float32)
+    k[:, 1] = _f16(rng.uniform(-1, 1, keys))
+    k[0] = 0.0
+    k[0, 0] = 1.0
+    v = _f16(rng.uniform(0.5, 1.5, (keys, 64)))
+    v[0] = 0.0
+    q = np.zeros((rows, 64), np.float32)
+    q[:, 0] = octaves * 8.0 / np.log2(np.e)
+    q[:, 1] = rng.uniform(-8, 8, rows)
+    return q, k, v
+
+
+def _sink_tol(ref, octaves):
+    """Relative error per output: each exponent argument is one product of at most
+    octaves + 2 in magnitude (operand split to 2^-22, scaling and product to 2^-24
+    each, differences of two of them), every weight the other way round to 2^-22,
+    and a mean of positive values, summed in f32 (2^-20)."""
+    arg = 2.0 * (octaves + 2.0) * (2.0 ** -22 + 3.0 * 2.0 ** -24) * np.log(2.0)
+    return np.abs(ref) * (arg + 2.0 ** -20 + 2.0 ** -22)
+
+
+@pytest.mark.parametrize("octaves", [2, 14, 17, 20, 23, 26, 32])
+@pytest.mark.parametrize("keys", [33, 448, 1500])
+def test_cross_rows_keep_small_weights(wrs, ctx, octaves, keys):
+    note(f"cross rows, one key {octaves} octaves up of {keys}")
+    q, k, v = _sink(27, keys, octaves, octaves + keys)
+    arena = wrs.KvArena(1, 1, 1, 16, keys, ctx=ctx)
+    arena.set_cross(0, k, v)
+    out = torch.zeros((27, 64), device="cuda")
+    ref, _, _ = _attend(q, k, v, 1)
+    arena.prefill_cross(0, dev(q), out)
+    assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves)).all()
+    arena.close()
+
+
+@pytest.mark.parametrize("octaves", [2, 14, 17, 20, 23, 26, 32])
+@pytest.mark.parametrize("rows,past", [(2, 31), (33, 415), (40, 1900)])
+def test_cached_self_rows_keep_small_weights(wrs, ctx, octaves, rows, past):
+    note(f"self rows, one key {octaves} octaves up of {past + rows}")
+    n = past + rows
+    q, k, v = _sink(rows, n, octaves, octaves + n)
+    arena = wrs.KvArena(1, 1, 1, n, 0, ctx=ctx)
+    arena.append(0, 0, k[:past], v[:past])
+    arena.advance(0, past)
+    arena.append(0, 0, np.ascontiguousarray(k[past:]), np.ascontiguousarray(v[past:]))
+    out = torch.zeros((rows, 64), device="cuda")
+    ref, _, _ = _attend(q, k, v, 1, past)
+    arena.prefill_self(0, 0, dev(q), out)
+    assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves)).all()
+    arena.close()
+
+
+@pytest.mark.parametrize("rows,past", [(2, 31), (33, 415)])
+def test_cached_self_rows_keep_small_queries(wrs, ctx, rows, past):
+    # A query column far above the others that no key answers: the others decide.
+    note(f"self rows, one dead query column, {past + rows} keys")
+    rng = np.random.default_rng(past)
+    n = past + rows
+    k, v = (_f16(rng.standard_normal((n, 64))) for _ in range(2))
+    k[:, 5] = 0.0
+    q = rng.standard_normal((rows, 64)).astype(np.float32)
+    arena = wrs.KvArena(1, 1, 1, n, 0, ctx=ctx)
+    arena.append(0, 0, k, v)
+    arena.advance(0, past)
+    out = torch.zeros((rows, 64), device="cuda")
+    ref, _, _ = _attend(q, k, v, 1, past)
+    tol = _bound(q, k, v, 1)
+    q[:, 5] = 2.0 ** 30
+    arena.prefill_self(0, 0, dev(q), out)
+    assert (np.abs(host(out) - ref) <= tol).all()
+    arena.close()

@@ -11,9 +11,14 @@
 //   The arithmetic runs on the f16 matrix pipe with split operands: each query
 //   row, times scale * log2(e) and a power of two that puts its largest element
 //   into [2^14, 2^15), is split into kParts f16 parts, and so are the softmax
-//   weights. Two parts (cross-attention) carry ~2^-22 relative error, as the
-//   split-K decode does; three (the cached self-attention, whose rows the f32
-//   kernel ran before) hold all 24 bits, so that only f32 accumulation rounds.
+//   weights in units of 2^-15. Each part stands in units of its own, 2^-11 of the
+//   one before, and has its own accumulator (f16 ends at 2^-24: in one unit, what
+//   the last part could hold of a weight shrank with the weight). Two parts
+//   (cross-attention) carry 2^-22 of every query element within 2^-28 of its row's
+//   largest and of every weight within 2^-29 of the wave's largest so far, and
+//   to 2^-50 of that largest below; three (the cached self-attention, whose rows
+//   the f32 kernel ran before) carry all 24 bits, and to
+//   2^-61 below.
 //   S^T = K Q^T puts one query per lane, and the packed weights are the B operand
 //   of O^T += V^T P^T as they stand; K comes from memory in operand layout, V
 //   passes through a wave's own swizzled LDS rows and is read transposed
@@ -21,10 +26,11 @@
 //   Bound by latency: launch, first loads, then ~1 us a step on few CUs, merge.
 //   Dealing a block's steps over several workgroups that merge through memory
 //   cost as much as it saved (128 rows x 1500 keys: 15.0 us in three).
-//   Measured, 20 heads x 1500 keys: 128 rows 32.3 -> 14.0 us (groups of 8 rows
-//   each read the planes again: 123 MB of L2 reads), 37 rows 17.0 -> 13.6 us
-//   (two launches); 37 cached self rows 14.5 -> 5.2 us (f32 matrix pipe, element
-//   loads).
+//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 16.2 us
+//   (groups of 8 rows each read the planes again: 123 MB of L2 reads), 37 rows 17.1
+//   -> 15.7 (two launches); 37 cached self rows 14.5 -> 5.6 us, 224 rows past 220
+//   37.9 -> 10.2 (f32 matrix pipe, element loads). One accumulator for all parts, all
+//   in the same units, took 14.2, 13.7, 5.3 and 9.1 us, and lost small weights.
 #include "wrs_internal.hpp"
 
 namespace wrs {
@@ -42,6 +48,7 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int kQ = 32;               // query rows per block
 constexpr int kN = 32;               // keys per step
+constexpr float kWeightUp = 0x1p15f;  // softmax weights, at most 1, are split in these units
 constexpr int kPitch = 66;           // LDS pitch (floats) of a merge row
 constexpr int kRawBuffer = 0x00020000;  // buffer resource word 3: raw, 32-bit data format
 
@@ -64,16 +71,31 @@ __device__ inline f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
-// Two floats as kParts packed f16 pairs whose sums are the floats.
+// Two floats of at most 2^15 as kParts packed f16 pairs, part p in units of
+// kPartUnit^p: what a part leaves is at most 2^-11 of the value, so the next one
+// holds 11 bits more at the same magnitude. Two parts carry 22 bits of values from
+// 2^-14 up (f16's normal range), three all 24.
+constexpr float kPartUnit = 0x1p-11f;
 template <int kParts>
 __device__ inline void split2(float x0, float x1, uint32_t (&out)[kParts]) {
+  constexpr float kUp = 1.f / kPartUnit;
 #pragma unroll
   for (int p = 0; p < kParts; ++p) {
     const f16x2 h = {static_cast<_Float16>(x0), static_cast<_Float16>(x1)};
     out[p] = __builtin_bit_cast(uint32_t, h);
-    x0 = __builtin_fmaf(static_cast<float>(h[0]), -1.f, x0);  // one v_fma_mix each
-    x1 = __builtin_fmaf(static_cast<float>(h[1]), -1.f, x1);
+    x0 = __builtin_fmaf(static_cast<float>(h[0]), -kUp, x0 * kUp);  // exact
+    x1 = __builtin_fmaf(static_cast<float>(h[1]), -kUp, x1 * kUp);
   }
+}
+// The sum of products of the parts, smallest first.
+template <int kParts>
+__device__ inline f32x16 join(const f32x16 (&x)[kParts]) {
+  f32x16 s = x[kParts - 1];
+#pragma unroll
+  for (int p = kParts - 2; p >= 0; --p)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(s[i], kPartUnit, x[p][i]);
+  return s;
 }
 __device__ inline void wave_sync() {
   // LDS operations of one wave complete in order: only the compiler must keep it.
@@ -160,14 +182,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
   f32x16 o[2] = {f32x16{}, f32x16{}};
   float m = -INFINITY, l = 0.f;
   for (; step < n_steps; step += kWaves) {
-    // Two chains over d (half the latency and half the roundings of one), the
-    // smallest parts first, so that few of the sums round at full size.
-    f32x16 s2[2] = {f32x16{}, f32x16{}};
+    // One chain over d per part.
+    f32x16 sp[kParts];
 #pragma unroll
-    for (int p = kParts - 1; p >= 0; --p)
+    for (int p = 0; p < kParts; ++p) sp[p] = f32x16{};
 #pragma unroll
-      for (int dk = 0; dk < 4; ++dk) s2[dk & 1] = mfma(kx[dk], qf[p][dk], s2[dk & 1]);
-    f32x16 s = s2[0] + s2[1];
+    for (int dk = 0; dk < 4; ++dk)
+#pragma unroll
+      for (int p = 0; p < kParts; ++p) sp[p] = mfma(kx[dk], qf[p][dk], sp[p]);
+    f32x16 s = join(sp);
     wave_sync();  // the last step's transposed reads are done
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -200,7 +223,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
       const float p1 = __builtin_amdgcn_exp2f(s[i + 1] - m_use);
       ls += p0 + p1;
       uint32_t w[kParts];
-      split2<kParts>(p0, p1, w);
+      split2<kParts>(p0 * kWeightUp, p1 * kWeightUp, w);
 #pragma unroll
       for (int p = 0; p < kParts; ++p) pf[p][i >> 3][(i >> 1) & 3] = w[p];
     }
@@ -218,11 +241,14 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
         }
         va[k2] = u32x4{t[0].x, t[0].y, t[1].x, t[1].y};
       }
-      f32x16 x = {};
+      f32x16 xp[kParts];
 #pragma unroll
-      for (int p = kParts - 1; p >= 0; --p)
+      for (int p = 0; p < kParts; ++p) xp[p] = f32x16{};
 #pragma unroll
-        for (int k2 = 0; k2 < 2; ++k2) x = mfma(va[k2], pf[p][k2], x);
+      for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+        for (int p = 0; p < kParts; ++p) xp[p] = mfma(va[k2], pf[p][k2], xp[p]);
+      const f32x16 x = join(xp);
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[cc][i] = __builtin_fmaf(o[cc][i], alpha, x[i]);
     }
@@ -257,7 +283,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
     for (int e = 0; e < 8; ++e)
       acc[e] = __builtin_fmaf(mo[w][row * kPitch + d0 + e], ew, acc[e]);
   }
-  const float inv = L > 0.f ? 1.f / L : 0.f;
+  const float inv = (L > 0.f ? 1.f / L : 0.f) * (1.f / kWeightUp);
   float* const op = a.o + static_cast<int64_t>(q0 + row) * a.o_rs + h * 64 + d0;
   *reinterpret_cast<f32x4u*>(op) = f32x4{acc[0], acc[1], acc[2], acc[3]} * inv;
   *reinterpret_cast<f32x4u*>(op + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]} * inv;
