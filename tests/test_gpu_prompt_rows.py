@@ -187,3 +187,41 @@ def test_cached_self_rows_keep_small_queries(wrs, ctx, rows, past):
     arena.prefill_self(0, 0, dev(q), out)
     assert (np.abs(host(out) - ref) <= tol).all()
     arena.close()
+
+
+@pytest.mark.parametrize("rows,past", [(2, 0), (33, 3), (40, 1000)])
+def test_cached_self_rows_over_infinite_keys(wrs, ctx, rows, past):
+    # A key value past f16's range is infinite in the cache. Rows whose score for
+    # it is -inf give it no weight, as the f32 arithmetic does; the others are NaN.
+    note(f"self rows, an infinite key value, past={past}")
+    rng = np.random.default_rng(rows)
+    n = past + rows
+    k, v = (_f16(rng.standard_normal((n, 64))) for _ in range(2))
+    q = rng.standard_normal((rows, 64)).astype(np.float32)
+    q[:, 7] = -1.0 - np.abs(q[:, 7])
+    q[-1, 7] = 1.5
+    k[past, 7] = 1e6
+    arena = wrs.KvArena(1, 1, 1, n, 0, ctx=ctx)
+    if past:
+        arena.append(0, 0, k[:past], v[:past])
+        arena.advance(0, past)
+    arena.append(0, 0, np.ascontiguousarray(k[past:]), np.ascontiguousarray(v[past:]))
+    out = torch.zeros((rows, 64), device="cuda")
+    arena.prefill_self(0, 0, dev(q), out)
+    got = host(out)
+    kz = k.copy()
+    kz[past, 7] = 0.0
+    qd, kd, vd = (a.astype(np.float64) for a in (q, kz, v))
+    s = qd @ kd.T / 8.0
+    j, i = np.arange(n)[None, :], np.arange(rows)[:, None]
+    s = np.where((j > past + i) | (j == past), -np.inf, s)
+    m = s.max(-1, keepdims=True)
+    with np.errstate(invalid="ignore"):
+        p = np.where(np.isfinite(m), np.exp(s - m), 0.0)
+        ref = (p @ vd) / p.sum(-1, keepdims=True)
+    seen = np.isfinite(m[:, 0])  # rows with a key besides it
+    seen[-1] = False
+    assert np.isnan(got[-1]).all()
+    tol = _bound(q, kz, v, 1)
+    assert (np.abs(got - ref) <= tol)[seen].all()
+    arena.close()

@@ -31,7 +31,7 @@
 //   -> 15.7 (two launches); 37 cached self rows 14.5 -> 5.6 us, 224 rows past 220
 //   37.9 -> 10.2 (f32 matrix pipe, element loads). One accumulator for all parts, all
 //   in the same units, took 14.2, 13.7, 5.3 and 9.1 us, and lost small weights.
-#include "wrs_internal.hpp"
+#include "prefill_f32_block.hpp"
 
 namespace wrs {
 namespace {
@@ -108,7 +108,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
   __shared__ __attribute__((aligned(128))) char vs[kWaves][kN * 128];
   __shared__ float mo[kWaves][kQ * kPitch];  // a wave's O rows
   __shared__ float ml[kWaves][2][kQ];        // and their max and sum
+  __shared__ int nonfinite;                  // some output of the block is inf or NaN
+  static_assert(sizeof(f32blk::Tiles<2>) <= sizeof(mo), "f32 tiles fit in the merge rows");
 
+  if (threadIdx.x == 0) nonfinite = 0;
   // The blocks of one head, which read the same planes, share an XCD's L2.
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
   const int qblk = lid % n_qblk, h = lid / n_qblk;
@@ -268,29 +271,61 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
   }
   __syncthreads();
   const int row = tid >> 3, d0 = 8 * (tid & 7);
-  if (row >= kQ || q0 + row >= a.n_rows) return;
-  float M = -INFINITY, L = 0.f, acc[8];
+  if (row < kQ && q0 + row < a.n_rows) {
+    float M = -INFINITY, L = 0.f, acc[8];
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) M = fmaxf(M, ml[w][0][row]);
+    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, ml[w][0][row]);
 #pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
 #pragma unroll
-  for (int w = 0; w < kWaves; ++w) {
-    const float mw = ml[w][0][row];
-    const float ew = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
-    L = __builtin_fmaf(ml[w][1][row], ew, L);
+    for (int w = 0; w < kWaves; ++w) {
+      const float mw = ml[w][0][row];
+      const float ew = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - M);
+      L = __builtin_fmaf(ml[w][1][row], ew, L);
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      acc[e] = __builtin_fmaf(mo[w][row * kPitch + d0 + e], ew, acc[e]);
+      for (int e = 0; e < 8; ++e)
+        acc[e] = __builtin_fmaf(mo[w][row * kPitch + d0 + e], ew, acc[e]);
+    }
+    const float inv = (L > 0.f ? 1.f / L : 0.f) * (1.f / kWeightUp);
+    float* const op = a.o + static_cast<int64_t>(q0 + row) * a.o_rs + h * 64 + d0;
+    *reinterpret_cast<f32x4u*>(op) = f32x4{acc[0], acc[1], acc[2], acc[3]} * inv;
+    *reinterpret_cast<f32x4u*>(op + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]} * inv;
+    if (a.lse && d0 == 0) {
+      float* const stat = a.lse + 2 * (static_cast<int64_t>(h) * a.n_rows + q0 + row);
+      stat[0] = M;
+      stat[1] = L;
+    }
+    if constexpr (kParts == 3) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (!__builtin_isfinite(acc[e] * inv)) nonfinite = 1;
+    }
   }
-  const float inv = (L > 0.f ? 1.f / L : 0.f) * (1.f / kWeightUp);
-  float* const op = a.o + static_cast<int64_t>(q0 + row) * a.o_rs + h * 64 + d0;
-  *reinterpret_cast<f32x4u*>(op) = f32x4{acc[0], acc[1], acc[2], acc[3]} * inv;
-  *reinterpret_cast<f32x4u*>(op + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]} * inv;
-  if (a.lse && d0 == 0) {
-    float* const stat = a.lse + 2 * (static_cast<int64_t>(h) * a.n_rows + q0 + row);
-    stat[0] = M;
-    stat[1] = L;
+  if constexpr (kParts == 3) {
+    // An infinite score (a key value past f16's range, an infinite query) gives its
+    // key all of the row's weight or none, but in parts it comes out NaN (infinity
+    // times a part of zero). The block's rows are then formed again with f32
+    // operands, as every cached self row was before this kernel.
+    __syncthreads();
+    if (nonfinite) {
+      PrefillArgs p{};
+      p.q = a.q;
+      p.k = a.k;
+      p.v = a.v;
+      p.o = a.o;
+      p.lq = {0, 64, a.q_rs};
+      p.lk = p.lv = {0, a.kv_hs, 64};
+      p.lo = {0, 64, a.o_rs};
+      p.n_heads = a.n_heads;
+      p.t_q = min(q0 + kQ, a.n_rows);  // the extra waves share the tiles and store nothing
+      p.t_kv = a.n_keys;
+      p.d_head = 64;
+      p.causal = 1;
+      p.q_pos_offset = a.pos0;
+      p.scale = 0.125f;
+      f32blk::fa2_block<float, _Float16, 2, kWaves>(
+          p, q0, h, 0, *reinterpret_cast<f32blk::Tiles<2>*>(mo));
+    }
   }
 }
 
