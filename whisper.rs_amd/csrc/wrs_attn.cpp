@@ -44,6 +44,7 @@ struct wrs_attn_ctx {
   size_t part_bytes = 0;
   unsigned* counters = nullptr;  // decode merge counters (kept zero between launches)
   size_t counter_bytes = 0;
+  bool part_recorded = false;  // a graph may hold part and counters
   float* cap_part = nullptr;  // alignment-head capture chunk statistics
   size_t cap_part_bytes = 0;
   void* lin_x = nullptr;  // projections: split f16 rows of f32 activations + row scales
@@ -481,6 +482,7 @@ int decode_impl(wrs_attn_ctx* c, const float* q, int64_t q_rs, float* out, int64
       if (rc) return rc;
       rc = grow(c, reinterpret_cast<void**>(&c->counters), &c->counter_bytes, cb, true);
       if (rc) return rc;
+      c->part_recorded = c->part_recorded || capturing(c);
     }
   }
   if (fixed) {
@@ -1293,8 +1295,9 @@ int rows_impl(wrs_attn_ctx* c, wrs_kv* kv, const float* q, size_t n, float* out,
 // decode groups hold run on K10; up to that, and planes past its 32-bit offsets,
 // on the split-K decode kernel: groups of kMaxRowsPerGroup rows (the last may
 // hold fewer) share each read of the plane, up to kMaxDecodeGroups per launch.
-// Partials are laid out by whole groups; where the scratch holds the full groups'
-// but not the last one's, its rows go in a launch of their own.
+// Partials are laid out by whole groups; where a graph holds (or is recording)
+// scratch that takes the full groups but not the last one, its rows go in a launch
+// of their own (9 rows x 1500 keys, 20 heads: 11.4 us, 7.4 in one).
 // With lse, the rows' statistics too ([head][n][2], exp2 domain).
 int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, size_t n,
                     float* out, float* lse) {
@@ -1340,8 +1343,8 @@ int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, s
     rows = std::min(per_launch, n - r0);
     const int full = static_cast<int>(rows / rpg), heads = static_cast<int>(kv->n_heads);
     const int len = static_cast<int>(L);
-    if (full > 0 && rows % rpg && decode_fits(c, full, heads, len, rpg) &&
-        !decode_fits(c, full + 1, heads, len, rpg))
+    if (full > 0 && rows % rpg && !decode_fits(c, full + 1, heads, len, rpg) &&
+        decode_fits(c, full, heads, len, rpg) && (c->part_recorded || capturing(c)))
       rows = static_cast<size_t>(full) * rpg;
     const int last = static_cast<int>(std::min<size_t>(rows, rpg));
     const size_t groups = (rows + last - 1) / last;
