@@ -93,14 +93,14 @@ const char *wrs_attn_status_string(int status);
  * reference allocates per call on the host). Device-resident entry points
  * never allocate once their sizes are reserved; a call that would grow
  * scratch while the context's stream records a graph fails with
- * WRS_ECAPTURE instead. One exception needs no reservation:
+ * WRS_ECAPTURE instead. Two exceptions need no reservation:
  * 16-bit prefill grids of fewer 128-query blocks than half the CUs merge
  * blocks split over two workgroups through a fixed context buffer (~9 MB on
  * 256 CUs), allocated by the first such call outside capture; during capture
- * before then, the call takes another schedule instead. Projections of more
- * than 8 rows over n_in >= 2048 whose tiles cover less than half the CUs split
- * k through the same buffer, under the same rule (reserving linear_tokens
- * allocates it). Switching streams
+ * before then, the call takes another schedule instead; and projections of more
+ * than 8 rows over n_in >= 2048 whose tiles cover less than half the CUs, which
+ * split k through another fixed buffer (~8 MB on 256 CUs) under the same rule
+ * (reserving linear_tokens allocates it). Switching streams
  * (wrs_attn_set_stream) drains the old stream unless either stream is
  * recording a graph. Zero fields are ignored; reserving never shrinks.
  * Synchronous. */

@@ -450,3 +450,36 @@ def test_captured_decode_outlives_cross_rows(wrs, fresh_ctx, held, rows):
     arena2.close()
     other.close()
     arena.close()
+
+
+def test_captured_projection_outlives_forced_prefill(wrs, fresh_ctx):
+    # A recorded projection that splits k keeps its partials when a forced prefill
+    # schedule on a larger grid outgrows the prefill's own.
+    from wrs_amd import workloads as W
+    note("captured k split, forced prefill schedules, replays")
+    ctx = fresh_ctx
+    rows, n_in, n_out = 37, 5120, 256
+    x = dev(W.normal((rows, n_in), 51))
+    w = dev(W.normal((n_out, n_in), 52, sigma=0.02), torch.float16)
+    out = torch.zeros((rows, n_out), device="cuda")
+    wrs.linear(x, w, None, out, ctx=ctx)
+    torch.cuda.synchronize()
+    ref = out.clone()
+    want = x.double() @ w.double().t()
+    assert float((ref.double() - want).abs().max()) < 1e-5 * float(want.abs().max())
+    g = _capture(ctx, lambda: wrs.linear(x, w, None, out, ctx=ctx))
+    H, T = 20, 1500
+    qkv = [dev(W.normal((T, H * 64), 53 + i, storage="f16")) for i in range(3)]
+    h16 = [t.half() for t in qkv]
+    lay = wrs.token_major(T, H * 64, 64)
+    o = torch.zeros((T, H * 64), device="cuda")
+
+    def forced():
+        for t, queries, f32_split in ((qkv, 0, 5), (h16, -3, -1), (h16, -2, -1)):
+            ctx.set_schedule(queries, f32_split)
+            wrs.prefill(t[0], t[1], t[2], o, batch=1, n_heads=H, t_q=T, t_kv=T, d_head=64,
+                        q_layout=lay, kv_layout=lay, out_layout=lay, ctx=ctx)
+        ctx.set_schedule()
+
+    forced()
+    _replays_equal(g, out, ref, forced)

@@ -49,6 +49,12 @@ struct wrs_attn_ctx {
   size_t cap_part_bytes = 0;
   void* lin_x = nullptr;  // projections: split f16 rows of f32 activations + row scales
   size_t lin_x_bytes = 0;
+  // Projections that split k: partials and merge counters (kept zero between
+  // launches), of one size from the first such call on.
+  float* lin_part = nullptr;
+  size_t lin_part_bytes = 0;
+  unsigned* lin_counters = nullptr;
+  size_t lin_counter_bytes = 0;
   float* ln_x = nullptr;  // fused projections of rows too long for the split: normalized rows
   size_t ln_x_bytes = 0;
   // f32 arena attention: score rows, chunk statistics and partials, and merge
@@ -244,23 +250,29 @@ int run_exact(wrs_attn_ctx* c, const float* q, size_t q_floats, const float* k, 
   return WRS_OK;
 }
 
-// Context scratch for launches that split a block or tile over workgroups (pf
-// floats of partials, cw counter words; 0 when the launch needs none). Outside
-// capture it is allocated here, at least the size that every default split of
-// either kind needs (so that graphs captured later keep valid pointers), or
-// grown for a forced prefill schedule on a larger grid; during capture the
-// kernels take another schedule when what exists does not fit.
+// Scratch for a prefill schedule that splits blocks over workgroups (pf
+// floats of partials, cw counter words; 0 when it needs none). Outside capture
+// it is allocated here, at least the size every default split needs (so that
+// graphs captured later keep valid pointers), or grown for a forced schedule
+// on a larger grid; during capture the kernels take another schedule when
+// what exists does not fit.
 int split_scratch(wrs_attn_ctx* c, size_t pf, size_t cw) {
   if (!pf || capturing(c)) return WRS_OK;
   int rc = grow(c, reinterpret_cast<void**>(&c->split_part), &c->split_part_bytes,
-                std::max({pf, wrs::prefill_split_floats_min(), wrs::linear_split_floats()}) *
-                    sizeof(float),
-                false);
+                std::max(pf, wrs::prefill_split_floats_min()) * sizeof(float), false);
   if (rc) return rc;
   return grow(c, reinterpret_cast<void**>(&c->split_counters), &c->split_counter_bytes,
-              std::max({cw, wrs::prefill_split_words_min(), wrs::linear_split_words()}) *
-                  sizeof(unsigned),
-              true);
+              std::max(cw, wrs::prefill_split_words_min()) * sizeof(unsigned), true);
+}
+// The same for projections that split k, which run unsplit when captured before
+// it exists. It never grows: no call takes it from a graph that holds it.
+int linear_scratch(wrs_attn_ctx* c) {
+  if (capturing(c)) return WRS_OK;
+  int rc = grow(c, reinterpret_cast<void**>(&c->lin_part), &c->lin_part_bytes,
+                wrs::linear_split_floats() * sizeof(float), false);
+  if (rc) return rc;
+  return grow(c, reinterpret_cast<void**>(&c->lin_counters), &c->lin_counter_bytes,
+              wrs::linear_split_words() * sizeof(unsigned), true);
 }
 void give_scratch(wrs_attn_ctx* c, wrs::PrefillArgs& a) {
   a.split_part = c->split_part;
@@ -557,6 +569,8 @@ void wrs_attn_destroy(wrs_attn_ctx* c) {
   if (c->counters) (void)hipFree(c->counters);
   if (c->cap_part) (void)hipFree(c->cap_part);
   if (c->lin_x) (void)hipFree(c->lin_x);
+  if (c->lin_part) (void)hipFree(c->lin_part);
+  if (c->lin_counters) (void)hipFree(c->lin_counters);
   if (c->ln_x) (void)hipFree(c->ln_x);
   if (c->exact_scores) (void)hipFree(c->exact_scores);
   if (c->exact_counters) (void)hipFree(c->exact_counters);
@@ -694,7 +708,7 @@ int wrs_attn_reserve(wrs_attn_ctx* c, const wrs_reserve* r) {
         align_up(r->linear_tokens * wrs::kSplitParts * static_cast<int64_t>(r->linear_n_in) * 2, 256);
     rc = grow(c, &c->lin_x, &c->lin_x_bytes, split_bytes + r->linear_tokens * 4, false);
     if (rc) return rc;
-    rc = split_scratch(c, wrs::linear_split_floats(), wrs::linear_split_words());
+    rc = linear_scratch(c);
     if (rc) return rc;
     if (r->linear_n_in > static_cast<size_t>(wrs::kSplitLnMax)) {
       rc = grow(c, reinterpret_cast<void**>(&c->ln_x), &c->ln_x_bytes,
@@ -1702,13 +1716,13 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
     a.out[gi] = out[gi];
   }
   if (wrs::linear_needs_split(a)) {
-    rc = split_scratch(c, wrs::linear_split_floats(), wrs::linear_split_words());
+    rc = linear_scratch(c);
     if (rc) return rc;
-    if (c->split_counters) {  // captured before any scratch: no split
-      a.part = c->split_part;
-      a.part_floats = c->split_part_bytes / sizeof(float);
-      a.counters = c->split_counters;
-      a.counter_words = c->split_counter_bytes / sizeof(unsigned);
+    if (c->lin_counters) {  // captured before any scratch: no split
+      a.part = c->lin_part;
+      a.part_floats = c->lin_part_bytes / sizeof(float);
+      a.counters = c->lin_counters;
+      a.counter_words = c->lin_counter_bytes / sizeof(unsigned);
     }
   }
   WRS_HIP(c, wrs::launch_linear_f16w(a, static_cast<wrs::DType>(out_dtype), c->stream));
