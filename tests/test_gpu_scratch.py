@@ -483,3 +483,27 @@ def test_captured_projection_outlives_forced_prefill(wrs, fresh_ctx):
 
     forced()
     _replays_equal(g, out, ref, forced)
+
+
+@pytest.mark.parametrize("f32,rows", [(False, 1), (False, 129), (True, 1000), (False, 4_200_001)])
+def test_copy_slot_of_any_length(wrs, fresh_ctx, f32, rows):
+    # Also planes of more 16 KB pieces than the grid has workgroups for.
+    from gpu_util import read_f16, read_f32
+    note(f"copy_slot of {rows} rows, f32={f32}")
+    arena = wrs.KvArena(1, 2, 1, rows, 0, ctx=fresh_ctx,
+                        dtype=wrs.WRS_F32 if f32 else wrs.WRS_F16)
+    k = (torch.arange(rows * 64, device="cuda", dtype=torch.float32) % 2039).view(rows, 64)
+    v = -k
+    arena.append(0, 0, k, v)
+    arena.advance(0, rows)
+    arena.copy_slot(1, 0)
+    assert arena.slot_len(1) == rows
+    torch.cuda.synchronize()
+    kp, vp, _, _ = arena.plane_pointers()
+    read = read_f32 if f32 else read_f16
+    n = min(rows * 64, 100_000)
+    for at in (0, rows * 64 - n):
+        want = host(k.view(-1)[at:at + n])
+        assert np.array_equal(read(kp, rows * 64 + at, n), want)
+        assert np.array_equal(read(vp, rows * 64 + at, n), -want)
+    arena.close()

@@ -8,6 +8,8 @@
 // f32 row as two f16-sized rows.
 #include "wrs_internal.hpp"
 
+#include <algorithm>
+
 namespace wrs {
 namespace {
 
@@ -78,9 +80,11 @@ __global__ __launch_bounds__(256) void kv_slide(_Float16* k, _Float16* v, int64_
 }
 
 // Copy rows [0, len) of every (layer, head) plane of K and V from one slot to
-// another, kCopyUnits 16-byte units per workgroup, all read before any is written
-// (a workgroup that walked a whole plane waited out a round trip per 4 KB).
+// another. A workgroup takes pieces of kCopyUnits 16-byte units, every parts-th,
+// each read whole before it is written (one that walked a whole plane 4 KB at a
+// time waited out a round trip for each).
 constexpr int kCopyUnits = 1024;
+constexpr int kCopyParts = 32767;  // of a plane, at most: K's and V's share a grid dimension
 __global__ __launch_bounds__(256) void kv_copy_planes(const _Float16* k_src, _Float16* k_dst,
                                                       const _Float16* v_src, _Float16* v_dst,
                                                       int64_t layer_stride, int64_t plane_stride,
@@ -89,17 +93,20 @@ __global__ __launch_bounds__(256) void kv_copy_planes(const _Float16* k_src, _Fl
   const int64_t off = blockIdx.y * layer_stride + blockIdx.x * plane_stride;
   const u32x4* s = reinterpret_cast<const u32x4*>((which ? v_src : k_src) + off);
   u32x4* d = reinterpret_cast<u32x4*>((which ? v_dst : k_dst) + off);
-  const int n = len * 8;  // 16-byte units
-  u32x4 x[kCopyUnits / 256];
+  const int64_t n = static_cast<int64_t>(len) * 8;  // 16-byte units
+  for (int64_t i0 = static_cast<int64_t>(part) * kCopyUnits; i0 < n;
+       i0 += static_cast<int64_t>(parts) * kCopyUnits) {
+    u32x4 x[kCopyUnits / 256];
 #pragma unroll
-  for (int u = 0; u < kCopyUnits / 256; ++u) {
-    const int i = part * kCopyUnits + 256 * u + threadIdx.x;
-    x[u] = s[i < n ? i : 0];
-  }
+    for (int u = 0; u < kCopyUnits / 256; ++u) {
+      const int64_t i = i0 + 256 * u + threadIdx.x;
+      x[u] = s[i < n ? i : 0];
+    }
 #pragma unroll
-  for (int u = 0; u < kCopyUnits / 256; ++u) {
-    const int i = part * kCopyUnits + 256 * u + threadIdx.x;
-    if (i < n) d[i] = x[u];
+    for (int u = 0; u < kCopyUnits / 256; ++u) {
+      const int64_t i = i0 + 256 * u + threadIdx.x;
+      if (i < n) d[i] = x[u];
+    }
   }
 }
 
@@ -173,11 +180,11 @@ hipError_t launch_kv_copy_planes(const _Float16* k_src, _Float16* k_dst, const _
                                  _Float16* v_dst, int64_t layer_stride, int64_t plane_stride,
                                  int n_layers, int n_heads, int len, hipStream_t s) {
   if (n_layers <= 0 || n_heads <= 0 || len <= 0) return hipSuccess;
-  const int64_t parts = (static_cast<int64_t>(len) * 8 + kCopyUnits - 1) / kCopyUnits;
-  if (len > (1 << 27) || 2 * parts > 65535) return hipErrorInvalidConfiguration;
+  const int64_t pieces = (static_cast<int64_t>(len) * 8 + kCopyUnits - 1) / kCopyUnits;
+  const int parts = static_cast<int>(std::min<int64_t>(pieces, kCopyParts));
   hipLaunchKernelGGL(kv_copy_planes, dim3(n_heads, n_layers, static_cast<unsigned>(2 * parts)),
                      dim3(256), 0, s, k_src, k_dst, v_src, v_dst, layer_stride, plane_stride, len,
-                     static_cast<int>(parts));
+                     parts);
   return hipGetLastError();
 }
 
