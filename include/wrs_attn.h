@@ -272,9 +272,9 @@ int wrs_attn_decode_cross_noalloc(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, c
  * offset t_past = slot_len(slot) over the slot's f16 cache (rows appended),
  * and attention.rs:107-243 cross-attention with t_q = n_tokens. f16 keys and
  * values on the f16 matrix pipe, with q and the weights split into f16 parts:
- * two (2^-22) for cross-attention (up to 24 rows on the split-K decode kernel in
- * groups of 8 that share each read of the plane), three (all 24 bits of query
- * elements and weights down to 2^-28 of the row's largest) for the cached
+ * two (2^-22) for cross-attention (few rows or heads on the split-K decode kernel,
+ * in groups of 8 rows that share each read of the plane), three (all 24 bits of
+ * query elements and weights down to 2^-28 of the row's largest) for the cached
  * self-attention. */
 int wrs_attn_prefill_self(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, size_t slot,
                           const float *q, size_t n_tokens, float *out);

@@ -111,6 +111,48 @@ def test_cached_self_rows(wrs, ctx, heads, rows, past):
     arena.close()
 
 
+# The same where rows times heads put cross rows on K10 (more than 112 pairs of eight
+# rows and a head; 320 over planes of up to 256 keys; more than 64 groups), at the
+# edges of its 32-row blocks and 32-key steps and of the choice of waves.
+@pytest.mark.parametrize("heads,rows,keys", [
+    (81, 25, 1), (81, 31, 31), (81, 32, 32), (65, 33, 33), (20, 136, 255), (41, 64, 256),
+    (29, 25, 257), (29, 32, 511), (23, 33, 513), (29, 31, 767), (23, 40, 768), (20, 48, 1500),
+    (8, 128, 1500), (1, 513, 100), (1, 513, 300), (29, 27, 4097)])
+def test_cross_rows_of_many_heads(wrs, ctx, heads, rows, keys):
+    test_cross_rows(wrs, ctx, heads, rows, keys)
+
+
+def test_cross_rows_recorded_without_scratch(wrs):
+    # Rows that an eager call runs in decode groups are recorded without scratch for
+    # those, on K10.
+    note("cross rows captured without scratch")
+    c = wrs.Context(0)
+    c.use_torch_stream()
+    heads, rows, keys = 3, 37, 700
+    rng = np.random.default_rng(5)
+    k, v = (_f16(rng.standard_normal((keys, heads * 64))) for _ in range(2))
+    q = rng.standard_normal((rows, heads * 64)).astype(np.float32)
+    arena = wrs.KvArena(1, 1, heads, 16, keys, ctx=c)
+    arena.set_cross(0, k, v)
+    qd, out = dev(q), torch.zeros((rows, heads * 64), device="cuda")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        c.use_torch_stream()
+        arena.prefill_cross(0, qd, out)
+    c.use_torch_stream()
+    ref, _, _ = _attend(q, k, v, heads)
+    tol = _bound(q, k, v, heads)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        g.replay()
+        assert (np.abs(host(out) - ref) <= tol).all()
+        out.fill_(float("nan"))
+        arena.prefill_cross(0, qd, out)
+        assert (np.abs(host(out) - ref) <= tol).all()
+    arena.close()
+    c.close()
+
+
 # Rows whose output lives on weights far below the row's largest: one key, whose V
 # row is zero, scores `octaves` powers of two above the others. Only columns 0 (that
 # key alone) and 1 (the others alone) of K meet q, so a score is one product.
@@ -141,11 +183,12 @@ def _sink_tol(ref, octaves):
 @pytest.mark.parametrize("keys", [33, 448, 1500])
 def test_cross_rows_keep_small_weights(wrs, ctx, octaves, keys):
     note(f"cross rows, one key {octaves} octaves up of {keys}")
-    q, k, v = _sink(27, keys, octaves, octaves + keys)
-    arena = wrs.KvArena(1, 1, 1, 16, keys, ctx=ctx)
+    heads = 81  # on K10
+    q, k, v = (np.tile(a, (1, heads)) for a in _sink(27, keys, octaves, octaves + keys))
+    arena = wrs.KvArena(1, 1, heads, 16, keys, ctx=ctx)
     arena.set_cross(0, k, v)
-    out = torch.zeros((27, 64), device="cuda")
-    ref, _, _ = _attend(q, k, v, 1)
+    out = torch.zeros((27, heads * 64), device="cuda")
+    ref, _, _ = _attend(q, k, v, heads)
     arena.prefill_cross(0, dev(q), out)
     assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves)).all()
     arena.close()

@@ -15,10 +15,9 @@
 //   one before, and has its own accumulator (f16 ends at 2^-24: in one unit, what
 //   the last part could hold of a weight shrank with the weight). Two parts
 //   (cross-attention) carry 2^-22 of every query element within 2^-28 of its row's
-//   largest and of every weight within 2^-29 of the wave's largest so far, and
-//   to 2^-50 of that largest below; three (the cached self-attention, whose rows
-//   the f32 kernel ran before) carry all 24 bits, and to
-//   2^-61 below.
+//   largest and of every weight within 2^-29 of the wave's largest so far, and hold
+//   smaller ones to 2^-50 of that; three (the cached self-attention, whose rows the
+//   f32 kernel ran before) carry all 24 bits, and hold smaller ones to 2^-61.
 //   S^T = K Q^T puts one query per lane, and the packed weights are the B operand
 //   of O^T += V^T P^T as they stand; K comes from memory in operand layout, V
 //   passes through a wave's own swizzled LDS rows and is read transposed
@@ -26,11 +25,11 @@
 //   Bound by latency: launch, first loads, then ~1 us a step on few CUs, merge.
 //   Dealing a block's steps over several workgroups that merge through memory
 //   cost as much as it saved (128 rows x 1500 keys: 15.0 us in three).
-//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 16.2 us
-//   (groups of 8 rows each read the planes again: 123 MB of L2 reads), 37 rows 17.1
-//   -> 15.7 (two launches); 37 cached self rows 14.5 -> 5.6 us, 224 rows past 220
-//   37.9 -> 10.2 (f32 matrix pipe, element loads). One accumulator for all parts, all
-//   in the same units, took 14.2, 13.7, 5.3 and 9.1 us, and lost small weights.
+//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 15.9 us
+//   (groups of 8 rows each read the planes again: 123 MB of L2 reads); 37 cached self
+//   rows 14.5 -> 5.6 us, 224 rows past 220 37.9 -> 10.1 (f32 matrix pipe, element
+//   loads). One accumulator for all parts, all in the same units, took 14.2, 5.3 and
+//   9.1 us, and lost small weights.
 #include "prefill_f32_block.hpp"
 
 namespace wrs {
@@ -340,8 +339,9 @@ hipError_t launch_attend_rows(const RowsArgs& a, hipStream_t s) {
   const int64_t wgs = static_cast<int64_t>(n_qblk) * a.n_heads;
   if (wgs > 0x7fffffff) return hipErrorInvalidConfiguration;
   const dim3 grid(static_cast<unsigned>(wgs));
-  // Eight waves where they get three steps or more each (1500 keys, 128 rows:
-  // 13.4 us, 14.4 on four); four below (300 keys: 7.1 us, 7.8 on eight).
+  // Eight waves where they get three steps or more each (128 rows x 1500 keys: 15.8
+  // us, 16.5 on four); four below (300 keys: 7.6 us, 8.2 on eight; 224 self rows past
+  // 220: 10.1, 11.0).
   const bool wide = a.n_keys >= 24 * kN;
 #define WRS_ROWS(P, W) \
   hipLaunchKernelGGL((attend_rows<P, W>), grid, dim3(64 * W), 0, s, a, n_qblk)

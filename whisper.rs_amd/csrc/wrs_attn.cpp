@@ -1305,9 +1305,9 @@ int rows_impl(wrs_attn_ctx* c, wrs_kv* kv, const float* q, size_t n, float* out,
   return WRS_OK;
 }
 
-// Cross-attention of n query rows over one layer's plane. More rows than three
-// decode groups hold run on K10; up to that, and planes past its 32-bit offsets,
-// on the split-K decode kernel: groups of kMaxRowsPerGroup rows (the last may
+// Cross-attention of n query rows over one layer's plane. Many rows times heads
+// run on K10 (rule below); fewer, and planes past its 32-bit offsets, on the
+// split-K decode kernel: groups of kMaxRowsPerGroup rows (the last may
 // hold fewer) share each read of the plane, up to kMaxDecodeGroups per launch.
 // Partials are laid out by whole groups; where a graph holds (or is recording)
 // scratch that takes the full groups but not the last one, its rows go in a launch
@@ -1346,19 +1346,29 @@ int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, s
                         lkv, wrs_kv::f32p(kv->v_cross, kv->cross_off(layer)), lkv, out, lq, 1,
                         kv->n_heads, n, L, 64, 0, 0);
   }
-  // Groups share no reads, so K10 wins where many would (1500 keys, 20 heads: 24
-  // rows 9.4 us in groups, 12.8 on K10; 37 rows 16.9 and 13.3).
-  if (n > 3 * static_cast<size_t>(wrs::kMaxRowsPerGroup) && L < wrs::kRowsMaxKeys)
+  // Every (group, head) reads the plane for itself; K10 reads it once per 32 rows,
+  // but a block of them takes all of it in. us, groups / K10: 300 keys, 96 pairs
+  // 7.4/7.3, 192 9.5/7.4; 700 keys, 96 8.9/10.1, 140 11.1/10.2; 1500 keys, 96
+  // 12.2/15.3, 120 15.7/15.4, 320 33.7/15.8; 3000 keys, 80 21.0/24.4, 120 28.5/24.5.
+  // Planes that a workgroup of the decode takes whole (256 keys): 192 pairs 4.7/6.5,
+  // 320 6.8/6.6. K10 also takes what is recorded without the scratch for groups.
+  const bool recorded = c->part_recorded || capturing(c);
+  const int heads = static_cast<int>(kv->n_heads), len = static_cast<int>(L);
+  const size_t n_groups = (n + wrs::kMaxRowsPerGroup - 1) / wrs::kMaxRowsPerGroup;
+  if (n_groups > 3 && L < wrs::kRowsMaxKeys &&
+      (n_groups > static_cast<size_t>(wrs::kMaxDecodeGroups) ||
+       n_groups * kv->n_heads > (decode_splits(len) == 1 ? 320u : 112u) ||
+       (recorded && !decode_fits(c, static_cast<int>(n_groups), heads, len,
+                                 wrs::kMaxRowsPerGroup))))
     return rows_impl(c, kv, q, n, out, kv->k_cross, kv->v_cross, kv->cross_off(layer),
                      kv->n_audio_max * 64, L, false, 0, lse);
   const int rpg = static_cast<int>(std::min<size_t>(n, wrs::kMaxRowsPerGroup));
   const size_t per_launch = static_cast<size_t>(wrs::kMaxDecodeGroups) * rpg;
   for (size_t r0 = 0, rows = 0; r0 < n; r0 += rows) {
     rows = std::min(per_launch, n - r0);
-    const int full = static_cast<int>(rows / rpg), heads = static_cast<int>(kv->n_heads);
-    const int len = static_cast<int>(L);
+    const int full = static_cast<int>(rows / rpg);
     if (full > 0 && rows % rpg && !decode_fits(c, full + 1, heads, len, rpg) &&
-        decode_fits(c, full, heads, len, rpg) && (c->part_recorded || capturing(c)))
+        decode_fits(c, full, heads, len, rpg) && recorded)
       rows = static_cast<size_t>(full) * rpg;
     const int last = static_cast<int>(std::min<size_t>(rows, rpg));
     const size_t groups = (rows + last - 1) / last;
