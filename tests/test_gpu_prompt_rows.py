@@ -153,6 +153,13 @@ def test_cross_rows_recorded_without_scratch(wrs):
     c.close()
 
 
+@pytest.mark.parametrize("heads,rows,past", [(1, 2, 2046), (1, 2, 2047), (2, 33, 3000),
+                                             (16, 32, 2500), (17, 32, 2500)])
+def test_cached_self_rows_of_long_caches(wrs, ctx, heads, rows, past):
+    # Few blocks over more than 2048 keys: the f32 kernel, its keys dealt over workgroups.
+    test_cached_self_rows(wrs, ctx, heads, rows, past)
+
+
 # Rows whose output lives on weights far below the row's largest: one key, whose V
 # row is zero, scores `octaves` powers of two above the others. Only columns 0 (that
 # key alone) and 1 (the others alone) of K meet q, so a score is one product.

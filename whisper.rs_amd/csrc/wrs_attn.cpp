@@ -1430,17 +1430,24 @@ int wrs_attn_prefill_self(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, size_t slot
     }
     return WRS_OK;
   }
-  if (t_past + n_tokens < wrs::kRowsMaxKeys) {
+  // K10, but for few blocks of 32 rows over long caches, whose keys the f32 kernel
+  // deals over workgroups (through scratch; us, K10 / f32 kernel, blocks x keys): 1 x
+  // 2000 21.4/21.3, 1 x 4000 37.6/28.9, 12 x 4000 39.0/33.2, 20 x 4000 38.2/36.4, 40 x
+  // 4000 39.3/60.8, 20 x 2000 21.8/28.5, 8 x 8000 71.2/55.0.
+  const size_t keys = t_past + n_tokens;
+  const bool dealt = keys > 2048 && (n_tokens + 31) / 32 * kv->n_heads <= 16 &&
+                     (c->split_part || !capturing(c));
+  if (keys < wrs::kRowsMaxKeys && !dealt) {
     if (!q || !out) return fail(c, WRS_EINVAL, "null tensor pointer");
     return rows_impl(c, kv, q, n_tokens, out, kv->k_self, kv->v_self, kv->self_off(layer, slot),
-                     kv->plane(), t_past + n_tokens, true, t_past, nullptr);
+                     kv->plane(), keys, true, t_past, nullptr);
   }
   const wrs_layout lq{0, 64, dm};
   const wrs_layout lkv{0, static_cast<int64_t>(kv->plane()), 64};
   const uint16_t* kb = wrs_kv::u16(kv->k_self, kv->self_off(layer, slot));
   const uint16_t* vb = wrs_kv::u16(kv->v_self, kv->self_off(layer, slot));
   return prefill_impl(c, WRS_F32, q, lq, WRS_F16, kb, lkv, vb, lkv, out, lq, 1, kv->n_heads,
-                      n_tokens, t_past + n_tokens, 64, 1, t_past);
+                      n_tokens, keys, 64, 1, t_past);
 }
 
 int wrs_attn_prefill_cross(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q,
