@@ -125,7 +125,10 @@ __global__ __launch_bounds__(64 * kMWaves) void decode_f16(DecodeArgs a) {
   const int dpart = kDS > 1 ? lid % kDS : 0;  // columns [64/kDS dpart, 64/kDS (dpart+1))
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   constexpr int rows = R;  // == a.rows_per_group
-  const int valid = min(rows, a.n_rows - g * rows);  // the last group may hold fewer
+  // The last of several groups may hold fewer rows: its last one again in their
+  // place, computed and not stored (a test per row on the way to the scores cost 0.2
+  // of 3.4 us).
+  const int valid = R == kMaxRowsPerGroup ? min(rows, a.n_rows - g * rows) : rows;
   const int len = a.len[g];
   const int col = lane & 15, kg = lane >> 4;
   const bool lo_part = col >= 8;
@@ -143,13 +146,14 @@ __global__ __launch_bounds__(64 * kMWaves) void decode_f16(DecodeArgs a) {
   // banks (at a 64-float pitch they shared them).
   __shared__ __attribute__((aligned(16))) float qs[kStageQ ? 8 : 1][kQsPitch];
   __shared__ float qdown[8];
-  const bool qload = kStageQ && tid < valid * 16;
+  const bool qload = kStageQ && tid < rows * 16;
   f32x4 qx = {0.f, 0.f, 0.f, 0.f};
   float qv[16];
   if constexpr (kStageQ) {
     if (qload)
-      qx = *reinterpret_cast<const f32x4*>(a.q + static_cast<int64_t>(g * rows + (tid >> 4)) *
-                                                     a.q_rs + h * 64 + 4 * (tid & 15));
+      qx = *reinterpret_cast<const f32x4*>(
+          a.q + static_cast<int64_t>(g * rows + min(tid >> 4, valid - 1)) * a.q_rs + h * 64 +
+          4 * (tid & 15));
   } else {
     const float* qp = a.q + static_cast<int64_t>(g) * a.q_rs + h * 64 + 8 * kg;
 #pragma unroll
@@ -212,12 +216,12 @@ __global__ __launch_bounds__(64 * kMWaves) void decode_f16(DecodeArgs a) {
     }
     __syncthreads();
     // Rows past the group's are zero.
-    down = qrow < valid ? qdown[qrow] : 1.f;
+    down = qrow < rows ? qdown[qrow] : 1.f;
     const f32x4 z4 = {0.f, 0.f, 0.f, 0.f};
-    const f32x4 q0 = qrow < valid ? *reinterpret_cast<const f32x4*>(&qs[qrow][8 * kg]) : z4;
-    const f32x4 q1 = qrow < valid ? *reinterpret_cast<const f32x4*>(&qs[qrow][8 * kg + 4]) : z4;
-    const f32x4 q2 = qrow < valid ? *reinterpret_cast<const f32x4*>(&qs[qrow][32 + 8 * kg]) : z4;
-    const f32x4 q3 = qrow < valid ? *reinterpret_cast<const f32x4*>(&qs[qrow][36 + 8 * kg]) : z4;
+    const f32x4 q0 = qrow < rows ? *reinterpret_cast<const f32x4*>(&qs[qrow][8 * kg]) : z4;
+    const f32x4 q1 = qrow < rows ? *reinterpret_cast<const f32x4*>(&qs[qrow][8 * kg + 4]) : z4;
+    const f32x4 q2 = qrow < rows ? *reinterpret_cast<const f32x4*>(&qs[qrow][32 + 8 * kg]) : z4;
+    const f32x4 q3 = qrow < rows ? *reinterpret_cast<const f32x4*>(&qs[qrow][36 + 8 * kg]) : z4;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       qv[j] = q0[j];
