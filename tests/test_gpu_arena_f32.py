@@ -346,3 +346,39 @@ def test_exact_decode_key_counts(wrs, ctx, keys, rows):
     wrs.single_token_mha_d64(qw, kw.ravel(), vw.ravel(), keys, H, wide, one, ctx=ctx)
     assert np.array_equal(one[:dm], got[0])
     arena.close()
+
+
+@pytest.mark.parametrize("H,past,rows", [(20, 0, 448), (17, 120, 150), (21, 200, 100), (9, 250, 262)])
+def test_exact_prompts_of_many_rows(wrs, ctx, H, past, rows):
+    """Prompts whose rows of up to 128 and 256 keys have launches of their own:
+    against float64, and bit for bit the single-token call at either side of them."""
+    note(f"exact prompt heads={H} past={past} rows={rows}")
+    dm, n = H * 64, past + rows
+    rng = np.random.default_rng(n)
+    k, v = (rng.standard_normal((n, dm)).astype(np.float32) for _ in range(2))
+    q = (2.0 * rng.standard_normal((rows, dm))).astype(np.float32)
+    arena = _arena(wrs, ctx, 1, 1, H, n + 3, 0)
+    if past:
+        arena.append(0, 0, k[:past], v[:past])
+        arena.advance(0, past)
+    arena.append(0, 0, np.ascontiguousarray(k[past:]), np.ascontiguousarray(v[past:]))
+    out = torch.full((rows + 1, dm), float("nan"), device="cuda")
+    arena.prefill_self(0, 0, dev(q), out[:rows])
+    got = host(out)
+    assert np.isnan(got[rows]).all()
+    qd, kd, vd = (a.astype(np.float64).reshape(-1, H, 64).transpose(1, 0, 2) for a in (q, k, v))
+    s = qd @ kd.transpose(0, 2, 1) / 8.0
+    s = np.where(np.arange(n)[None, :] > past + np.arange(rows)[:, None], -np.inf, s)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    ref = (np.where(p < 1e-7, 0.0, p) @ vd).transpose(1, 0, 2).reshape(rows, dm)
+    # f32 sums of 64 products and of n weights, and weights at the 1e-7 line
+    assert np.abs(got[:rows] - ref).max() <= 4e-6 + 5e-7
+    for seen in {past + 1, 127, 128, 129, 255, 256, 257, n}:
+        r = seen - 1 - past
+        if 0 <= r < rows:
+            one = np.zeros(dm, np.float32)
+            wrs.single_token_mha_d64(q[r].copy(), k[:seen].ravel(), v[:seen].ravel(), seen, H, dm,
+                                     one, ctx=ctx)
+            assert np.array_equal(one, got[r]), seen
+    arena.close()
