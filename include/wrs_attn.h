@@ -361,8 +361,11 @@ int wrs_linear_group(wrs_attn_ctx *ctx, int x_dtype, const void *x, size_t x_len
  * each output (before rounding when out_dtype is f16/bf16). x is f32;
  * ln_gamma and ln_beta (16-byte aligned, n_in values) are both NULL to skip
  * the norm; activation is WRS_ACT_NONE or WRS_ACT_GELU. Batches above 8 rows
- * (or x beyond the weight-stream kernel's LDS) run the norm as its own
- * launch and then need packed rows (x_row_stride == n_in). */
+ * (or x beyond the weight-stream kernel's LDS) need packed rows (x_row_stride ==
+ * n_in) for the norm, which runs with their split into f16 parts up to n_in =
+ * 2048 and as a launch of its own beyond; so it does for one or two rows of more
+ * than 1280 over many features (through a fixed context buffer of 160 KB, which
+ * the first such call outside capture allocates). */
 int wrs_linear_fused(wrs_attn_ctx *ctx, const float *x, size_t x_len, int64_t x_row_stride,
                      const float *ln_gamma, const float *ln_beta, float ln_eps,
                      size_t n_groups, const void *const *w, const float *const *bias,

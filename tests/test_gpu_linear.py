@@ -618,3 +618,54 @@ def test_linear_long_rows_few_tiles(wrs, ctx, n_tokens, n_in, n_out, n_groups):
         bound = _gamma_bound(x, w) + 2.0 ** -23 * np.abs(b)
         assert (np.abs(host(o) - _exact(x, w, b)) <= bound).all()
         assert torch.equal(o, o2)
+
+
+@pytest.mark.parametrize("rows,n_in,n_out,groups", [
+    (1, 1344, 9728, 1), (2, 1344, 3277, 3), (1, 5120, 5120, 1), (2, 5120, 5119, 1), (3, 1344, 9728, 1)])
+def test_fused_norm_of_long_decode_rows(wrs, ctx, rows, n_in, n_out, groups):
+    # The norm of one or two long rows over many features runs as a launch of its own:
+    # bit for bit the separate calls, eager and (before its buffer exists) captured,
+    # from rows with a stride of their own too.
+    note(f"fused norm rows={rows} {n_in} -> {groups} x {n_out}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n_in + n_out)
+    wide = torch.randn((rows, n_in + 8), generator=g, device="cuda")
+    x = wide[:, :n_in].contiguous()
+    ws = [(torch.randn((n_out, n_in), generator=g, device="cuda") / n_in ** 0.5).half()
+          for _ in range(groups)]
+    gamma = torch.rand(n_in, generator=g, device="cuda")
+    beta = torch.randn(n_in, generator=g, device="cuda")
+    normed = torch.empty_like(x)
+    wrs.layer_norm(x, gamma, beta, 1e-5, normed, ctx=ctx)
+    ref = [torch.empty((rows, n_out), device="cuda") for _ in range(groups)]
+    wrs.linear_group(normed, ws, None, ref, ctx=ctx)
+    want = normed.double() @ ws[0].double().t()
+    assert float((ref[0].double() - want).norm() / want.norm()) < 1e-6
+    own = wrs.Context(0)
+    own.use_torch_stream()
+    outs = [torch.zeros((rows, n_out), device="cuda") for _ in range(groups)]
+
+    def run(rows_in):
+        wrs.linear_fused(rows_in, ws, None, outs, ln=(gamma, beta, 1e-5), ctx=own)
+
+    def check():
+        torch.cuda.synchronize()
+        for a, b in zip(outs, ref):
+            assert torch.equal(a, b)
+            a.zero_()
+
+    graphs = []
+    for _ in range(2):  # recorded without the buffer, then with it
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            own.use_torch_stream()
+            run(x)
+        own.use_torch_stream()
+        run(x)
+        check()
+    for graph in graphs * 2:
+        graph.replay()
+        check()
+        run(wide[:, :n_in])
+        check()
+    own.close()

@@ -57,6 +57,8 @@ struct wrs_attn_ctx {
   size_t lin_counter_bytes = 0;
   float* ln_x = nullptr;  // fused projections of rows too long for the split: normalized rows
   size_t ln_x_bytes = 0;
+  float* ln_rows = nullptr;  // fused decode projections of long rows: normalized rows (one size)
+  size_t ln_rows_bytes = 0;
   // f32 arena attention: score rows, chunk statistics and partials, and merge
   // counters (kept zero between launches).
   float* exact_scores = nullptr;
@@ -572,6 +574,7 @@ void wrs_attn_destroy(wrs_attn_ctx* c) {
   if (c->lin_part) (void)hipFree(c->lin_part);
   if (c->lin_counters) (void)hipFree(c->lin_counters);
   if (c->ln_x) (void)hipFree(c->ln_x);
+  if (c->ln_rows) (void)hipFree(c->ln_rows);
   if (c->exact_scores) (void)hipFree(c->exact_scores);
   if (c->exact_counters) (void)hipFree(c->exact_counters);
   if (c->split_part) (void)hipFree(c->split_part);
@@ -1677,6 +1680,30 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
     if (x_row_stride < static_cast<int64_t>(n_in) || n_in > (1u << 24) ||
         n_out > static_cast<size_t>(INT32_MAX / 2))
       return fail(c, WRS_EINVAL, "projection shape");
+    // One or two rows too long for a workgroup's registers, whose statistics every
+    // workgroup would form again: over many features they are normalized once, by a
+    // launch of its own (captured before its buffer exists, they are formed again).
+    // us, in the kernel / in a launch, 2 rows: 1344 -> 10240 10.9/8.3, -> 51866
+    // 43.5/24.5; 3072 -> 4096 8.8/10.4, -> 5120 15.4/12.9; 5120 -> 4096 22.0/24.3, ->
+    // 5120 30.3/25.7, -> 51866 263/114. From three rows on the launch gains nothing.
+    const int64_t features = static_cast<int64_t>(n_out) * n_groups;
+    if (ln_g && n_tokens <= 2 && n_in > static_cast<size_t>(wrs::kGemvLnMax) &&
+        (n_tokens == 1 || x_row_stride == static_cast<int64_t>(n_in)) && features >= 5120 &&
+        static_cast<int64_t>(n_in) * features >= (12 << 20)) {
+      if (!capturing(c)) {
+        const int rc = grow(c, reinterpret_cast<void**>(&c->ln_rows), &c->ln_rows_bytes,
+                            wrs::kGemvXFloats * sizeof(float), false);
+        if (rc) return rc;
+      }
+      if (c->ln_rows) {  // n_tokens * n_in <= kGemvXFloats
+        WRS_HIP(c, wrs::launch_layer_norm(static_cast<const float*>(x), ln_g, ln_b, ln_eps,
+                                          static_cast<int>(n_tokens), static_cast<int>(n_in),
+                                          wrs::kF32, c->ln_rows, c->stream));
+        x = c->ln_rows;
+        x_row_stride = static_cast<int64_t>(n_in);
+        ln_g = ln_b = nullptr;
+      }
+    }
     wrs::GemvArgs gv{};
     gv.x = x;
     gv.x_rs = x_row_stride;

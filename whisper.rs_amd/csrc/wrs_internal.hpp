@@ -294,6 +294,7 @@ constexpr int kGemvMaxRows = 8;
 // room for 64 groups cost 0.5 us of a 6.7 us call (5 rows 768 x 768), room for 8 is
 // what a layer's projections need (3).
 constexpr int kMaxGemvGroups = 8;
+constexpr int kGemvLnMax = 1280;  // longer f32 rows do not fit the decode kernels' registers
 constexpr int kGemvXFloats = 40960;  // n_tokens * n_in staged in LDS (160 KB)
 struct GemvArgs {
   const void* x;
