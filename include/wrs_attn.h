@@ -272,10 +272,10 @@ int wrs_attn_decode_cross_noalloc(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, c
  * offset t_past = slot_len(slot) over the slot's f16 cache (rows appended),
  * and attention.rs:107-243 cross-attention with t_q = n_tokens. f16 keys and
  * values on the f16 matrix pipe, with q and the weights split into f16 parts:
- * two (2^-22) for cross-attention (few rows or heads on the split-K decode kernel,
- * in groups of 8 rows that share each read of the plane), three (all 24 bits of
- * query elements and weights down to 2^-28 of the row's largest) for the cached
- * self-attention (on the f32 kernel where few rows meet more than 2048 keys). */
+ * two (2^-22 down to 2^-18 of the row's largest) for cross-attention (few rows or
+ * heads on the split-K decode kernel, in groups of 8 rows that share each read of
+ * the plane), three (all 24 bits down to 2^-28) for the cached self-attention (on
+ * the f32 kernel where few rows meet more than 2048 keys). */
 int wrs_attn_prefill_self(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, size_t slot,
                           const float *q, size_t n_tokens, float *out);
 int wrs_attn_prefill_cross(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, const float *q,

@@ -111,7 +111,7 @@ def test_cached_self_rows(wrs, ctx, heads, rows, past):
     arena.close()
 
 
-# The same where rows times heads put cross rows on K10 (more than 112 pairs of eight
+# The same where rows times heads put cross rows on K10 (more than 104 pairs of eight
 # rows and a head; 320 over planes of up to 256 keys; more than 64 groups), at the
 # edges of its 32-row blocks and 32-key steps and of the choice of waves.
 @pytest.mark.parametrize("heads,rows,keys", [
@@ -177,13 +177,14 @@ def _sink(rows, keys, octaves, seed):
     return q, k, v
 
 
-def _sink_tol(ref, octaves):
+def _sink_tol(ref, octaves, end):
     """Relative error per output: each exponent argument is one product of at most
     octaves + 2 in magnitude (operand split to 2^-22, scaling and product to 2^-24
-    each, differences of two of them), every weight the other way round to 2^-22,
-    and a mean of positive values, summed in f32 (2^-20)."""
+    each, differences of two of them), every weight the other way round to 2^-22 or
+    to half of the parts' end (2^-end of the largest, the weights being down to
+    octaves + 2 below it), and a mean of positive values, summed in f32 (2^-20)."""
     arg = 2.0 * (octaves + 2.0) * (2.0 ** -22 + 3.0 * 2.0 ** -24) * np.log(2.0)
-    return np.abs(ref) * (arg + 2.0 ** -20 + 2.0 ** -22)
+    return np.abs(ref) * (arg + 2.0 ** -20 + 2.0 ** -22 + 2.0 ** (octaves + 1 - end))
 
 
 @pytest.mark.parametrize("octaves", [2, 14, 17, 20, 23, 26, 32])
@@ -197,7 +198,7 @@ def test_cross_rows_keep_small_weights(wrs, ctx, octaves, keys):
     out = torch.zeros((27, heads * 64), device="cuda")
     ref, _, _ = _attend(q, k, v, heads)
     arena.prefill_cross(0, dev(q), out)
-    assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves)).all()
+    assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves, 39)).all()
     arena.close()
 
 
@@ -214,7 +215,7 @@ def test_cached_self_rows_keep_small_weights(wrs, ctx, octaves, rows, past):
     out = torch.zeros((rows, 64), device="cuda")
     ref, _, _ = _attend(q, k, v, 1, past)
     arena.prefill_self(0, 0, dev(q), out)
-    assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves)).all()
+    assert (np.abs(host(out) - ref) <= _sink_tol(ref, octaves, 61)).all()
     arena.close()
 
 

@@ -11,13 +11,12 @@
 //   The arithmetic runs on the f16 matrix pipe with split operands: each query
 //   row, times scale * log2(e) and a power of two that puts its largest element
 //   into [2^14, 2^15), is split into kParts f16 parts, and so are the softmax
-//   weights in units of 2^-15. Each part stands in units of its own, 2^-11 of the
-//   one before, and has its own accumulator (f16 ends at 2^-24: in one unit, what
-//   the last part could hold of a weight shrank with the weight). Two parts
-//   (cross-attention) carry 2^-22 of every query element within 2^-28 of its row's
-//   largest and of every weight within 2^-29 of the wave's largest so far, and hold
-//   smaller ones to 2^-50 of that; three (the cached self-attention, whose rows the
-//   f32 kernel ran before) carry all 24 bits, and hold smaller ones to 2^-61.
+//   weights in units of 2^-15. Two parts in one unit (cross-attention, as the
+//   split-K decode) carry 2^-22 of every query element and weight within 2^-18 of
+//   the row's largest, and smaller ones to 2^-40 of it, where f16 ends. Three parts
+//   (the cached self-attention, whose rows the f32 kernel ran before), each in a unit
+//   2^-11 of the one before and with an accumulator of its own, carry all 24 bits down
+//   to 2^-28, and smaller ones to 2^-60.
 //   S^T = K Q^T puts one query per lane, and the packed weights are the B operand
 //   of O^T += V^T P^T as they stand; K comes from memory in operand layout, V
 //   passes through a wave's own swizzled LDS rows and is read transposed
@@ -25,11 +24,12 @@
 //   Bound by latency: launch, first loads, then ~1 us a step on few CUs, merge.
 //   Dealing a block's steps over several workgroups that merge through memory
 //   cost as much as it saved (128 rows x 1500 keys: 15.0 us in three).
-//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 15.9 us
+//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 15.0 us
 //   (groups of 8 rows each read the planes again: 123 MB of L2 reads); 37 cached self
-//   rows 14.5 -> 5.6 us, 224 rows past 220 37.9 -> 10.1 (f32 matrix pipe, element
-//   loads). One accumulator for all parts, all in the same units, took 14.2, 5.3 and
-//   9.1 us, and lost small weights.
+//   rows 14.5 -> 5.6 us, 224 rows past 220 37.9 -> 10.2 (f32 matrix pipe, element
+//   loads). Weights in units of 1 and three parts in one unit took 14.2, 5.3 and 9.1
+//   us, but a weight 2^-20 of the largest kept four bits; two parts in units of their
+//   own 16.2.
 #include "prefill_f32_block.hpp"
 
 namespace wrs {
@@ -47,7 +47,7 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int kQ = 32;               // query rows per block
 constexpr int kN = 32;               // keys per step
-constexpr float kWeightUp = 0x1p15f;  // softmax weights, at most 1, are split in these units
+constexpr float kWeightUp = 0x1p15f;  // softmax weights, at most 1, are split in units of its inverse
 constexpr int kPitch = 66;           // LDS pitch (floats) of a merge row
 constexpr int kRawBuffer = 0x00020000;  // buffer resource word 3: raw, 32-bit data format
 
@@ -70,28 +70,36 @@ __device__ inline f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a),
                                                 __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
 }
-// Two floats of at most 2^15 as kParts packed f16 pairs, part p in units of
-// kPartUnit^p: what a part leaves is at most 2^-11 of the value, so the next one
-// holds 11 bits more at the same magnitude. Two parts carry 22 bits of values from
-// 2^-14 up (f16's normal range), three all 24.
+// Two floats, times `scale` at most 2^15, as packed f16 pairs: two parts in one unit,
+// whose last ends at f16's 2^-24, or three, part p in units of kPartUnit^p: what a
+// part leaves is at most 2^-11 of the value, so the next one holds 11 bits more at
+// the same magnitude.
 constexpr float kPartUnit = 0x1p-11f;
-template <int kParts>
-__device__ inline void split2(float x0, float x1, uint32_t (&out)[kParts]) {
+__device__ inline void split2(float x0, float x1, float scale, uint32_t (&out)[2]) {
+  const f16x2 h = {static_cast<_Float16>(x0 * scale), static_cast<_Float16>(x1 * scale)};
+  const f16x2 l = {
+      static_cast<_Float16>(__builtin_fmaf(x0, scale, -static_cast<float>(h[0]))),
+      static_cast<_Float16>(__builtin_fmaf(x1, scale, -static_cast<float>(h[1])))};
+  out[0] = __builtin_bit_cast(uint32_t, h);
+  out[1] = __builtin_bit_cast(uint32_t, l);
+}
+__device__ inline void split2(float x0, float x1, float scale, uint32_t (&out)[3]) {
   constexpr float kUp = 1.f / kPartUnit;
+  x0 *= scale;
+  x1 *= scale;
 #pragma unroll
-  for (int p = 0; p < kParts; ++p) {
+  for (int p = 0; p < 3; ++p) {
     const f16x2 h = {static_cast<_Float16>(x0), static_cast<_Float16>(x1)};
     out[p] = __builtin_bit_cast(uint32_t, h);
     x0 = __builtin_fmaf(static_cast<float>(h[0]), -kUp, x0 * kUp);  // exact
     x1 = __builtin_fmaf(static_cast<float>(h[1]), -kUp, x1 * kUp);
   }
 }
-// The sum of products of the parts, smallest first.
-template <int kParts>
-__device__ inline f32x16 join(const f32x16 (&x)[kParts]) {
-  f32x16 s = x[kParts - 1];
+// Three parts' sums of products as one, smallest first.
+__device__ inline f32x16 join(const f32x16 (&x)[3]) {
+  f32x16 s = x[2];
 #pragma unroll
-  for (int p = kParts - 2; p >= 0; --p)
+  for (int p = 1; p >= 0; --p)
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(s[i], kPartUnit, x[p][i]);
   return s;
@@ -170,7 +178,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     uint32_t w[kParts];
-    split2<kParts>(qx[i >> 1][2 * (i & 1)] * up, qx[i >> 1][2 * (i & 1) + 1] * up, w);
+    split2(qx[i >> 1][2 * (i & 1)], qx[i >> 1][2 * (i & 1) + 1], up, w);
 #pragma unroll
     for (int p = 0; p < kParts; ++p) qf[p][i >> 2][i & 3] = w[p];
   }
@@ -184,15 +192,26 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
   f32x16 o[2] = {f32x16{}, f32x16{}};
   float m = -INFINITY, l = 0.f;
   for (; step < n_steps; step += kWaves) {
-    // One chain over d per part.
-    f32x16 sp[kParts];
+    f32x16 s;
+    if constexpr (kParts == 3) {
+      f32x16 sp[kParts];  // a chain over d per part
 #pragma unroll
-    for (int p = 0; p < kParts; ++p) sp[p] = f32x16{};
+      for (int p = 0; p < kParts; ++p) sp[p] = f32x16{};
 #pragma unroll
-    for (int dk = 0; dk < 4; ++dk)
+      for (int dk = 0; dk < 4; ++dk)
 #pragma unroll
-      for (int p = 0; p < kParts; ++p) sp[p] = mfma(kx[dk], qf[p][dk], sp[p]);
-    f32x16 s = join(sp);
+        for (int p = 0; p < kParts; ++p) sp[p] = mfma(kx[dk], qf[p][dk], sp[p]);
+      s = join(sp);
+    } else {
+      // Two chains over d (half the latency and half the roundings of one), the
+      // smaller part first, so that few of the sums round at full size.
+      f32x16 s2[2] = {f32x16{}, f32x16{}};
+#pragma unroll
+      for (int p = kParts - 1; p >= 0; --p)
+#pragma unroll
+        for (int dk = 0; dk < 4; ++dk) s2[dk & 1] = mfma(kx[dk], qf[p][dk], s2[dk & 1]);
+      s = s2[0] + s2[1];
+    }
     wave_sync();  // the last step's transposed reads are done
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -225,7 +244,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
       const float p1 = __builtin_amdgcn_exp2f(s[i + 1] - m_use);
       ls += p0 + p1;
       uint32_t w[kParts];
-      split2<kParts>(p0 * kWeightUp, p1 * kWeightUp, w);
+      split2(p0, p1, kWeightUp, w);
 #pragma unroll
       for (int p = 0; p < kParts; ++p) pf[p][i >> 3][(i >> 1) & 3] = w[p];
     }
@@ -243,14 +262,22 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
         }
         va[k2] = u32x4{t[0].x, t[0].y, t[1].x, t[1].y};
       }
-      f32x16 xp[kParts];
+      f32x16 x = {};
+      if constexpr (kParts == 3) {
+        f32x16 xp[kParts];
 #pragma unroll
-      for (int p = 0; p < kParts; ++p) xp[p] = f32x16{};
+        for (int p = 0; p < kParts; ++p) xp[p] = f32x16{};
 #pragma unroll
-      for (int k2 = 0; k2 < 2; ++k2)
+        for (int k2 = 0; k2 < 2; ++k2)
 #pragma unroll
-        for (int p = 0; p < kParts; ++p) xp[p] = mfma(va[k2], pf[p][k2], xp[p]);
-      const f32x16 x = join(xp);
+          for (int p = 0; p < kParts; ++p) xp[p] = mfma(va[k2], pf[p][k2], xp[p]);
+        x = join(xp);
+      } else {
+#pragma unroll
+        for (int p = kParts - 1; p >= 0; --p)
+#pragma unroll
+          for (int k2 = 0; k2 < 2; ++k2) x = mfma(va[k2], pf[p][k2], x);
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) o[cc][i] = __builtin_fmaf(o[cc][i], alpha, x[i]);
     }
@@ -339,9 +366,9 @@ hipError_t launch_attend_rows(const RowsArgs& a, hipStream_t s) {
   const int64_t wgs = static_cast<int64_t>(n_qblk) * a.n_heads;
   if (wgs > 0x7fffffff) return hipErrorInvalidConfiguration;
   const dim3 grid(static_cast<unsigned>(wgs));
-  // Eight waves where they get three steps or more each (128 rows x 1500 keys: 15.8
-  // us, 16.5 on four); four below (300 keys: 7.6 us, 8.2 on eight; 224 self rows past
-  // 220: 10.1, 11.0).
+  // Eight waves where they get three steps or more each (128 rows x 1500 keys: 14.6
+  // us, 15.7 on four); four below (300 keys: 7.4 us, 7.9 on eight; 224 self rows past
+  // 220: 10.0, 10.9).
   const bool wide = a.n_keys >= 24 * kN;
 #define WRS_ROWS(P, W) \
   hipLaunchKernelGGL((attend_rows<P, W>), grid, dim3(64 * W), 0, s, a, n_qblk)

@@ -1350,17 +1350,17 @@ int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, s
                         kv->n_heads, n, L, 64, 0, 0);
   }
   // Every (group, head) reads the plane for itself; K10 reads it once per 32 rows,
-  // but a block of them takes all of it in. us, groups / K10: 300 keys, 96 pairs
-  // 7.4/7.3, 192 9.5/7.4; 700 keys, 96 8.9/10.1, 140 11.1/10.2; 1500 keys, 96
-  // 12.2/15.3, 120 15.7/15.4, 320 33.7/15.8; 3000 keys, 80 21.0/24.4, 120 28.5/24.5.
-  // Planes that a workgroup of the decode takes whole (256 keys): 192 pairs 4.7/6.5,
-  // 320 6.8/6.6. K10 also takes what is recorded without the scratch for groups.
+  // but a block of them takes all of it in. us, groups / K10: 300 keys, 100 pairs
+  // 7.1/7.2, 192 9.1/7.2; 700 keys, 96 9.1/9.8, 140 10.9/9.9; 1500 keys, 96 12.8/14.2,
+  // 120 15.9/14.4, 320 33.4/14.6; 3000 keys, 80 20.8/22.0, 100 24.4/22.0. Planes that a
+  // workgroup of the decode takes whole (256 keys): 192 pairs 4.7/6.4, 320 6.7/6.5.
+  // K10 also takes what is recorded without the scratch for groups.
   const bool recorded = c->part_recorded || capturing(c);
   const int heads = static_cast<int>(kv->n_heads), len = static_cast<int>(L);
   const size_t n_groups = (n + wrs::kMaxRowsPerGroup - 1) / wrs::kMaxRowsPerGroup;
   if (n_groups > 3 && L < wrs::kRowsMaxKeys &&
       (n_groups > static_cast<size_t>(wrs::kMaxDecodeGroups) ||
-       n_groups * kv->n_heads > (decode_splits(len) == 1 ? 320u : 112u) ||
+       n_groups * kv->n_heads > (decode_splits(len) == 1 ? 320u : 104u) ||
        (recorded && !decode_fits(c, static_cast<int>(n_groups), heads, len,
                                  wrs::kMaxRowsPerGroup))))
     return rows_impl(c, kv, q, n, out, kv->k_cross, kv->v_cross, kv->cross_off(layer),
