@@ -358,7 +358,7 @@ def test_linear_fused_equals_unfused_calls(wrs, ctx, n_tokens, n_groups, act, ou
     """layer_norm -> linear group -> gelu in one launch (decoder.rs:586-611,
     :737-753) gives bit for bit what wrs_layer_norm, wrs_linear_group and
     wrs_gelu_inplace give one after another (GELU in f32, then the output
-    rounding); 40 rows take the batched path with the norm as its own launch."""
+    rounding); 40 rows take the batched path, where the norm runs with the rows' split."""
     note(f"linear fused T={n_tokens} groups={n_groups} act={act} out={out_dt}")
     n_in, n_out = 1280, 384
     rng = np.random.default_rng(n_tokens * 13 + n_groups)

@@ -82,7 +82,8 @@ __global__ __launch_bounds__(256) void kv_slide(_Float16* k, _Float16* v, int64_
 // Copy rows [0, len) of every (layer, head) plane of K and V from one slot to
 // another. A workgroup takes pieces of kCopyUnits 16-byte units, every parts-th,
 // each read whole before it is written (one that walked a whole plane 4 KB at a
-// time waited out a round trip for each).
+// time waited out a round trip for each). K and V in one launch, us, before / now: 12
+// layers x 12 heads x 64 rows 4.0/2.5, 224 rows 6.0/3.6; 32 x 20 x 448 23.1/22.3.
 constexpr int kCopyUnits = 1024;
 constexpr int kCopyParts = 32767;  // of a plane, at most: K's and V's share a grid dimension
 __global__ __launch_bounds__(256) void kv_copy_planes(const _Float16* k_src, _Float16* k_dst,

@@ -8,7 +8,7 @@
 //   "k-contiguous" rows as stored (W [n_out][n_in] f16, X [n_tokens][k] f16),
 //   so neither needs a transpose. A workgroup owns a tile of output features x
 //   tokens (LinTile: 64 x 64 up to 256 x 256, picked by grid size in
-//   launch_parts); k advances 32 or 64 per LDS stage through a ring of 2 to 4
+//   launch_parts); k advances 32 or 64 per LDS stage through a ring of 2 to 6
 //   stages: tiles move global -> LDS with buffer_load ... lds (no staging
 //   registers), rows past the matrix edge read as zero through the buffer range
 //   check, and one barrier separates stages. Inside a stage every 16-k step
@@ -1549,8 +1549,8 @@ hipError_t launch_tile(const LinearArgs& a, int splits, hipStream_t s) {
   return hipGetLastError();
 }
 
-// A tile shape's time over `tiles` workgroups: fixed + per256 for every started
-// round of one workgroup per CU, in units of us at n_in = 1280 (every shape
+// A tile shape's time: fixed, `round` for every started round of one workgroup per
+// CU, and `tile` for every workgroup, in units of us at n_in = 1280 (every shape
 // grows alike with n_in, so one fit serves all), measured at 37 to 6000 rows
 // and 384 to 5120 features, f32 output.
 struct TileCost {
