@@ -93,14 +93,15 @@ const char *wrs_attn_status_string(int status);
  * reference allocates per call on the host). Device-resident entry points
  * never allocate once their sizes are reserved; a call that would grow
  * scratch while the context's stream records a graph fails with
- * WRS_ECAPTURE instead. Two exceptions need no reservation:
+ * WRS_ECAPTURE instead. Three exceptions need no reservation:
  * 16-bit prefill grids of fewer 128-query blocks than half the CUs merge
  * blocks split over two workgroups through a fixed context buffer (~9 MB on
  * 256 CUs), allocated by the first such call outside capture; during capture
- * before then, the call takes another schedule instead; and projections of more
+ * before then, the call takes another schedule instead; projections of more
  * than 8 rows over n_in >= 2048 whose tiles cover less than half the CUs, which
- * split k through another fixed buffer (~8 MB on 256 CUs) under the same rule
- * (reserving linear_tokens allocates it). Switching streams
+ * split k through another fixed buffer (~8 MB on 256 CUs) under the same rule;
+ * and fused norms of long decode rows (wrs_linear_fused; 160 KB), likewise
+ * (reserving linear_tokens allocates both). Switching streams
  * (wrs_attn_set_stream) drains the old stream unless either stream is
  * recording a graph. Zero fields are ignored; reserving never shrinks.
  * Synchronous. */
@@ -363,9 +364,10 @@ int wrs_linear_group(wrs_attn_ctx *ctx, int x_dtype, const void *x, size_t x_len
  * the norm; activation is WRS_ACT_NONE or WRS_ACT_GELU. Batches above 8 rows
  * (or x beyond the weight-stream kernel's LDS) need packed rows (x_row_stride ==
  * n_in) for the norm, which runs with their split into f16 parts up to n_in =
- * 2048 and as a launch of its own beyond; so it does for one or two rows of more
+ * 2048 and as a launch of its own beyond; so it does for packed decode rows of more
  * than 1280 over many features (through a fixed context buffer of 160 KB, which
- * the first such call outside capture allocates). */
+ * reserving linear_tokens of that n_in or the first such call outside capture
+ * allocates; captured before, the norm runs in the projection). */
 int wrs_linear_fused(wrs_attn_ctx *ctx, const float *x, size_t x_len, int64_t x_row_stride,
                      const float *ln_gamma, const float *ln_beta, float ln_eps,
                      size_t n_groups, const void *const *w, const float *const *bias,

@@ -1397,6 +1397,24 @@ bool gemv_by_fma(int n_tokens, int n_in, int n_out) {
 
 }  // namespace
 
+// Rows too long for a workgroup's registers, whose statistics and normalized values
+// every workgroup of K7f forms again: over many features they are normalized once. us,
+// in the kernel / in a launch of its own:
+//   1 and 2 rows     2048 -> 5120 7.2/7.3 8.6/8.2, 2112 -> 5120 10.7/9.7 12.0/10.4
+//   2 rows           3072 -> 4096 8.8/10.4, 5120 -> 5120 30.3/25.7
+//   3, 4 and 5 rows  1344 -> 2560 6.6/7.3 7.3/7.9 8.4/8.8, -> 2 x 1664 7.6/7.7 8.6/8.1
+//                    9.5/8.8; 2112 -> 2560 7.7/9.6 9.2/10.5 10.8/12.3, -> 2 x 1664
+//                    11.6/10.2 13.1/11.1 14.1/11.9; 5120 -> 2048 19.1/15.6 20.1/17.2
+//                    22.3/18.3
+//   6 rows           2048 -> 3 x 1280 13.5/10.0, 2112 -> 2 x 1664 19.5/13.3
+// K7l stages the rows per batch and gains up to 2048 columns only.
+bool gemv_norms_apart(int n_tokens, int n_in, int n_out, int n_groups) {
+  if (n_in <= kGemvLnMax) return false;
+  const int64_t features = static_cast<int64_t>(n_out) * n_groups, weights = features * n_in;
+  if (n_tokens <= 2) return features >= 5120 && weights > (10 << 20);
+  return gemv_by_fma(n_tokens, n_in, n_out) && (features >= 3072 || weights >= (10 << 20));
+}
+
 hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s) {
   if (a.n_tokens <= 0 || a.n_out <= 0 || a.n_groups <= 0) return hipSuccess;
   if (a.n_tokens > kGemvMaxRows) return hipErrorInvalidValue;

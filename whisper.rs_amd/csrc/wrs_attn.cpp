@@ -276,6 +276,12 @@ int linear_scratch(wrs_attn_ctx* c) {
   return grow(c, reinterpret_cast<void**>(&c->lin_counters), &c->lin_counter_bytes,
               wrs::linear_split_words() * sizeof(unsigned), true);
 }
+// And for the rows of fused decode projections that are normalized first.
+int ln_rows_scratch(wrs_attn_ctx* c) {
+  if (capturing(c)) return WRS_OK;
+  return grow(c, reinterpret_cast<void**>(&c->ln_rows), &c->ln_rows_bytes,
+              wrs::kGemvXFloats * sizeof(float), false);
+}
 void give_scratch(wrs_attn_ctx* c, wrs::PrefillArgs& a) {
   a.split_part = c->split_part;
   a.split_part_floats = c->split_part_bytes / sizeof(float);
@@ -704,6 +710,10 @@ int wrs_attn_reserve(wrs_attn_ctx* c, const wrs_reserve* r) {
               wrs::capture_part_floats(wrs::kMaxCapturePairs, static_cast<int>(r->capture_tokens),
                                        static_cast<int>(r->capture_keys)) * sizeof(float),
               false);
+    if (rc) return rc;
+  }
+  if (r->linear_tokens && r->linear_n_in > static_cast<size_t>(wrs::kGemvLnMax)) {
+    rc = ln_rows_scratch(c);
     if (rc) return rc;
   }
   if (r->linear_tokens > static_cast<size_t>(wrs::kGemvMaxRows) && r->linear_n_in) {
@@ -1680,21 +1690,13 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
     if (x_row_stride < static_cast<int64_t>(n_in) || n_in > (1u << 24) ||
         n_out > static_cast<size_t>(INT32_MAX / 2))
       return fail(c, WRS_EINVAL, "projection shape");
-    // One or two rows too long for a workgroup's registers, whose statistics every
-    // workgroup would form again: over many features they are normalized once, by a
-    // launch of its own (captured before its buffer exists, they are formed again).
-    // us, in the kernel / in a launch, 2 rows: 1344 -> 10240 10.9/8.3, -> 51866
-    // 43.5/24.5; 3072 -> 4096 8.8/10.4, -> 5120 15.4/12.9; 5120 -> 4096 22.0/24.3, ->
-    // 5120 30.3/25.7, -> 51866 263/114. From three rows on the launch gains nothing.
-    const int64_t features = static_cast<int64_t>(n_out) * n_groups;
-    if (ln_g && n_tokens <= 2 && n_in > static_cast<size_t>(wrs::kGemvLnMax) &&
-        (n_tokens == 1 || x_row_stride == static_cast<int64_t>(n_in)) && features >= 5120 &&
-        static_cast<int64_t>(n_in) * features >= (12 << 20)) {
-      if (!capturing(c)) {
-        const int rc = grow(c, reinterpret_cast<void**>(&c->ln_rows), &c->ln_rows_bytes,
-                            wrs::kGemvXFloats * sizeof(float), false);
-        if (rc) return rc;
-      }
+    // Rows whose fused LayerNorm runs better as a launch of its own (captured before
+    // its buffer exists, they are normalized in the kernel).
+    if (ln_g && (n_tokens == 1 || x_row_stride == static_cast<int64_t>(n_in)) &&
+        wrs::gemv_norms_apart(static_cast<int>(n_tokens), static_cast<int>(n_in),
+                              static_cast<int>(n_out), n_groups)) {
+      const int rc = ln_rows_scratch(c);
+      if (rc) return rc;
       if (c->ln_rows) {  // n_tokens * n_in <= kGemvXFloats
         WRS_HIP(c, wrs::launch_layer_norm(static_cast<const float*>(x), ln_g, ln_b, ln_eps,
                                           static_cast<int>(n_tokens), static_cast<int>(n_in),

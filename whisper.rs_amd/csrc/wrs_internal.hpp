@@ -312,6 +312,8 @@ struct GemvArgs {
   void* out[kMaxGemvGroups];
 };
 hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s);
+// Whether a fused LayerNorm is better taken out of such a launch (any number of groups).
+bool gemv_norms_apart(int n_tokens, int n_in, int n_out, int n_groups);
 // f32 rows -> [hi | lo] f16 rows (kSplitParts n_in each) and per-row 2^-shift,
 // normalized first when ln_g is set (n_in <= kSplitLnMax; gamma and beta
 // 16-byte aligned).
