@@ -554,8 +554,8 @@ __device__ inline void ln_row_norm(int d, float eps, f32x4 (&v)[kLnCache],
     for (int j = 0; j < 4; ++j) v[i][j] = fmaf((v[i][j] - mean) * inv_std, gg[i][j], bb[i][j]);
 }
 
-template <int NT, int kGemvRowsPerWave, typename OutT>
-__global__ __launch_bounds__(64 * kGemvWaves) void gemv_f16w(GemvArgs a) {
+template <int NT, int kGemvRowsPerWave, typename OutT, int kGroups>
+__global__ __launch_bounds__(64 * kGemvWaves) void gemv_f16w(GemvArgs<kGroups> a) {
   __shared__ __attribute__((aligned(16))) float xs[kGemvXFloats];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
@@ -718,8 +718,8 @@ __device__ inline float wave_max64(float v) {
   return fmaxf(v, __shfl_xor(v, 32));
 }
 
-template <typename XT, typename OutT, bool kLn>
-__global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_mfma(GemvArgs a, int T) {
+template <typename XT, typename OutT, bool kLn, int kGroups>
+__global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_mfma(GemvArgs<kGroups> a, int T) {
   extern __shared__ __attribute__((aligned(16))) _Float16 gxs[];  // [parts * nt][n_in + 8]
   __shared__ __attribute__((aligned(16))) float red[2][kGmWaves][kGmRedFloats];
   __shared__ float dn[8];
@@ -877,8 +877,8 @@ __global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_mfma(GemvArgs a, i
 constexpr int kGlKB = 4;                       // k-steps per wave per batch: 128 columns
 constexpr int kGlPitch = 32 * kGlKB + 8;       // f16 elements of a staged row
 
-template <typename OutT, bool kLn>
-__global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_long(GemvArgs a, int T) {
+template <typename OutT, bool kLn, int kGroups>
+__global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_long(GemvArgs<kGroups> a, int T) {
   __shared__ __attribute__((aligned(16))) _Float16 xs[kGmWaves][16][kGlPitch];  // hi rows, lo rows
   __shared__ __attribute__((aligned(16))) float red[2][kGmWaves][kGmRedFloats];
   __shared__ float dn[kGmWaves][8], row_mean[8], row_inv[8];
@@ -1079,9 +1079,9 @@ __global__ __launch_bounds__(64 * kGmWaves, 4) void gemv_f16w_long(GemvArgs a, i
 constexpr int gf_rows(int n_tokens) { return n_tokens <= 2 ? 8 : 5; }  // features of a workgroup
 constexpr int kGfWaves = 12;  // waves of a workgroup, at most
 
-template <int NT, int kGfRows, bool kLn, bool kDeep>
-__global__ __launch_bounds__(64 * kGfWaves) void gemv_f16w_rows(GemvArgs a, int T, int n_kw,
-                                                                DType out_dt) {
+template <int NT, int kGfRows, bool kLn, bool kDeep, int kGroups>
+__global__ __launch_bounds__(64 * kGfWaves) void gemv_f16w_rows(GemvArgs<kGroups> a, int T,
+                                                                int n_kw, DType out_dt) {
   __shared__ float part[kGfWaves][kGfRows * NT + 3];
   __shared__ float row_mean[NT], row_inv[NT];
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
@@ -1415,9 +1415,10 @@ bool gemv_norms_apart(int n_tokens, int n_in, int n_out, int n_groups) {
   return gemv_by_fma(n_tokens, n_in, n_out) && (features >= 3072 || weights >= (10 << 20));
 }
 
-hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s) {
+template <int kGroups>
+hipError_t launch_gemv_f16w(const GemvArgs<kGroups>& a, DType x_dt, DType out_dt, hipStream_t s) {
   if (a.n_tokens <= 0 || a.n_out <= 0 || a.n_groups <= 0) return hipSuccess;
-  if (a.n_tokens > kGemvMaxRows) return hipErrorInvalidValue;
+  if (a.n_tokens > kGemvMaxRows || a.n_groups > kGroups) return hipErrorInvalidValue;
   if (a.n_tokens * a.n_in > kGemvXFloats) return hipErrorInvalidValue;
   const int n_cu = linear_cus();
   int dev = 0;
@@ -1434,17 +1435,17 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
     const int64_t per_cu = (share + gf_rows(a.n_tokens) - 1) / gf_rows(a.n_tokens);
     const int T = static_cast<int>((share + per_cu - 1) / per_cu);
     const dim3 fgrid((a.n_out + T - 1) / T, a.n_groups), fblock(64 * waves);
-#define WRS_GF_L(KERNEL)                                                           \
-  {                                                                                \
-    hipLaunchKernelGGL((KERNEL), fgrid, fblock, 0, s, a, T, n_kw, out_dt);         \
-    return hipGetLastError();                                                      \
+#define WRS_GF_L(KERNEL)                                                   \
+  {                                                                        \
+    hipLaunchKernelGGL((KERNEL), fgrid, fblock, 0, s, a, T, n_kw, out_dt); \
+    return hipGetLastError();                                              \
   }
-#define WRS_GF_K(NT, R)                                                            \
-  {                                                                                \
-    if (rounds > 1 && a.ln_g) WRS_GF_L((gemv_f16w_rows<NT, R, true, true>))        \
-    if (rounds > 1) WRS_GF_L((gemv_f16w_rows<NT, R, false, true>))                 \
-    if (a.ln_g) WRS_GF_L((gemv_f16w_rows<NT, R, true, false>))                     \
-    WRS_GF_L((gemv_f16w_rows<NT, R, false, false>))                                \
+#define WRS_GF_K(NT, R)                                                              \
+  {                                                                                  \
+    if (rounds > 1 && a.ln_g) WRS_GF_L((gemv_f16w_rows<NT, R, true, true, kGroups>)) \
+    if (rounds > 1) WRS_GF_L((gemv_f16w_rows<NT, R, false, true, kGroups>))          \
+    if (a.ln_g) WRS_GF_L((gemv_f16w_rows<NT, R, true, false, kGroups>))              \
+    WRS_GF_L((gemv_f16w_rows<NT, R, false, false, kGroups>))                         \
   }
     switch (a.n_tokens) {
       case 1: if (T > 5) WRS_GF_K(1, 8) else WRS_GF_K(1, 5)
@@ -1479,30 +1480,30 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
     // hold their registers to 128).
     const size_t lds = kGmStaticLds + (long_rows ? 0 : gm_lds);
     const int per_cu = long_rows || 2 * lds <= 160 * 1024 ? 2 : 1;
-#define WRS_GM_K(KERNEL, LDS)                                                                 \
-  {                                                                                           \
-    const void* fn = reinterpret_cast<const void*>(&KERNEL);                                  \
-    static std::atomic<uint64_t> attr_set{0};  /* one bit per device */                       \
-    if (LDS > 0 && dev < 64 &&                                                                \
-        !(attr_set.load(std::memory_order_acquire) & (uint64_t{1} << dev))) {                 \
-      const hipError_t e = hipFuncSetAttribute(                                               \
-          fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGmMaxDynLds));    \
-      if (e != hipSuccess) return e;                                                          \
-      attr_set.fetch_or(uint64_t{1} << dev, std::memory_order_acq_rel);                       \
-    }                                                                                         \
-    const dim3 ggrid(std::min(n_tiles, n_cu * per_cu), a.n_groups);                            \
-    hipLaunchKernelGGL((KERNEL), ggrid, gblock, LDS, s, a, T);                                \
-    return hipGetLastError();                                                                 \
+#define WRS_GM_K(KERNEL, LDS)                                                              \
+  {                                                                                        \
+    const void* fn = reinterpret_cast<const void*>(&KERNEL);                               \
+    static std::atomic<uint64_t> attr_set{0};  /* one bit per device */                    \
+    if (LDS > 0 && dev < 64 &&                                                             \
+        !(attr_set.load(std::memory_order_acquire) & (uint64_t{1} << dev))) {              \
+      const hipError_t e = hipFuncSetAttribute(                                            \
+          fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kGmMaxDynLds)); \
+      if (e != hipSuccess) return e;                                                       \
+      attr_set.fetch_or(uint64_t{1} << dev, std::memory_order_acq_rel);                    \
+    }                                                                                      \
+    const dim3 ggrid(std::min(n_tiles, n_cu * per_cu), a.n_groups);                        \
+    hipLaunchKernelGGL((KERNEL), ggrid, gblock, LDS, s, a, T);                             \
+    return hipGetLastError();                                                              \
   }
 #define WRS_GM(OT)                                                              \
   if (x_dt == kF16) {                                                           \
     if (a.ln_g) return hipErrorInvalidValue;  /* a fused LayerNorm takes f32 */ \
-    WRS_GM_K((gemv_f16w_mfma<_Float16, OT, false>), gm_lds)                     \
+    WRS_GM_K((gemv_f16w_mfma<_Float16, OT, false, kGroups>), gm_lds)            \
   }                                                                             \
-  if (long_rows && a.ln_g) WRS_GM_K((gemv_f16w_long<OT, true>), 0)              \
-  if (long_rows) WRS_GM_K((gemv_f16w_long<OT, false>), 0)                       \
-  if (a.ln_g) WRS_GM_K((gemv_f16w_mfma<float, OT, true>), gm_lds)               \
-  WRS_GM_K((gemv_f16w_mfma<float, OT, false>), gm_lds)
+  if (long_rows && a.ln_g) WRS_GM_K((gemv_f16w_long<OT, true, kGroups>), 0)     \
+  if (long_rows) WRS_GM_K((gemv_f16w_long<OT, false, kGroups>), 0)              \
+  if (a.ln_g) WRS_GM_K((gemv_f16w_mfma<float, OT, true, kGroups>), gm_lds)      \
+  WRS_GM_K((gemv_f16w_mfma<float, OT, false, kGroups>), gm_lds)
     switch (out_dt) {
       case kF32: WRS_GM(float)
       case kF16: WRS_GM(_Float16)
@@ -1521,15 +1522,15 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
   const int wgs = std::min(n_cu, (groups + kGemvWaves - 1) / kGemvWaves);
   dim3 grid(std::max(wgs, 1), a.n_groups);
   dim3 block(64 * kGemvWaves);
-#define WRS_GEMV(OT)                                                                       \
-  if (rpw == 1 && a.n_tokens == 1)                                                         \
-    hipLaunchKernelGGL((gemv_f16w<1, 1, OT>), grid, block, 0, s, a);                       \
-  else if (rpw == 1)                                                                       \
-    hipLaunchKernelGGL((gemv_f16w<2, 1, OT>), grid, block, 0, s, a);                       \
-  else if (a.n_tokens == 1)                                                                \
-    hipLaunchKernelGGL((gemv_f16w<1, 4, OT>), grid, block, 0, s, a);                       \
-  else                                                                                     \
-    hipLaunchKernelGGL((gemv_f16w<2, 4, OT>), grid, block, 0, s, a);
+#define WRS_GEMV(OT)                                                          \
+  if (rpw == 1 && a.n_tokens == 1)                                            \
+    hipLaunchKernelGGL((gemv_f16w<1, 1, OT, kGroups>), grid, block, 0, s, a); \
+  else if (rpw == 1)                                                          \
+    hipLaunchKernelGGL((gemv_f16w<2, 1, OT, kGroups>), grid, block, 0, s, a); \
+  else if (a.n_tokens == 1)                                                   \
+    hipLaunchKernelGGL((gemv_f16w<1, 4, OT, kGroups>), grid, block, 0, s, a); \
+  else                                                                        \
+    hipLaunchKernelGGL((gemv_f16w<2, 4, OT, kGroups>), grid, block, 0, s, a);
   switch (out_dt) {
     case kF32: WRS_GEMV(float) break;
     case kF16: WRS_GEMV(_Float16) break;
@@ -1539,6 +1540,8 @@ hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStre
 #undef WRS_GEMV
   return hipGetLastError();
 }
+template hipError_t launch_gemv_f16w(const GemvArgs<kFewGemvGroups>&, DType, DType, hipStream_t);
+template hipError_t launch_gemv_f16w(const GemvArgs<kMaxLinearGroups>&, DType, DType, hipStream_t);
 
 namespace {
 

@@ -1706,28 +1706,31 @@ int linear_impl(wrs_attn_ctx* c, int x_dtype, const void* x, size_t x_len, int64
         ln_g = ln_b = nullptr;
       }
     }
-    wrs::GemvArgs gv{};
-    gv.x = x;
-    gv.x_rs = x_row_stride;
-    gv.n_tokens = static_cast<int>(n_tokens);
-    gv.n_in = static_cast<int>(n_in);
-    gv.n_out = static_cast<int>(n_out);
-    gv.out_rs = out_row_stride;
-    gv.out_hs = out_head_stride;
-    gv.ln_g = ln_g;
-    gv.ln_b = ln_b;
-    gv.ln_eps = ln_eps;
-    gv.act = act;
-    for (int g0 = 0; g0 < n_groups; g0 += wrs::kMaxGemvGroups) {
-      gv.n_groups = std::min(wrs::kMaxGemvGroups, n_groups - g0);
-      for (int gi = 0; gi < gv.n_groups; ++gi) {
-        gv.w[gi] = static_cast<const _Float16*>(w[g0 + gi]);
-        gv.bias[gi] = bias ? bias[g0 + gi] : nullptr;
-        gv.out[gi] = out[g0 + gi];
+    auto launch = [&](auto gv) {
+      gv.x = x;
+      gv.x_rs = x_row_stride;
+      gv.n_tokens = static_cast<int>(n_tokens);
+      gv.n_in = static_cast<int>(n_in);
+      gv.n_out = static_cast<int>(n_out);
+      gv.n_groups = n_groups;
+      gv.out_rs = out_row_stride;
+      gv.out_hs = out_head_stride;
+      gv.ln_g = ln_g;
+      gv.ln_b = ln_b;
+      gv.ln_eps = ln_eps;
+      gv.act = act;
+      for (int gi = 0; gi < n_groups; ++gi) {
+        gv.w[gi] = static_cast<const _Float16*>(w[gi]);
+        gv.bias[gi] = bias ? bias[gi] : nullptr;
+        gv.out[gi] = out[gi];
       }
-      WRS_HIP(c, wrs::launch_gemv_f16w(gv, static_cast<wrs::DType>(x_dtype),
-                                       static_cast<wrs::DType>(out_dtype), c->stream));
-    }
+      return wrs::launch_gemv_f16w(gv, static_cast<wrs::DType>(x_dtype),
+                                   static_cast<wrs::DType>(out_dtype), c->stream);
+    };
+    if (n_groups <= wrs::kFewGemvGroups)
+      WRS_HIP(c, launch(wrs::GemvArgs<wrs::kFewGemvGroups>{}));
+    else
+      WRS_HIP(c, launch(wrs::GemvArgs<wrs::kMaxLinearGroups>{}));
     return WRS_OK;
   }
   for (int gi = 0; gi < n_groups; ++gi)

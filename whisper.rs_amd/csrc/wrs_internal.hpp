@@ -289,13 +289,14 @@ size_t linear_split_words();
 // Decode-sized batches (n_tokens <= kGemvMaxRows) of the same product on the
 // f16 weight stream; x is f32 or f16 with row stride x_rs, no split needed.
 constexpr int kGemvMaxRows = 8;
-// Weight groups of one launch; more take further launches. A launch copies its
-// arguments, and these launches are host-bound in a step that is not captured:
-// room for 64 groups cost 0.5 us of a 6.7 us call (5 rows 768 x 768), room for 8 is
-// what a layer's projections need (3).
-constexpr int kMaxGemvGroups = 8;
+// Weight groups that a launch's arguments have room for: the arguments are copied, and
+// these launches are host-bound in a step that is not captured. Room for 64 groups cost
+// 0.5 us of a 6.7 us call (5 rows 768 x 768), room for 8 is what a layer's projections
+// need (3). More groups still run in one launch, of the same kernels on larger arguments.
+constexpr int kFewGemvGroups = 8;
 constexpr int kGemvLnMax = 1280;  // longer f32 rows do not fit the decode kernels' registers
 constexpr int kGemvXFloats = 40960;  // n_tokens * n_in staged in LDS (160 KB)
+template <int kGroups>
 struct GemvArgs {
   const void* x;
   int64_t x_rs;
@@ -307,11 +308,13 @@ struct GemvArgs {
   const float* ln_b;
   float ln_eps;
   int act;  // Act, applied after the bias
-  const _Float16* w[kMaxGemvGroups];
-  const float* bias[kMaxGemvGroups];
-  void* out[kMaxGemvGroups];
+  const _Float16* w[kGroups];
+  const float* bias[kGroups];
+  void* out[kGroups];
 };
-hipError_t launch_gemv_f16w(const GemvArgs& a, DType x_dt, DType out_dt, hipStream_t s);
+// kGroups: kFewGemvGroups or kMaxLinearGroups.
+template <int kGroups>
+hipError_t launch_gemv_f16w(const GemvArgs<kGroups>& a, DType x_dt, DType out_dt, hipStream_t s);
 // Whether a fused LayerNorm is better taken out of such a launch (any number of groups).
 bool gemv_norms_apart(int n_tokens, int n_in, int n_out, int n_groups);
 // f32 rows -> [hi | lo] f16 rows (kSplitParts n_in each) and per-row 2^-shift,
