@@ -100,7 +100,7 @@ const char *wrs_attn_status_string(int status);
  * before then, the call takes another schedule instead; projections of more
  * than 8 rows over n_in >= 2048 whose tiles cover less than half the CUs, which
  * split k through another fixed buffer (~8 MB on 256 CUs) under the same rule;
- * and fused norms of long decode rows (wrs_linear_fused; 160 KB), likewise
+ * and fused norms of decode rows over many features (wrs_linear_fused), likewise
  * (reserving linear_tokens allocates both). Switching streams
  * (wrs_attn_set_stream) drains the old stream unless either stream is
  * recording a graph. Zero fields are ignored; reserving never shrinks.
@@ -365,9 +365,9 @@ int wrs_linear_group(wrs_attn_ctx *ctx, int x_dtype, const void *x, size_t x_len
  * (or x beyond the weight-stream kernel's LDS) need packed rows (x_row_stride ==
  * n_in) for the norm, which runs with their split into f16 parts up to n_in =
  * 2048 and as a launch of its own beyond; so it does for packed decode rows of more
- * than 1280 over many features (through a fixed context buffer of 160 KB, which
- * reserving linear_tokens of that n_in or the first such call outside capture
- * allocates; captured before, the norm runs in the projection). */
+ * than 1280 over many features, and of any width over very many (through a fixed
+ * context buffer of 160 KB, which reserving linear_tokens or the first such call
+ * outside capture allocates; captured before, the norm runs in the projection). */
 int wrs_linear_fused(wrs_attn_ctx *ctx, const float *x, size_t x_len, int64_t x_row_stride,
                      const float *ln_gamma, const float *ln_beta, float ln_eps,
                      size_t n_groups, const void *const *w, const float *const *bias,

@@ -622,7 +622,8 @@ def test_linear_long_rows_few_tiles(wrs, ctx, n_tokens, n_in, n_out, n_groups):
 
 @pytest.mark.parametrize("rows,n_in,n_out,groups", [
     (1, 1344, 9728, 1), (2, 1344, 3277, 3), (1, 5120, 5120, 1), (2, 5120, 5119, 1), (3, 1344, 9728, 1),
-    (3, 1344, 1664, 2), (4, 5120, 2048, 1), (6, 2112, 1664, 2), (8, 2112, 1280, 3), (8, 5120, 1023, 3)])
+    (3, 1344, 1664, 2), (4, 5120, 2048, 1), (6, 2112, 1664, 2), (8, 2112, 1280, 3), (8, 5120, 1023, 3),
+    (3, 1280, 1024, 8), (5, 768, 257, 32)])
 def test_fused_norm_of_long_decode_rows(wrs, ctx, rows, n_in, n_out, groups):
     # The norm of long rows over many features runs as a launch of its own:
     # bit for bit the separate calls, eager and (before its buffer exists) captured,

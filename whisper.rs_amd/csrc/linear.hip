@@ -1407,12 +1407,14 @@ bool gemv_by_fma(int n_tokens, int n_in, int n_out) {
 //                    11.6/10.2 13.1/11.1 14.1/11.9; 5120 -> 2048 19.1/15.6 20.1/17.2
 //                    22.3/18.3
 //   6 rows           2048 -> 3 x 1280 13.5/10.0, 2112 -> 2 x 1664 19.5/13.3
-// K7l stages the rows per batch and gains up to 2048 columns only.
+// K7l stages the rows per batch and gains up to 2048 columns only. Rows that fit gain
+// from 3 rows on where a call has many groups (5 rows 384 -> 12 x 384 7.0/6.3, 768 -> 16
+// x 768 14.0/10.0, 1280 -> 9 x 1280 16.5/13.6; a layer's three of 1280 7.7/7.3).
 bool gemv_norms_apart(int n_tokens, int n_in, int n_out, int n_groups) {
-  if (n_in <= kGemvLnMax) return false;
   const int64_t features = static_cast<int64_t>(n_out) * n_groups, weights = features * n_in;
-  if (n_tokens <= 2) return features >= 5120 && weights > (10 << 20);
-  return gemv_by_fma(n_tokens, n_in, n_out) && (features >= 3072 || weights >= (10 << 20));
+  if (n_tokens <= 2) return n_in > kGemvLnMax && features >= 5120 && weights > (10 << 20);
+  if (!gemv_by_fma(n_tokens, n_in, n_out)) return false;
+  return n_in > kGemvLnMax ? features >= 3072 || weights >= (10 << 20) : features >= 8192;
 }
 
 template <int kGroups>

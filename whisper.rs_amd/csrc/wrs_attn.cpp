@@ -712,7 +712,7 @@ int wrs_attn_reserve(wrs_attn_ctx* c, const wrs_reserve* r) {
               false);
     if (rc) return rc;
   }
-  if (r->linear_tokens && r->linear_n_in > static_cast<size_t>(wrs::kGemvLnMax)) {
+  if (r->linear_tokens && r->linear_n_in) {
     rc = ln_rows_scratch(c);
     if (rc) return rc;
   }
