@@ -276,3 +276,39 @@ def test_cached_self_rows_over_infinite_keys(wrs, ctx, rows, past):
     tol = _bound(q, kz, v, 1)
     assert (np.abs(got - ref) <= tol)[seen].all()
     arena.close()
+
+
+@pytest.mark.parametrize("keys", [300, 1500])
+@pytest.mark.parametrize("where,value", [("k", 1e6), ("k", -1e6), ("k", float("nan")),
+                                         ("q", float("inf")), ("q", float("nan"))])
+def test_cross_rows_with_infinite_scores(wrs, ctx, keys, where, value):
+    # A key or query that gives a row a NaN score: on K10 the row comes out as the
+    # single-row decode has it (zeros; a row whose score is -inf gives that key no
+    # weight), and the other rows are untouched.
+    note(f"cross rows, {value} in {where}, {keys} keys")
+    heads, rows = 29, 27
+    rng = np.random.default_rng(keys)
+    k, v = (_f16(rng.standard_normal((keys, heads * 64))) for _ in range(2))
+    q = rng.standard_normal((rows, heads * 64)).astype(np.float32)
+    plain, _, _ = _attend(q, k, v, heads)
+    tol = _bound(q, k, v, heads)
+    if where == "k":
+        k[keys // 2, 7] = value
+    else:
+        q[5, 7] = value
+    arena = wrs.KvArena(1, 1, heads, 16, keys, ctx=ctx)
+    arena.set_cross(0, k, v)
+    qd, out = dev(q), torch.full((rows, heads * 64), float("nan"), device="cuda")
+    arena.prefill_cross(0, qd, out)
+    one = torch.zeros((rows, heads * 64), device="cuda")
+    for r in range(rows):
+        arena.decode_cross(0, qd[r:r + 1].contiguous(), one[r:r + 1])
+    got, ref = host(out), host(one)
+    hit = np.zeros(got.shape, bool)  # head 0, whose key or query it is
+    hit[(slice(None) if where == "k" else 5), :64] = True
+    # the same rows are zero; the others lie within tol of the same exact result each
+    assert np.array_equal(got[hit] == 0.0, ref[hit] == 0.0)
+    assert (np.abs(got - ref) <= 2 * tol)[hit].all()
+    assert value == value and where == "k" or (got[hit] == 0.0).all()
+    assert (np.abs(got - plain) <= tol)[~hit].all()
+    arena.close()

@@ -313,6 +313,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void attend_rows(RowsArgs a, int n_
         acc[e] = __builtin_fmaf(mo[w][row * kPitch + d0 + e], ew, acc[e]);
     }
     const float inv = (L > 0.f ? 1.f / L : 0.f) * (1.f / kWeightUp);
+    if constexpr (kParts == 2) {
+      // A cross row whose sum is NaN (an infinite key or query) is zero, as the split-K
+      // decode has it, whose groups take the shorter prompts.
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] = L > 0.f ? acc[e] : 0.f;
+    }
     float* const op = a.o + static_cast<int64_t>(q0 + row) * a.o_rs + h * 64 + d0;
     *reinterpret_cast<f32x4u*>(op) = f32x4{acc[0], acc[1], acc[2], acc[3]} * inv;
     *reinterpret_cast<f32x4u*>(op + 4) = f32x4{acc[4], acc[5], acc[6], acc[7]} * inv;
