@@ -24,10 +24,10 @@
 //   Bound by latency: launch, first loads, then ~1 us a step on few CUs, merge.
 //   Dealing a block's steps over several workgroups that merge through memory
 //   cost as much as it saved (128 rows x 1500 keys: 15.0 us in three).
-//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 15.0 us
+//   Measured, 20 heads, queued back to back: 128 rows x 1500 keys 32.5 -> 14.2 us
 //   (groups of 8 rows each read the planes again: 123 MB of L2 reads); 37 cached self
-//   rows 14.5 -> 5.6 us, 224 rows past 220 37.9 -> 10.2 (f32 matrix pipe, element
-//   loads). Weights in units of 1 and three parts in one unit took 14.2, 5.3 and 9.1
+//   rows 14.5 -> 5.4 us, 224 rows past 220 37.9 -> 9.4 (f32 matrix pipe, element
+//   loads). Weights in units of 1 and three parts in one unit took 14.1, 5.4 and 8.9
 //   us, but a weight 2^-20 of the largest kept four bits; two parts in units of their
 //   own 16.2.
 #include "prefill_f32_block.hpp"
@@ -75,8 +75,18 @@ __device__ inline f32x16 mfma(const u32x4& a, const u32x4& b, const f32x16& c) {
 // part leaves is at most 2^-11 of the value, so the next one holds 11 bits more at
 // the same magnitude.
 constexpr float kPartUnit = 0x1p-11f;
+// The pair is formed once (v_fma_mixlo, v_fma_mixhi): with nothing to hide its origin the
+// compiler rounds each element again where the next part subtracts it (23 of the 285
+// instructions of a two-part step, 41 of 472 with three).
+__device__ inline f16x2 pack2(float x0, float x1, float scale) {
+  const f16x2 h = {static_cast<_Float16>(__builtin_fmaf(x0, scale, 0.f)),
+                   static_cast<_Float16>(__builtin_fmaf(x1, scale, 0.f))};
+  uint32_t w = __builtin_bit_cast(uint32_t, h);
+  asm("" : "+v"(w));
+  return __builtin_bit_cast(f16x2, w);
+}
 __device__ inline void split2(float x0, float x1, float scale, uint32_t (&out)[2]) {
-  const f16x2 h = {static_cast<_Float16>(x0 * scale), static_cast<_Float16>(x1 * scale)};
+  const f16x2 h = pack2(x0, x1, scale);
   const f16x2 l = {
       static_cast<_Float16>(__builtin_fmaf(x0, scale, -static_cast<float>(h[0]))),
       static_cast<_Float16>(__builtin_fmaf(x1, scale, -static_cast<float>(h[1])))};
@@ -85,15 +95,17 @@ __device__ inline void split2(float x0, float x1, float scale, uint32_t (&out)[2
 }
 __device__ inline void split2(float x0, float x1, float scale, uint32_t (&out)[3]) {
   constexpr float kUp = 1.f / kPartUnit;
-  x0 *= scale;
-  x1 *= scale;
-#pragma unroll
-  for (int p = 0; p < 3; ++p) {
-    const f16x2 h = {static_cast<_Float16>(x0), static_cast<_Float16>(x1)};
-    out[p] = __builtin_bit_cast(uint32_t, h);
-    x0 = __builtin_fmaf(static_cast<float>(h[0]), -kUp, x0 * kUp);  // exact
-    x1 = __builtin_fmaf(static_cast<float>(h[1]), -kUp, x1 * kUp);
-  }
+  const f16x2 h = pack2(x0, x1, scale);
+  x0 = __builtin_fmaf(x0, scale, -static_cast<float>(h[0]));  // exact
+  x1 = __builtin_fmaf(x1, scale, -static_cast<float>(h[1]));
+  const f16x2 m = pack2(x0, x1, kUp);
+  x0 = __builtin_fmaf(static_cast<float>(m[0]), -kPartUnit, x0);  // exact
+  x1 = __builtin_fmaf(static_cast<float>(m[1]), -kPartUnit, x1);
+  const f16x2 l = {static_cast<_Float16>(__builtin_fmaf(x0, kUp * kUp, 0.f)),
+                   static_cast<_Float16>(__builtin_fmaf(x1, kUp * kUp, 0.f))};
+  out[0] = __builtin_bit_cast(uint32_t, h);
+  out[1] = __builtin_bit_cast(uint32_t, m);
+  out[2] = __builtin_bit_cast(uint32_t, l);
 }
 // Three parts' sums of products as one, smallest first.
 __device__ inline f32x16 join(const f32x16 (&x)[3]) {
@@ -372,9 +384,9 @@ hipError_t launch_attend_rows(const RowsArgs& a, hipStream_t s) {
   const int64_t wgs = static_cast<int64_t>(n_qblk) * a.n_heads;
   if (wgs > 0x7fffffff) return hipErrorInvalidConfiguration;
   const dim3 grid(static_cast<unsigned>(wgs));
-  // Eight waves where they get three steps or more each (128 rows x 1500 keys: 14.6
-  // us, 15.7 on four); four below (300 keys: 7.4 us, 7.9 on eight; 224 self rows past
-  // 220: 10.0, 10.9).
+  // Eight waves where they get three steps or more each (128 rows x 1500 keys: 14.2
+  // us, 15.4 on four); four below (300 keys: 7.4 us, 8.0 on eight; 224 self rows past
+  // 220: 9.6, 10.5).
   const bool wide = a.n_keys >= 24 * kN;
 #define WRS_ROWS(P, W) \
   hipLaunchKernelGGL((attend_rows<P, W>), grid, dim3(64 * W), 0, s, a, n_qblk)

@@ -1361,9 +1361,9 @@ int cross_rows_impl(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, const float* q, s
   }
   // Every (group, head) reads the plane for itself; K10 reads it once per 32 rows,
   // but a block of them takes all of it in. us, groups / K10: 300 keys, 100 pairs
-  // 7.1/7.2, 192 9.1/7.2; 700 keys, 96 9.1/9.8, 140 10.9/9.9; 1500 keys, 96 12.8/14.2,
-  // 120 15.9/14.4, 320 33.4/14.6; 3000 keys, 80 20.8/22.0, 100 24.4/22.0. Planes that a
-  // workgroup of the decode takes whole (256 keys): 192 pairs 4.7/6.4, 320 6.7/6.5.
+  // 7.2/7.3, 192 9.0/7.3; 700 keys, 104 8.9/9.8, 140 10.4/9.9; 1500 keys, 104 13.4/13.6,
+  // 112 14.0/13.7, 320 31.1/14.2; 3000 keys, 80 19.5/21.1, 100 22.9/21.3. Planes that a
+  // workgroup of the decode takes whole (256 keys): 192 pairs 4.7/6.4, 336 6.6/6.5.
   // K10 also takes what is recorded without the scratch for groups.
   const bool recorded = c->part_recorded || capturing(c);
   const int heads = static_cast<int>(kv->n_heads), len = static_cast<int>(L);
