@@ -276,7 +276,7 @@ int wrs_attn_decode_cross_noalloc(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, c
  * two (2^-22 down to 2^-18 of the row's largest) for cross-attention (few rows or
  * heads on the split-K decode kernel, in groups of 8 rows that share each read of
  * the plane), three (all 24 bits down to 2^-28) for the cached self-attention (on
- * the f32 kernel where few rows meet more than 2048 keys). */
+ * the f32 kernel where few rows meet more than 3584 keys). */
 int wrs_attn_prefill_self(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, size_t slot,
                           const float *q, size_t n_tokens, float *out);
 int wrs_attn_prefill_cross(wrs_attn_ctx *ctx, wrs_kv *kv, size_t layer, const float *q,

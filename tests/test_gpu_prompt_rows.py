@@ -153,10 +153,11 @@ def test_cross_rows_recorded_without_scratch(wrs):
     c.close()
 
 
-@pytest.mark.parametrize("heads,rows,past", [(1, 2, 2046), (1, 2, 2047), (2, 33, 3000),
-                                             (16, 32, 2500), (17, 32, 2500)])
+@pytest.mark.parametrize("heads,rows,past", [(1, 2, 3582), (1, 2, 3583), (2, 33, 3800),
+                                             (16, 32, 3600), (17, 32, 3600), (16, 32, 6218),
+                                             (16, 32, 6219)])
 def test_cached_self_rows_of_long_caches(wrs, ctx, heads, rows, past):
-    # Few blocks over more than 2048 keys: the f32 kernel, its keys dealt over workgroups.
+    # Few blocks over more than 3584 keys: the f32 kernel, its keys dealt over workgroups.
     test_cached_self_rows(wrs, ctx, heads, rows, past)
 
 

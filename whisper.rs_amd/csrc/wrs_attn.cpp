@@ -1444,11 +1444,13 @@ int wrs_attn_prefill_self(wrs_attn_ctx* c, wrs_kv* kv, size_t layer, size_t slot
     return WRS_OK;
   }
   // K10, but for few blocks of 32 rows over long caches, whose keys the f32 kernel
-  // deals over workgroups (through scratch; us, K10 / f32 kernel, blocks x keys): 1 x
-  // 2000 21.4/21.3, 1 x 4000 37.6/28.9, 12 x 4000 39.0/33.2, 20 x 4000 38.2/36.4, 40 x
-  // 4000 39.3/60.8, 20 x 2000 21.8/28.5, 8 x 8000 71.2/55.0.
+  // deals over workgroups (through scratch; us, K10 / f32 kernel, 8 rows of 6 and 32 of
+  // 12 heads: 2500 keys 23.3/29.3 24.6/33.2, 3500 30.6/29.3 31.9/33.3, 4000 34.3/29.4
+  // 35.5/33.2, 5000 41.5/37.0 42.8/41.1, 8000 62.0/45.0 63.4/48.8; 16 blocks: 6000
+  // 49.0/41.2, 8000 63.7/73.1; 18 blocks: 4000 35.6/40.1, 5000 42.9/40.3, 6000 49.3/71.3).
   const size_t keys = t_past + n_tokens;
-  const bool dealt = keys > 2048 && (n_tokens + 31) / 32 * kv->n_heads <= 16 &&
+  const size_t blocks = (n_tokens + 31) / 32 * kv->n_heads;
+  const bool dealt = keys > 3584 && blocks <= 16 && blocks * keys <= 100000 &&
                      (c->split_part || !capturing(c));
   if (keys < wrs::kRowsMaxKeys && !dealt) {
     if (!q || !out) return fail(c, WRS_EINVAL, "null tensor pointer");
