@@ -186,9 +186,9 @@ int wrs_attn_prefill(wrs_attn_ctx *ctx, int q_dtype, const void *q, const wrs_la
  * scores). On f32 arenas wrs_attn_decode_cross_noalloc,
  * wrs_attn_prefill_cross_lse and wrs_attn_capture_cross_heads_lse return
  * WRS_EUNSUPPORTED, and the attention calls size their score scratch (9
- * bytes per row, head and key) on the first eager call; only those over more
- * than 512 keys use it, and such a first call under stream capture fails
- * with WRS_ECAPTURE. */
+ * bytes per row, head and key; calls of up to 8 rows for the arena's longest
+ * rows) on the first eager call; only those over more than 512 keys use it, and
+ * such a first call under stream capture fails with WRS_ECAPTURE. */
 
 /* DecoderKvCache::new (decoder.rs:148-157) with the arena capacity fixed;
  * f16 planes. */
